@@ -12,7 +12,7 @@ CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libffsim_amd.so"
 
 SOURCES = ["ffsim_amd.hip", "noalloc.hip", "host_core.cpp"]
-HEADERS = ["kernels.hpp", "host_core.hpp", "status.hpp", "diag_params.hpp"]
+HEADERS = ["kernels.hpp", "fiber_pipe.hpp", "host_core.hpp", "status.hpp", "diag_params.hpp"]
 
 
 def hipcc() -> str:

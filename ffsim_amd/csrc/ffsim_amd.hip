@@ -29,6 +29,7 @@
 #include "../../include/ffsim_amd.h"
 #include "diag_params.hpp"
 #include "host_core.hpp"
+#include "fiber_pipe.hpp"
 #include "kernels.hpp"
 #include "status.hpp"
 
@@ -718,6 +719,109 @@ void launch_fiber_t(const void* src, void* dst, long ld_src, long ld_dst, int n_
   prof_stop(pk, stream);
 }
 
+// LDS of a pipelined launch, following the kernel's layout.
+size_t pipe_lds_bytes(int W, int gd_cap, int gm_cap, bool tstore, bool diag, int n_fac, int win) {
+  constexpr size_t R = kPipeMaxRows;
+  size_t b = (R + kPipeStep) * 128 + (tstore ? 0 : kPipeSlots * R * 4) +
+             kMaxLoSlots * sizeof(GroupSlot) + 2 * align16((size_t)gd_cap * 4) +
+             align16((size_t)gm_cap * 2) + (size_t)kMaxLoSlots * kPipeCompute * 8;
+  if (diag || n_fac) b += kPipeSlots * R * 2;
+  if (n_fac)
+    b += 16 + ((size_t)W * n_fac + (size_t)fuse_nibble_entries(win, W)) * sizeof(Cx<double>);
+  else if (diag)
+    b += 68 * sizeof(Cx<double>);
+  return b;
+}
+
+int pipe_tile_width(int dtype) { return dtype == FFSIM_C128 ? pipe_width<double>() : pipe_width<float>(); }
+
+// The largest group tables any pass of this window can stage (every sub-window start).
+void group_caps(const DevGroups& gr, int& gd_cap, int& gm_cap) {
+  gd_cap = gm_cap = 0;
+  for (int kp = 0; kp <= gr.w; ++kp) {
+    int nd = 0, nm = 0;
+    for (int lo2 = 0; lo2 < gr.n_lo2; ++lo2) {
+      const int* ix = gr.host_index.data() + ((size_t)kp * gr.n_lo2 + lo2) * 4;
+      nd += ix[1];
+      nm += ix[3];
+    }
+    gd_cap = std::max(gd_cap, nd);
+    gm_cap = std::max(gm_cap, nm);
+  }
+}
+
+// Whether a row pass over these fibers runs pipelined (fiber_pipe_kernel).
+// Both kernels walk their tiles in rounds over the CUs, one pipelined tile per
+// CU against one plain complex128 tile or three plain complex64 tiles of a
+// quarter of the columns.  Measured on the LUCJ passes of norb 13 to 16: a
+// round takes about 17.6 / 21 us (complex128) and 25.6 / 21.5 us (complex64),
+// and a pipelined launch 16 us more to fill and drain, so it wins from 5
+// rounds on in complex128 (norb=15: 482 against 538 us per launch; norb=13
+// with 2 rounds: 58 against 53).  Fibers whose plain tiles leave room for a
+// second workgroup per CU gain nothing from it in complex128 (norb=16 (4,4),
+// 495 strings: 180 against 126 us).
+bool pipe_applies(Context& ctx, int dtype, const DevWindow& win, bool all_fibers,
+                  const DevGroups& gr, long n_batch) {
+  const int W = pipe_tile_width(dtype);
+  const int rows = all_fibers ? win.max_rows : win.max_rows_active;
+  const long n_f = all_fibers ? win.n_fibers : win.n_active;
+  if (gr.w2 != kMaxSubWindow || gr.n_lo2 > kMaxLoSlots || n_batch < W || win.w > 16 ||
+      rows > kPipeMaxRows || n_batch > (1l << 30))
+    return false;
+  const bool c128 = dtype == FFSIM_C128;
+  if (c128 ? 2 * (size_t)rows * 128 <= ctx.lds_max : rows < 400) return false;
+  auto rounds = [&](int width, long per_cu) {
+    const long tiles = (n_batch + width - 1) / width * n_f;
+    return (double)((tiles + per_cu * g_n_cu - 1) / (per_cu * g_n_cu));
+  };
+  return (c128 ? 17.6 : 25.6) * rounds(W, 1) + 16.0 <
+         (c128 ? 21.0 * rounds(8, 1) : 21.5 * rounds(4, 3));
+}
+
+template <typename T>
+void launch_fiber_pipe(const void* src, void* dst, long ld_src, long ld_dst, int n_batch,
+                       bool tstore, const DevWindow& win, bool all_fibers, const DevGroups& gr,
+                       const LoSlots& los, int gd_cap, int gm_cap, const SubPass* d_subs, int n_sub,
+                       const LayerPair* d_layers, const double* d_diag, const uint64_t* d_strings,
+                       const Cx<double>* cfac, const PipeFuse& fz, size_t lds_max,
+                       hipStream_t stream) {
+  constexpr int W = pipe_width<T>();
+  const int n_f = all_fibers ? win.n_fibers : win.n_active;
+  if (n_f == 0 || n_batch == 0) return;
+  const bool fuse = fz.bfac != nullptr;
+  const bool dg = !fuse && (d_diag != nullptr);
+  require(!tstore || win.lo == 0, FFSIM_ERR_VALUE, "pipelined pass: transposing window not at 0");
+  require(!fuse || tstore, FFSIM_ERR_VALUE, "pipelined pass: fused diagonal without transposition");
+  require(!cfac || (tstore && dg), FFSIM_ERR_VALUE, "pipelined pass: column factors");
+  const size_t lds = pipe_lds_bytes(W, gd_cap, gm_cap, tstore, dg, fz.n_fac, win.w);
+  require(lds <= lds_max, FFSIM_ERR_VALUE, "pipelined tile exceeds LDS");
+  constexpr int W2 = kMaxSubWindow;
+  auto kern = fuse ? fiber_pipe_kernel<T, W2, true, false, true>
+              : tstore ? (dg ? fiber_pipe_kernel<T, W2, true, true, false>
+                             : fiber_pipe_kernel<T, W2, true, false, false>)
+                       : (dg ? fiber_pipe_kernel<T, W2, false, true, false>
+                             : fiber_pipe_kernel<T, W2, false, false, false>);
+  const DevSchedule& sched = dev_schedule(context(), gr, kPipeCompute, W);
+  static bool attr_set[5] = {};
+  const int variant = fuse ? 4 : 2 * tstore + dg;
+  if (!attr_set[variant]) {
+    HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)lds_max));
+    attr_set[variant] = true;
+  }
+  const long n_tiles = (long)((n_batch + W - 1) / W) * n_f;
+  const long grid = std::min<long>(n_tiles, g_n_cu);
+  const double moved = 2.0 * (double)sizeof(Cx<T>) * (double)n_batch *
+                       (double)(all_fibers ? win.rows_all : win.rows_active);
+  const long pk = prof_start(PROF_FIBER, moved, stream);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kPipeThreads), lds, stream,
+                     reinterpret_cast<const Cx<T>*>(src), reinterpret_cast<Cx<T>*>(dst), ld_src,
+                     ld_dst, n_batch, win.fibers, n_f, win.rows, gr.args(sched), los, d_subs, n_sub,
+                     d_layers, d_diag, d_strings, win.lo, win.w, gd_cap, gm_cap, cfac, fz);
+  HIP_CHECK(hipGetLastError());
+  prof_stop(pk, stream);
+}
+
 template <typename T>
 void launch_fiber_multi(int mode, const MultiTiles& mt, long ld, int n_batch,
                         const DevWindow& win, bool all_fibers, const DevGroups& gr,
@@ -951,6 +1055,7 @@ std::pair<size_t, size_t> append_diag_params(Program& prog, const DiagSpec& spec
 struct FuseTables {
   size_t bfac_off = 0, rfac_off = 0;
   int n_fac = 0;
+  bool columns_later = false;  // pipelined: the tile strings' own factor is left to the next gate
 };
 
 // The sub-window slots of a pass and the largest group tables that any fiber
@@ -977,10 +1082,18 @@ void pass_slots(const DevGroups& gr, const std::vector<SubPass>& subs, LoSlots& 
   }
 }
 
+// Orbital phases of one (the factor tables of a pass without phases of its own).
+size_t append_unit_phases(Program& prog, int norb) {
+  std::vector<double> one(2 * (size_t)norb, 0.0);
+  for (int k = 0; k < norb; ++k) one[2 * k] = 1.0;
+  return prog.append(one.data(), one.size() * sizeof(double));
+}
+
 void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, long ld,
                 int n_batch, int norb, int nocc, const SectorRotation& rot, void* tstore_dst,
                 long ld_t, hipStream_t stream, std::vector<std::function<void()>>& launches,
-                const FuseTables* fuse = nullptr, bool* fused = nullptr) {
+                const FuseTables* fuse = nullptr, bool* fused = nullptr,
+                const size_t* cfac_off = nullptr) {
   if (fused) *fused = false;
   const int w = (mode == MODE_COLS) ? norb : choose_window(ctx, norb, nocc, dtype);
   const bool tstore = tstore_dst != nullptr;
@@ -1018,11 +1131,37 @@ void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, l
     void* dst = ts ? tstore_dst : state;
     const long ld_dst = ts ? ld_t : ld;
     const bool all = ts || dg;
+    if (mode == MODE_ROWS && pipe_applies(ctx, dtype, win, all, gr, n_batch)) {
+      const bool fz_pipe = ts && fuse && fuse->columns_later;
+      if (fz_pipe && fused) *fused = true;
+      const FuseTables fp = fz_pipe ? *fuse : FuseTables{};
+      const bool cf = ts && cfac_off;
+      const size_t coff = cf ? *cfac_off : 0;
+      if (cf && !dg) diag_off = append_unit_phases(prog, norb);
+      const bool ph = dg || cf;
+      launches.push_back([=, &ctx, &prog, &win, &gr, &ds]() {
+        PipeFuse pf{nullptr, 0};
+        if (fz_pipe) pf = PipeFuse{prog.scratch<Cx<double>>(fp.bfac_off), fp.n_fac};
+        const Cx<double>* c = cf ? prog.scratch<Cx<double>>(coff) : nullptr;
+        auto launch = [&](auto tag) {
+          launch_fiber_pipe<decltype(tag)>(
+              state, dst, ld, ld_dst, n_batch, ts, win, all, gr, los, gd_cap, gm_cap,
+              prog.dev<SubPass>(poff), n_sub, prog.dev<LayerPair>(soff),
+              ph ? prog.dev<double>(diag_off) : nullptr, ds.d, c, pf, ctx.lds_max, stream);
+        };
+        if (dtype == FFSIM_C128)
+          launch(double{});
+        else
+          launch(float{});
+      });
+      continue;
+    }
+    require(!(ts && cfac_off), FFSIM_ERR_VALUE, "column factors need a pipelined pass");
     // fuse the diagonal into this pass when the kernel's fused layout applies
     bool fz_on = false;
     // (the fused store takes the pass's window to be [0, w), w <= 16)
     const int wf = dtype == FFSIM_C128 ? 8 : 4;
-    if (ts && fuse && mode == MODE_ROWS && tile_width(dtype) == wf && gr.w2 == kMaxSubWindow &&
+    if (ts && fuse && !fuse->columns_later && mode == MODE_ROWS && tile_width(dtype) == wf && gr.w2 == kMaxSubWindow &&
         n_sub > 0 && P.lo == 0 && w <= 16) {
       const int rows = win.max_rows;
       const size_t lds = fiber_lds_bytes(elem_bytes(dtype), wf, false, 16, rows, gd_cap, gm_cap,
@@ -1055,18 +1194,42 @@ long transposed_ld(int dtype, long dim_a) {
   return (dim_a + q - 1) / q * q;
 }
 
+// What became of the diagonal evolution that follows a rotation.
+enum class Fused { kNo, kYes, kAllButColumns };
+
+// Whether the fused diagonal of this shape runs in the pipelined kernel: both
+// transposing passes (the beta sector's, which applies it, and the alpha
+// sector's of the next rotation, which applies the factor it leaves) do.
+bool pipe_fuse_applies(Context& ctx, int dtype, int norb, int na, int nb, int w_a, int w_b,
+                       int n_fac) {
+  const int W = pipe_tile_width(dtype);
+  const DevGroups& ga = dev_groups(ctx, w_a, dtype == FFSIM_C64);
+  const DevGroups& gb = dev_groups(ctx, w_b, dtype == FFSIM_C64);
+  if (!pipe_applies(ctx, dtype, dev_window(ctx, norb, na, 0, w_a), true, ga, (long)binom(norb, nb)) ||
+      !pipe_applies(ctx, dtype, dev_window(ctx, norb, nb, 0, w_b), true, gb, (long)binom(norb, na)))
+    return false;
+  int gd = 0, gm = 0;
+  group_caps(gb, gd, gm);
+  return W * n_fac <= 512 &&
+         pipe_lds_bytes(W, gd, gm, true, true, n_fac, w_b) <= ctx.lds_max;
+}
+
 // Full spinful orbital rotation (both sectors) on a dim_a x dim_b state.
 // With `then_diag`, the diagonal Coulomb evolution that follows the rotation is
 // fused into the final pass when that pass is a transposing c128 row pass and
-// everything fits; returns true when it was (the caller applies it otherwise).
+// everything fits; says whether it was (the caller applies it otherwise).  With
+// may_leave_columns (the caller's next gate is a rotation of both sectors) it
+// may leave out the factor of the beta strings alone: the next call then gets
+// the same spec as left_columns.
 // ld_w: row pitch of the transposed state in `work` (0: transposed_ld, the
 // layout ffsim_orbital_rotation_work_elements sizes the buffer for).
-bool orbital_rotation_impl(Context& ctx, void* vec, void* work, int dtype, int norb, int na,
-                           int nb, const cdouble* mat_a, const cdouble* mat_b,
-                           hipStream_t stream, const DiagSpec* then_diag = nullptr,
-                           long ld_w = 0) {
+Fused orbital_rotation_impl(Context& ctx, void* vec, void* work, int dtype, int norb, int na,
+                            int nb, const cdouble* mat_a, const cdouble* mat_b,
+                            hipStream_t stream, const DiagSpec* then_diag = nullptr,
+                            long ld_w = 0, bool may_leave_columns = false,
+                            const DiagSpec* left_columns = nullptr) {
   const long dim_a = (long)binom(norb, na), dim_b = (long)binom(norb, nb);
-  if (dim_a == 0 || dim_b == 0 || norb == 0) return false;
+  if (dim_a == 0 || dim_b == 0 || norb == 0) return Fused::kNo;
   require(dim_a < (1l << 31) && dim_b < (1l << 31), FFSIM_ERR_VALUE, "dimension too large");
   const bool beta_cols = beta_in_columns(norb, dim_b, dtype, ctx);
   const int w_a = choose_window(ctx, norb, na, dtype);
@@ -1094,8 +1257,25 @@ bool orbital_rotation_impl(Context& ctx, void* vec, void* work, int dtype, int n
                    norb + 1 <= 64;
   if (want_fuse) {
     ft.n_fac = norb + 1;
+    ft.columns_later = may_leave_columns &&
+                       pipe_fuse_applies(ctx, dtype, norb, na, nb, w_a, w_b, ft.n_fac);
     want_fuse = prog.reserve((size_t)dim_a * ft.n_fac * sizeof(Cx<double>), &ft.bfac_off) &&
-                prog.reserve((size_t)dim_b * sizeof(Cx<double>), &ft.rfac_off);
+                (ft.columns_later ||
+                 prog.reserve((size_t)dim_b * sizeof(Cx<double>), &ft.rfac_off));
+  }
+  // the previous gate's diagonal left its factor of the beta strings alone to
+  // this rotation: the last alpha pass multiplies its columns by it
+  size_t cfac_off = 0;
+  if (left_columns) {
+    require(beta_transposed && prog.reserve((size_t)dim_b * sizeof(Cx<double>), &cfac_off),
+            FFSIM_ERR_VALUE, "column factors: no scratch");
+    const auto [hoff, coff] = append_diag_params(prog, *left_columns);
+    const DevStrings& sb = dev_strings(ctx, norb, nb);
+    launches.push_back([=, &prog, &sb, h = hoff, c = coff]() {
+      launch_diag_col_term(dim_b, sb.d, prog.dev<DiagHeader>(h), prog.dev<double>(c),
+                           prog.scratch<double>(cfac_off), 1, stream);
+      HIP_CHECK(hipGetLastError());
+    });
   }
   if (want_fuse) {
     const std::pair<size_t, size_t> par = append_diag_params(prog, *then_diag);
@@ -1103,12 +1283,14 @@ bool orbital_rotation_impl(Context& ctx, void* vec, void* work, int dtype, int n
     const DevStrings& sa = dev_strings(ctx, norb, na);
     const DevStrings& sb = dev_strings(ctx, norb, nb);
     const int nf = ft.n_fac;
+    const bool later = ft.columns_later;
     launches.push_back([=, &prog, &sa, &sb]() {
       const long n_a = dim_a * nf;
       hipLaunchKernelGGL(diag_row_factor_kernel, dim3((unsigned)((n_a + 255) / 256)), dim3(256),
                          0, stream, (int)dim_a, sa.d, prog.dev<DiagHeader>(hoff),
                          prog.dev<double>(coff), prog.scratch<Cx<double>>(ft.bfac_off));
       HIP_CHECK(hipGetLastError());
+      if (later) return;
       hipLaunchKernelGGL(diag_col_term_kernel, dim3((unsigned)((dim_b + 255) / 256)), dim3(256),
                          0, stream, (int)dim_b, sb.d, prog.dev<DiagHeader>(hoff),
                          prog.dev<double>(coff), prog.scratch<double>(ft.rfac_off), 1, 0l, 0l);
@@ -1120,7 +1302,8 @@ bool orbital_rotation_impl(Context& ctx, void* vec, void* work, int dtype, int n
     SectorRotation empty;
     const SectorRotation& r = mat_a ? ra : empty;
     run_sector(ctx, prog, dtype, MODE_ROWS, vec, dim_b, (int)dim_b, norb, na, r,
-               beta_transposed ? work : nullptr, ld_w, stream, launches);
+               beta_transposed ? work : nullptr, ld_w, stream, launches, nullptr, nullptr,
+               left_columns ? &cfac_off : nullptr);
   }
   if (mat_b) {
     if (beta_cols) {
@@ -1134,7 +1317,7 @@ bool orbital_rotation_impl(Context& ctx, void* vec, void* work, int dtype, int n
   prog.commit();
   for (auto& f : launches) f();
   prog.finish();
-  return fused;
+  return !fused ? Fused::kNo : ft.columns_later ? Fused::kAllButColumns : Fused::kYes;
 }
 
 
@@ -1260,18 +1443,24 @@ void diag_coulomb_sequence_impl(Context& ctx, void* vec, void* work, int dtype, 
                                 int nb, int n_terms, const cdouble* const* rots,
                                 const double* const* mats /* aa, ab, bb per term (3 ptrs) */,
                                 const double* times, int z_rep, hipStream_t st, long ld_w = 0) {
+  DiagSpec left_spec;  // a fused diagonal's factor of the beta strings, left to the next rotation
+  bool left = false;
   for (int t = 0; t < n_terms; ++t) {
     DiagSpec s = diag_coulomb_spec(norb, mats[3 * t], mats[3 * t + 1], mats[3 * t + 2], z_rep,
                                    times[t]);
-    bool fused = false;
+    Fused fused = Fused::kNo;
     if (rots[t])
       fused = orbital_rotation_impl(ctx, vec, work, dtype, norb, na, nb, rots[t], rots[t], st,
-                                    s.flags ? &s : nullptr, ld_w);
-    if (s.flags && !fused) diag_impl(ctx, DIAG_EVOLVE, vec, vec, dtype, norb, na, nb, s, st);
+                                    s.flags ? &s : nullptr, ld_w, rots[t + 1] != nullptr,
+                                    left ? &left_spec : nullptr);
+    left = fused == Fused::kAllButColumns;
+    if (left) left_spec = s;
+    if (s.flags && fused == Fused::kNo)
+      diag_impl(ctx, DIAG_EVOLVE, vec, vec, dtype, norb, na, nb, s, st);
   }
   if (rots[n_terms])
     orbital_rotation_impl(ctx, vec, work, dtype, norb, na, nb, rots[n_terms], rots[n_terms], st,
-                          nullptr, ld_w);
+                          nullptr, ld_w, false, left ? &left_spec : nullptr);
 }
 
 std::vector<cdouble> matmul(const cdouble* A, const cdouble* B, int n, bool adj_a) {
