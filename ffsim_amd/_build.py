@@ -5,13 +5,16 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libffsim_amd.so"
 
-SOURCES = ["ffsim_amd.hip", "noalloc.hip", "host_core.cpp"]
+SOURCES = ["ffsim_amd.hip", "fiber_pipe_c128.hip", "fiber_pipe_c64.hip", "noalloc.hip",
+           "host_core.cpp"]
 HEADERS = ["kernels.hpp", "fiber_pipe.hpp", "host_core.hpp", "status.hpp", "diag_params.hpp"]
 
 
@@ -23,15 +26,13 @@ def hipcc() -> str:
 
 
 def build(verbose: bool = False) -> Path:
-    """Compile libffsim_amd.so for gfx950 (always recompiles)."""
+    """Compile libffsim_amd.so for gfx950 (always recompiles), one object per source at once."""
     tmp = LIB_PATH.with_suffix(".so.tmp")
-    cmd = [
-        hipcc(),
+    flags = [
         "-O3",
         "-std=c++17",
         "--offload-arch=gfx950",
         "-fPIC",
-        "-shared",
         # keep the compiler from forming packed FP32 instructions
         "-Xclang",
         "-target-feature",
@@ -39,18 +40,22 @@ def build(verbose: bool = False) -> Path:
         "-packed-fp32-ops",
         "-Wall",
         "-Wno-unused-function",
-        *[str(CSRC / s) for s in SOURCES],
-        "-L/opt/rocm/lib",
-        "-lrocblas",
-        "-Wl,-rpath,/opt/rocm/lib",
-        "-o",
-        str(tmp),
     ]
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + res.stdout + res.stderr)
-    if verbose:
-        print(res.stderr)
+
+    def run(args):
+        res = subprocess.run([hipcc(), *args], capture_output=True, text=True)
+        if res.returncode != 0:
+            raise RuntimeError("hipcc failed:\n" + res.stdout + res.stderr)
+        if verbose:
+            print(res.stderr)
+
+    with tempfile.TemporaryDirectory() as objs:
+        targets = [(str(CSRC / s), str(Path(objs) / (s + ".o"))) for s in SOURCES]
+        with ThreadPoolExecutor(len(targets)) as pool:
+            for job in [pool.submit(run, [*flags, "-c", src, "-o", obj]) for src, obj in targets]:
+                job.result()
+        run(["--offload-arch=gfx950", "-shared", *[obj for _, obj in targets], "-L/opt/rocm/lib",
+             "-lrocblas", "-Wl,-rpath,/opt/rocm/lib", "-o", str(tmp)])
     os.replace(tmp, LIB_PATH)
     return LIB_PATH
 

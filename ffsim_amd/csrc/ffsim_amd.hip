@@ -11,6 +11,7 @@
 #include <rocblas/rocblas.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <complex>
 #include <cstdlib>
@@ -195,6 +196,14 @@ struct ProgramRing {
   std::condition_variable freed;
 };
 
+// Tables of the pipelined passes over a window of w orbitals whose fibers hold
+// kp_lo..kp_hi electrons.
+struct DevPipe {
+  PipeGroups host;
+  uint32_t *desc = nullptr, *offs = nullptr, *chunks = nullptr;
+  int32_t *index = nullptr, *offs_index = nullptr, *wave_index = nullptr;
+};
+
 struct Context {
   // rocBLAS handle of the batched small-state path (created on first use;
   // calls that use it hold blas_mu, the handle being bound to one stream at a time)
@@ -216,6 +225,7 @@ struct Context {
   // once (created on first use, default priority)
   std::vector<hipStream_t> aux;
   std::map<int, std::pair<uint32_t*, int32_t*>> ob_links;
+  std::map<std::tuple<int, int, int, bool, int>, std::unique_ptr<DevPipe>> pipe;
   ProgramRing ring;
 };
 
@@ -444,6 +454,25 @@ const DevSchedule& dev_schedule(Context& ctx, const DevGroups& gr, int n_waves, 
   ds.chunks = upload_table(ws.chunks);
   ds.index = upload_table(ws.index);
   return g.schedules[key] = ds;
+}
+
+const DevPipe& dev_pipe(Context& ctx, int w, int kp_lo, int kp_hi, bool merge, int units,
+                        size_t elem) {
+  std::lock_guard<std::mutex> lk(ctx.mu);
+  const auto key = std::make_tuple(w, kp_lo, kp_hi, merge, units);
+  auto it = ctx.pipe.find(key);
+  if (it != ctx.pipe.end()) return *it->second;
+  auto dp = std::make_unique<DevPipe>();
+  dp->host = make_pipe_groups(w, kp_lo, kp_hi, merge, units, kPipeCompute,
+                              64 / pipe_width(units, elem));
+  const PipeGroups& T = dp->host;
+  dp->desc = upload_table(T.desc);
+  dp->offs = upload_table(T.offs);
+  dp->chunks = upload_table(T.chunks);
+  dp->index = upload_table(T.index);
+  dp->offs_index = upload_table(T.offs_index);
+  dp->wave_index = upload_table(T.wave_index);
+  return *(ctx.pipe[key] = std::move(dp));
 }
 
 size_t pow2_ceil(size_t x) {
@@ -719,106 +748,165 @@ void launch_fiber_t(const void* src, void* dst, long ld_src, long ld_dst, int n_
   prof_stop(pk, stream);
 }
 
+// Entries of a pipelined pass's tables in LDS, over the window's electron
+// counts: groups, member offsets and chunks of the given sub-window starts.
+struct PipeCaps {
+  int groups = 0, offsets = 0, chunks = 0;
+};
+PipeCaps pipe_caps(const PipeGroups& T, const int* lo2, int n) {
+  PipeCaps c;
+  for (int kp = 0; kp <= T.w; ++kp) {
+    int nd = 0, nc = 0;
+    for (int u = 0; u < n; ++u) {
+      const size_t set = (size_t)kp * T.n_lo2 + lo2[u];
+      nd += T.index[2 * set + 1];
+      for (int wv = 0; wv < kPipeCompute; ++wv)
+        nc += T.wave_index[(set * kPipeCompute + wv) * 2 + 1];
+    }
+    c.groups = std::max(c.groups, nd);
+    c.chunks = std::max(c.chunks, nc);
+  }
+  for (int u = 0; u < n; ++u) c.offsets += T.offs_index[2 * lo2[u] + 1];
+  return c;
+}
+
 // LDS of a pipelined launch, following the kernel's layout.
-size_t pipe_lds_bytes(int W, int gd_cap, int gm_cap, bool tstore, bool diag, int n_fac, int win) {
-  constexpr size_t R = kPipeMaxRows;
-  size_t b = (R + kPipeStep) * 128 + (tstore ? 0 : kPipeSlots * R * 4) +
-             kMaxLoSlots * sizeof(GroupSlot) + 2 * align16((size_t)gd_cap * 4) +
-             align16((size_t)gm_cap * 2) + (size_t)kMaxLoSlots * kPipeCompute * 8;
-  if (diag || n_fac) b += kPipeSlots * R * 2;
+size_t pipe_lds_bytes(int units, size_t elem, const PipeCaps& c, bool tstore, bool diag,
+                      int n_fac, int win) {
+  const size_t R = pipe_max_rows(units), W = pipe_width(units, elem);
+  const size_t slots = units < 8 ? 1 : kPipeSlots;
+  size_t b = (size_t)(pipe_sweeps(units) + 1) * 4096 + (tstore || units < 8 ? 0 : slots * R * 4) +
+             align16(kPipeMaxLo * sizeof(PipeSlot)) + align16((size_t)c.offsets * 4) +
+             align16((size_t)c.groups * 4) + (size_t)kPipeMaxLo * kPipeCompute * 8 +
+             align16((size_t)c.chunks * 4);
+  if (diag || n_fac) b += slots * R * 2;
   if (n_fac)
-    b += 16 + ((size_t)W * n_fac + (size_t)fuse_nibble_entries(win, W)) * sizeof(Cx<double>);
+    b += 16 + (W * n_fac + (size_t)fuse_nibble_entries(win, (int)W)) * sizeof(Cx<double>);
   else if (diag)
     b += 68 * sizeof(Cx<double>);
   return b;
 }
 
-int pipe_tile_width(int dtype) { return dtype == FFSIM_C128 ? pipe_width<double>() : pipe_width<float>(); }
-
-// The largest group tables any pass of this window can stage (every sub-window start).
-void group_caps(const DevGroups& gr, int& gd_cap, int& gm_cap) {
-  gd_cap = gm_cap = 0;
-  for (int kp = 0; kp <= gr.w; ++kp) {
-    int nd = 0, nm = 0;
-    for (int lo2 = 0; lo2 < gr.n_lo2; ++lo2) {
-      const int* ix = gr.host_index.data() + ((size_t)kp * gr.n_lo2 + lo2) * 4;
-      nd += ix[1];
-      nm += ix[3];
-    }
-    gd_cap = std::max(gd_cap, nd);
-    gm_cap = std::max(gm_cap, nm);
-  }
+// How the passes of a sector with strings on rows run: the window width, and
+// the 16-byte units per string of a pipelined tile (0: plain passes).
+//
+// Up to norb 16, a sector whose strings all fit one tile at some tile width
+// runs as one pass over all orbitals instead of three over 12-orbital windows:
+// a third of the traffic and of the launches, and 8 to 10 register sub-passes
+// instead of 10 to 12, for narrower segments in memory (64, 32 or 16 bytes of
+// a row; neighbouring tiles run on one XCD and share its L2).  Measured per
+// sector rotation, LUCJ: norb=13 (1716 strings, 4 complex128 columns) 160 ->
+// 107 us, norb=14 (3432, 2 columns) 449 -> 281 us, norb=15 (6435, 1 column)
+// 1614 -> 945 us; complex64 153 -> 81, 324 -> 220 and 1080 -> 810 us.
+struct SectorGeom {
+  int w = 0, units = 0;
+  bool whole = false;  // a tile holds every string of the sector (one pass)
+};
+int choose_window(Context& ctx, int norb, int nocc, int dtype);
+SectorGeom sector_geom(Context& ctx, int dtype, int norb, int nocc, long n_batch) {
+  SectorGeom g;
+  g.w = choose_window(ctx, norb, nocc, dtype);
+  const size_t elem = elem_bytes(dtype);
+  if (n_batch > (1l << 30) || tile_width(dtype) != (dtype == FFSIM_C64 ? 4 : 8)) return g;
+  if (norb > window_cap() && norb >= kMaxSubWindow && norb <= 16)
+    for (int units : {8, 4, 2, 1})
+      if ((long)binom(norb, nocc) <= pipe_max_rows(units) &&
+          n_batch >= pipe_width(units, elem)) {
+        g.w = norb;
+        g.units = units;
+        g.whole = true;
+        return g;
+      }
+  if (g.w >= kMaxSubWindow && g.w <= 16 && n_batch >= pipe_width(8, elem)) g.units = 8;
+  return g;
 }
 
 // Whether a row pass over these fibers runs pipelined (fiber_pipe_kernel).
-// Both kernels walk their tiles in rounds over the CUs, one pipelined tile per
-// CU against one plain complex128 tile or three plain complex64 tiles of a
-// quarter of the columns.  Measured on the LUCJ passes of norb 13 to 16: a
-// round takes about 17.6 / 21 us (complex128) and 25.6 / 21.5 us (complex64),
-// and a pipelined launch 16 us more to fill and drain, so it wins from 5
-// rounds on in complex128 (norb=15: 482 against 538 us per launch; norb=13
-// with 2 rounds: 58 against 53).  Fibers whose plain tiles leave room for a
-// second workgroup per CU gain nothing from it in complex128 (norb=16 (4,4),
-// 495 strings: 180 against 126 us).
-bool pipe_applies(Context& ctx, int dtype, const DevWindow& win, bool all_fibers,
-                  const DevGroups& gr, long n_batch) {
-  const int W = pipe_tile_width(dtype);
+// Whole-sector tiles always do.  For the others, both kernels walk their tiles
+// in rounds over the CUs, one pipelined tile per CU against one plain
+// complex128 tile or three plain complex64 tiles of a quarter of the columns.
+// Measured on the 12-orbital passes of norb 13 to 16: a round takes about 17.6
+// / 21 us (complex128) and 25.6 / 21.5 us (complex64), and a pipelined launch
+// 16 us more to fill and drain, so it wins from 5 rounds on in complex128 (25
+// rounds: 482 against 538 us per launch; 2 rounds: 58 against 53).  Fibers
+// whose plain tiles leave room for a second workgroup per CU gain nothing from
+// it in complex128 (norb=16 (4,4) in 12-orbital windows, 495 strings: 180
+// against 126 us).
+bool pipe_applies(Context& ctx, int dtype, const SectorGeom& g, const DevWindow& win,
+                  bool all_fibers, long n_batch) {
+  if (g.units == 0) return false;
+  if (g.whole) return true;
   const int rows = all_fibers ? win.max_rows : win.max_rows_active;
   const long n_f = all_fibers ? win.n_fibers : win.n_active;
-  if (gr.w2 != kMaxSubWindow || gr.n_lo2 > kMaxLoSlots || n_batch < W || win.w > 16 ||
-      rows > kPipeMaxRows || n_batch > (1l << 30))
-    return false;
+  if (rows > pipe_max_rows(8)) return false;
   const bool c128 = dtype == FFSIM_C128;
   if (c128 ? 2 * (size_t)rows * 128 <= ctx.lds_max : rows < 400) return false;
   auto rounds = [&](int width, long per_cu) {
     const long tiles = (n_batch + width - 1) / width * n_f;
     return (double)((tiles + per_cu * g_n_cu - 1) / (per_cu * g_n_cu));
   };
-  return (c128 ? 17.6 : 25.6) * rounds(W, 1) + 16.0 <
+  return (c128 ? 17.6 : 25.6) * rounds(pipe_width(8, elem_bytes(dtype)), 1) + 16.0 <
          (c128 ? 21.0 * rounds(8, 1) : 21.5 * rounds(4, 3));
 }
 
-template <typename T>
-void launch_fiber_pipe(const void* src, void* dst, long ld_src, long ld_dst, int n_batch,
-                       bool tstore, const DevWindow& win, bool all_fibers, const DevGroups& gr,
-                       const LoSlots& los, int gd_cap, int gm_cap, const SubPass* d_subs, int n_sub,
-                       const LayerPair* d_layers, const double* d_diag, const uint64_t* d_strings,
-                       const Cx<double>* cfac, const PipeFuse& fz, size_t lds_max,
-                       hipStream_t stream) {
-  constexpr int W = pipe_width<T>();
-  const int n_f = all_fibers ? win.n_fibers : win.n_active;
-  if (n_f == 0 || n_batch == 0) return;
-  const bool fuse = fz.bfac != nullptr;
-  const bool dg = !fuse && (d_diag != nullptr);
-  require(!tstore || win.lo == 0, FFSIM_ERR_VALUE, "pipelined pass: transposing window not at 0");
-  require(!fuse || tstore, FFSIM_ERR_VALUE, "pipelined pass: fused diagonal without transposition");
-  require(!cfac || (tstore && dg), FFSIM_ERR_VALUE, "pipelined pass: column factors");
-  const size_t lds = pipe_lds_bytes(W, gd_cap, gm_cap, tstore, dg, fz.n_fac, win.w);
+const DevPipe& sector_pipe(Context& ctx, int dtype, int norb, int nocc, const SectorGeom& g) {
+  return dev_pipe(ctx, g.w, std::max(1, nocc - (norb - g.w)), std::min(nocc, g.w - 1),
+                  dtype == FFSIM_C64, g.units, elem_bytes(dtype));
+}
+
+struct PipeLaunch {
+  const void* src;
+  void* dst;
+  long ld_src, ld_dst;
+  int n_batch;
+  bool tstore, all_fibers;
+  const SubPass* subs;
+  int n_sub;
+  const LayerPair* layers;
+  int n_layers;
+  const double* diag;
+  const uint64_t* strings;
+  const Cx<double>* cfac;
+  PipeFuse fz;
+};
+
+void pipe_pass(int dtype, int units, PipeLaunch L, const DevWindow& win, PipeTables tb,
+               const PipeCaps& caps, size_t lds_max, hipStream_t stream) {
+  const size_t elem = elem_bytes(dtype);
+  const int W = pipe_width(units, elem);
+  int n_f = L.all_fibers ? win.n_fibers : win.n_active;
+  if (n_f == 0 || L.n_batch == 0) return;
+  const bool fuse = L.fz.bfac != nullptr;
+  const bool dg = !fuse && L.diag != nullptr;
+  require(L.n_batch >= W && (L.all_fibers ? win.max_rows : win.max_rows_active) <=
+                                pipe_max_rows(units),
+          FFSIM_ERR_VALUE, "pipelined pass: shape");
+  require((!L.tstore && units == 8) || (win.lo == 0 && (units == 8 || win.n_fibers == 1)),
+          FFSIM_ERR_VALUE, "pipelined pass: rows not contiguous");
+  require(!fuse || L.tstore, FFSIM_ERR_VALUE, "pipelined pass: fused diagonal without transposition");
+  require(!L.cfac || (L.tstore && dg), FFSIM_ERR_VALUE, "pipelined pass: column factors");
+  const size_t lds = pipe_lds_bytes(units, elem, caps, L.tstore, dg, L.fz.n_fac, win.w);
   require(lds <= lds_max, FFSIM_ERR_VALUE, "pipelined tile exceeds LDS");
-  constexpr int W2 = kMaxSubWindow;
-  auto kern = fuse ? fiber_pipe_kernel<T, W2, true, false, true>
-              : tstore ? (dg ? fiber_pipe_kernel<T, W2, true, true, false>
-                             : fiber_pipe_kernel<T, W2, true, false, false>)
-                       : (dg ? fiber_pipe_kernel<T, W2, false, true, false>
-                             : fiber_pipe_kernel<T, W2, false, false, false>);
-  const DevSchedule& sched = dev_schedule(context(), gr, kPipeCompute, W);
-  static bool attr_set[5] = {};
-  const int variant = fuse ? 4 : 2 * tstore + dg;
-  if (!attr_set[variant]) {
-    HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)lds_max));
-    attr_set[variant] = true;
+  const int variant = fuse ? PIPE_FUSED : 2 * L.tstore + dg;
+  const void* kern = dtype == FFSIM_C128 ? pipe_kernel_c128(units, variant)
+                                         : pipe_kernel_c64(units, variant);
+  static std::atomic<bool> attr_set[2][9][PIPE_VARIANTS] = {};
+  if (!attr_set[dtype][units][variant]) {
+    HIP_CHECK(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max));
+    attr_set[dtype][units][variant] = true;
   }
-  const long n_tiles = (long)((n_batch + W - 1) / W) * n_f;
+  const long n_tiles = (long)((L.n_batch + W - 1) / W) * n_f;
   const long grid = std::min<long>(n_tiles, g_n_cu);
-  const double moved = 2.0 * (double)sizeof(Cx<T>) * (double)n_batch *
-                       (double)(all_fibers ? win.rows_all : win.rows_active);
+  const double moved = 2.0 * (double)elem * (double)L.n_batch *
+                       (double)(L.all_fibers ? win.rows_all : win.rows_active);
   const long pk = prof_start(PROF_FIBER, moved, stream);
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kPipeThreads), lds, stream,
-                     reinterpret_cast<const Cx<T>*>(src), reinterpret_cast<Cx<T>*>(dst), ld_src,
-                     ld_dst, n_batch, win.fibers, n_f, win.rows, gr.args(sched), los, d_subs, n_sub,
-                     d_layers, d_diag, d_strings, win.lo, win.w, gd_cap, gm_cap, cfac, fz);
-  HIP_CHECK(hipGetLastError());
+  int lo = win.lo, w = win.w, gd = caps.groups, go = caps.offsets, gc = caps.chunks;
+  const Fiber* fibers = win.fibers;
+  const int32_t* rows = win.rows;
+  void* args[] = {&L.src,   &L.dst,      &L.ld_src, &L.ld_dst,  &L.n_batch, &fibers, &n_f, &rows,
+                  &tb,      &L.subs,     &L.n_sub,  &L.layers,  &L.n_layers, &L.diag, &L.strings,
+                  &lo,      &w,          &gd,       &go,        &gc,        &L.cfac, &L.fz};
+  HIP_CHECK(hipLaunchKernel(kern, dim3((unsigned)grid), dim3(kPipeThreads), args, lds, stream));
   prof_stop(pk, stream);
 }
 
@@ -984,10 +1072,12 @@ std::vector<KStep> generic_steps(int n, bool triangle) {
 
 // Whether the passes of a sector rotation at window width w run the triangle
 // order: when it needs fewer window passes than ffsim's (Clements) order, or
-// as many with fewer layer pairs.  At 12-orbital windows that is norb 15, 17,
-// 18 and 20; at norb 18 it makes 30 fiber launches per LUCJ n_reps=4
-// application instead of 40 (measured 17% faster), while at norb 16 the
-// Clements order's fewer layer pairs measured 2% faster for complex64.
+// as many at a lower cost, a sub-pass (its LDS reads and writes and its
+// barrier) costing 2.5 layer pairs: norb 14 in one pass (32 layer pairs and 9
+// sub-passes against 30 and 10) measured 2.4% faster in the triangle order,
+// norb 16 in 12-orbital windows (42 and 12 against 39 and 13) 1% slower.  At
+// 12-orbital windows norb 17, 18 and 20 take it for the pass it saves (norb
+// 18: 30 launches per LUCJ n_reps=4 application instead of 40).
 // FFSIM_AMD_GIVENS_ORDER=clements or =triangle forces one order.
 bool triangle_order(int norb, int w) {
   const char* e = std::getenv("FFSIM_AMD_GIVENS_ORDER");
@@ -1001,7 +1091,7 @@ bool triangle_order(int norb, int w) {
     auto it = cache.find(key);
     if (it != cache.end()) return it->second;
   }
-  long cost[2][3];
+  long cost[2][2];
   for (int t = 0; t < 2; ++t) {
     std::vector<PlannedPass> passes = plan_passes(generic_steps(norb, t == 1), norb, w, true, -1);
     long lp = 0, sub = 0;
@@ -1013,10 +1103,9 @@ bool triangle_order(int norb, int w) {
       sub += (long)subs.size();
     }
     cost[t][0] = (long)passes.size();
-    cost[t][1] = lp;
-    cost[t][2] = sub;
+    cost[t][1] = 2 * lp + 5 * sub;
   }
-  const bool tri = std::lexicographical_compare(cost[1], cost[1] + 3, cost[0], cost[0] + 3);
+  const bool tri = std::lexicographical_compare(cost[1], cost[1] + 2, cost[0], cost[0] + 2);
   std::lock_guard<std::mutex> lk(mu);
   cache[key] = tri;
   return tri;
@@ -1095,12 +1184,12 @@ void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, l
                 const FuseTables* fuse = nullptr, bool* fused = nullptr,
                 const size_t* cfac_off = nullptr) {
   if (fused) *fused = false;
-  const int w = (mode == MODE_COLS) ? norb : choose_window(ctx, norb, nocc, dtype);
+  SectorGeom geom;
+  if (mode == MODE_ROWS) geom = sector_geom(ctx, dtype, norb, nocc, n_batch);
+  const int w = std::max(1, mode == MODE_COLS ? norb : geom.w);
   const bool tstore = tstore_dst != nullptr;
-  std::vector<PlannedPass> passes =
-      plan_passes(rot.steps, norb, std::max(w, 1), tstore, -1);
+  std::vector<PlannedPass> passes = plan_passes(rot.steps, norb, w, tstore, -1);
   const DevStrings& ds = dev_strings(ctx, norb, nocc);
-  const DevGroups& gr = dev_groups(ctx, std::max(w, 1), dtype == FFSIM_C64);
   const bool need_diag = !rot.trivial_diag;
   require(!need_diag || norb <= kMaxDiagOrbitals, FFSIM_ERR_VALUE, "norb above 64");
   size_t diag_off = 0;
@@ -1119,43 +1208,47 @@ void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, l
     const bool ts = last && tstore;
     const bool dg = last && need_diag;
     if (P.steps.empty() && !ts && !dg) continue;
-    plan_sub_passes(P.steps, std::max(w, 1), kMaxSubWindow, subs, sub_layers);
+    plan_sub_passes(P.steps, w, kMaxSubWindow, subs, sub_layers);
     const size_t soff = prog.append(sub_layers.data(), sub_layers.size() * sizeof(LayerPair));
     const size_t poff = prog.append(subs.data(), subs.size() * sizeof(SubPass));
     const int n_layers = (int)sub_layers.size();
     const int n_sub = (int)subs.size();
-    LoSlots los{};
-    int gd_cap = 0, gm_cap = 0;
-    pass_slots(gr, subs, los, gd_cap, gm_cap);
-    const DevWindow& win = dev_window(ctx, norb, nocc, P.lo, std::max(w, 1));
+    const DevWindow& win = dev_window(ctx, norb, nocc, P.lo, w);
     void* dst = ts ? tstore_dst : state;
     const long ld_dst = ts ? ld_t : ld;
     const bool all = ts || dg;
-    if (mode == MODE_ROWS && pipe_applies(ctx, dtype, win, all, gr, n_batch)) {
+    if (mode == MODE_ROWS && pipe_applies(ctx, dtype, geom, win, all, n_batch)) {
+      const DevPipe& dp = sector_pipe(ctx, dtype, norb, nocc, geom);
+      PipeTables tb{dp.desc,   dp.index,      dp.offs,       dp.offs_index,
+                    dp.chunks, dp.wave_index, dp.host.n_lo2, 0, {}};
+      for (const SubPass& sp : subs) {
+        require(sp.slot < kPipeMaxLo, FFSIM_ERR_VALUE, "too many sub-window starts");
+        tb.lo2[sp.slot] = sp.lo2;
+        tb.n_slots = std::max(tb.n_slots, sp.slot + 1);
+      }
+      const PipeCaps caps = pipe_caps(dp.host, tb.lo2, tb.n_slots);
       const bool fz_pipe = ts && fuse && fuse->columns_later;
       if (fz_pipe && fused) *fused = true;
       const FuseTables fp = fz_pipe ? *fuse : FuseTables{};
       const bool cf = ts && cfac_off;
       const size_t coff = cf ? *cfac_off : 0;
+      // (column factors ride on the phases of the pass: phases of one if it has none)
       if (cf && !dg) diag_off = append_unit_phases(prog, norb);
+      const size_t doff = diag_off;
       const bool ph = dg || cf;
-      launches.push_back([=, &ctx, &prog, &win, &gr, &ds]() {
-        PipeFuse pf{nullptr, 0};
-        if (fz_pipe) pf = PipeFuse{prog.scratch<Cx<double>>(fp.bfac_off), fp.n_fac};
-        const Cx<double>* c = cf ? prog.scratch<Cx<double>>(coff) : nullptr;
-        auto launch = [&](auto tag) {
-          launch_fiber_pipe<decltype(tag)>(
-              state, dst, ld, ld_dst, n_batch, ts, win, all, gr, los, gd_cap, gm_cap,
-              prog.dev<SubPass>(poff), n_sub, prog.dev<LayerPair>(soff),
-              ph ? prog.dev<double>(diag_off) : nullptr, ds.d, c, pf, ctx.lds_max, stream);
-        };
-        if (dtype == FFSIM_C128)
-          launch(double{});
-        else
-          launch(float{});
+      launches.push_back([=, &ctx, &prog, &win, &ds]() {
+        PipeLaunch L{state, dst, ld, ld_dst, n_batch, ts, all, prog.dev<SubPass>(poff), n_sub,
+                     prog.dev<LayerPair>(soff), n_layers, ph ? prog.dev<double>(doff) : nullptr,
+                     ds.d, cf ? prog.scratch<Cx<double>>(coff) : nullptr, PipeFuse{nullptr, 0}};
+        if (fz_pipe) L.fz = PipeFuse{prog.scratch<Cx<double>>(fp.bfac_off), fp.n_fac};
+        pipe_pass(dtype, geom.units, L, win, tb, caps, ctx.lds_max, stream);
       });
       continue;
     }
+    const DevGroups& gr = dev_groups(ctx, w, dtype == FFSIM_C64);
+    LoSlots los{};
+    int gd_cap = 0, gm_cap = 0;
+    pass_slots(gr, subs, los, gd_cap, gm_cap);
     require(!(ts && cfac_off), FFSIM_ERR_VALUE, "column factors need a pipelined pass");
     // fuse the diagonal into this pass when the kernel's fused layout applies
     bool fz_on = false;
@@ -1199,19 +1292,25 @@ enum class Fused { kNo, kYes, kAllButColumns };
 
 // Whether the fused diagonal of this shape runs in the pipelined kernel: both
 // transposing passes (the beta sector's, which applies it, and the alpha
-// sector's of the next rotation, which applies the factor it leaves) do.
-bool pipe_fuse_applies(Context& ctx, int dtype, int norb, int na, int nb, int w_a, int w_b,
-                       int n_fac) {
-  const int W = pipe_tile_width(dtype);
-  const DevGroups& ga = dev_groups(ctx, w_a, dtype == FFSIM_C64);
-  const DevGroups& gb = dev_groups(ctx, w_b, dtype == FFSIM_C64);
-  if (!pipe_applies(ctx, dtype, dev_window(ctx, norb, na, 0, w_a), true, ga, (long)binom(norb, nb)) ||
-      !pipe_applies(ctx, dtype, dev_window(ctx, norb, nb, 0, w_b), true, gb, (long)binom(norb, na)))
+// sector's of the next rotation, which applies the factor it leaves) do, with
+// room for their tables whatever sub-windows a rotation uses.
+bool pipe_fuse_applies(Context& ctx, int dtype, int norb, int na, int nb, int n_fac) {
+  const long da = (long)binom(norb, na), db = (long)binom(norb, nb);
+  const SectorGeom ga = sector_geom(ctx, dtype, norb, na, db);
+  const SectorGeom gb = sector_geom(ctx, dtype, norb, nb, da);
+  if (!pipe_applies(ctx, dtype, ga, dev_window(ctx, norb, na, 0, ga.w), true, db) ||
+      !pipe_applies(ctx, dtype, gb, dev_window(ctx, norb, nb, 0, gb.w), true, da))
     return false;
-  int gd = 0, gm = 0;
-  group_caps(gb, gd, gm);
-  return W * n_fac <= 512 &&
-         pipe_lds_bytes(W, gd, gm, true, true, n_fac, w_b) <= ctx.lds_max;
+  const size_t elem = elem_bytes(dtype);
+  int lo2[kPipeMaxLo];
+  for (int k = 0; k < kPipeMaxLo; ++k) lo2[k] = k;
+  auto caps = [&](int nocc, const SectorGeom& g) {
+    const PipeGroups& T = sector_pipe(ctx, dtype, norb, nocc, g).host;
+    return pipe_caps(T, lo2, T.n_lo2);
+  };
+  return pipe_width(gb.units, elem) * n_fac <= 512 &&
+         pipe_lds_bytes(ga.units, elem, caps(na, ga), true, true, 0, ga.w) <= ctx.lds_max &&
+         pipe_lds_bytes(gb.units, elem, caps(nb, gb), true, true, n_fac, gb.w) <= ctx.lds_max;
 }
 
 // Full spinful orbital rotation (both sectors) on a dim_a x dim_b state.
@@ -1232,8 +1331,8 @@ Fused orbital_rotation_impl(Context& ctx, void* vec, void* work, int dtype, int 
   if (dim_a == 0 || dim_b == 0 || norb == 0) return Fused::kNo;
   require(dim_a < (1l << 31) && dim_b < (1l << 31), FFSIM_ERR_VALUE, "dimension too large");
   const bool beta_cols = beta_in_columns(norb, dim_b, dtype, ctx);
-  const int w_a = choose_window(ctx, norb, na, dtype);
-  const int w_b = beta_cols ? norb : choose_window(ctx, norb, nb, dtype);
+  const int w_a = sector_geom(ctx, dtype, norb, na, dim_b).w;
+  const int w_b = beta_cols ? norb : sector_geom(ctx, dtype, norb, nb, dim_a).w;
   if (ld_w == 0) ld_w = transposed_ld(dtype, dim_a);
   require(ld_w >= dim_a, FFSIM_ERR_VALUE, "work row pitch below dim_a");
   SectorRotation ra, rb;
@@ -1258,7 +1357,7 @@ Fused orbital_rotation_impl(Context& ctx, void* vec, void* work, int dtype, int 
   if (want_fuse) {
     ft.n_fac = norb + 1;
     ft.columns_later = may_leave_columns &&
-                       pipe_fuse_applies(ctx, dtype, norb, na, nb, w_a, w_b, ft.n_fac);
+                       pipe_fuse_applies(ctx, dtype, norb, na, nb, ft.n_fac);
     want_fuse = prog.reserve((size_t)dim_a * ft.n_fac * sizeof(Cx<double>), &ft.bfac_off) &&
                 (ft.columns_later ||
                  prog.reserve((size_t)dim_b * sizeof(Cx<double>), &ft.rfac_off));

@@ -37,14 +37,52 @@ typedef u32x4 u32x4_a8 __attribute__((aligned(8)));
 constexpr int kPipeCompute = 8;  // compute waves
 constexpr int kPipeMemory = 4;   // memory waves
 constexpr int kPipeThreads = 64 * (kPipeCompute + kPipeMemory);
-constexpr int kPipeUnits = 8;    // 16-byte units of a string's batch in a tile (128 bytes)
-constexpr int kPipeStep = 64 * kPipeMemory / kPipeUnits;  // strings per sweep of the memory waves
-constexpr int kPipeSweeps = 29;  // 116 registers; 28 would not hold a 12-orbital fiber of 924
-constexpr int kPipeMaxRows = kPipeStep * kPipeSweeps;  // 928 >= C(12, 6)
 constexpr int kPipeSlots = 3;    // fibers whose rows are in LDS at once
+constexpr int kPipeMaxLo = 11;   // sub-window starts of a 16-orbital window
 
-template <typename T>
-constexpr int pipe_width() { return 128 / (int)sizeof(Cx<T>); }
+// Geometry of a tile with `units` 16-byte units per string: 8 for windows of
+// part of the orbitals (128-byte segments), and fewer where that lets a tile
+// hold every string of a sector, whose rotation is then a single pass.
+// A sweep is one 16-byte access of every memory lane.
+constexpr int pipe_step(int units) { return 64 * kPipeMemory / units; }  // strings per sweep
+constexpr int pipe_sweeps(int units) { return units == 8 ? 29 : units == 1 ? 26 : 27; }
+constexpr int pipe_max_rows(int units) { return pipe_step(units) * pipe_sweeps(units); }
+constexpr int pipe_width(int units, size_t elem) { return units * 16 / (int)elem; }
+
+// Tables of a pipelined pass (PipeGroups in device memory) and the distinct
+// sub-window starts that its sub-passes use.
+struct PipeTables {
+  const uint32_t* desc;
+  const int32_t* index;
+  const uint32_t* offs;
+  const int32_t* offs_index;
+  const uint32_t* chunks;
+  const int32_t* wave_index;
+  int n_lo2;
+  int n_slots;
+  int lo2[kPipeMaxLo];
+};
+struct PipeSlot {
+  int d_off;  // first group of this sub-window start in LDS
+  int o_off;  // first member offset
+};
+
+// Applies the layer pairs of one sub-pass to one register group (one batch
+// column): p is the group's base address in the tile, off its members' offsets.
+template <typename T, int W2, int K2>
+__device__ __forceinline__ void pipe_group_apply(unsigned char* p, const uint32_t* __restrict__ off,
+                                                 const LayerPair* lp, int n_lp, bool flip) {
+  constexpr int N = binom_const(W2, K2);
+  Cx<T> v[N];
+  Cx<T>* at[N];
+#pragma unroll
+  for (int m = 0; m < N; ++m) at[m] = reinterpret_cast<Cx<T>*>(p + off[m]);
+#pragma unroll
+  for (int m = 0; m < N; ++m) v[m] = *at[m];
+  apply_layers<T, W2, K2>(v, lp, n_lp, flip);
+#pragma unroll
+  for (int m = 0; m < N; ++m) *at[m] = v[m];
+}
 
 // A diagonal Coulomb evolution fused into the store of a transposing pass,
 // without its factor of the tile's strings alone (that one commutes with
@@ -55,39 +93,47 @@ struct PipeFuse {
   int n_fac;               // norb + 1
 };
 
-template <typename T, int W2, bool TST, bool DG, bool FUSE>
+// UNITS: 16-byte units per string.  TST: store the transposed state (rows of a
+// window [0, w), contiguous).  DG: multiply by the orbital phases (and cfac, a
+// factor per column).  FUSE: multiply by a diagonal evolution, transposing.
+// Tiles of fewer than 8 units hold a whole sector (contiguous rows, one fiber).
+template <typename T, int UNITS, bool TST, bool DG, bool FUSE>
 __global__ void __launch_bounds__(kPipeThreads)
     fiber_pipe_kernel(const Cx<T>* src, Cx<T>* dst, long ld_src, long ld_dst, int n_batch,
                       const Fiber* __restrict__ fibers, int n_fibers,
-                      const int32_t* __restrict__ row_table, GroupArgs ga, LoSlots los,
+                      const int32_t* __restrict__ row_table, PipeTables tb,
                       const SubPass* __restrict__ subs_g, int n_sub,
-                      const LayerPair* __restrict__ layers_g, const double* __restrict__ diag,
-                      const uint64_t* __restrict__ strings, int win_lo, int win_w, int gd_cap,
-                      int gm_cap, const Cx<double>* __restrict__ cfac, PipeFuse fz) {
+                      const LayerPair* __restrict__ layers_g, int n_layers,
+                      const double* __restrict__ diag, const uint64_t* __restrict__ strings,
+                      int win_lo, int win_w, int gd_cap, int go_cap, int gc_cap,
+                      const Cx<double>* __restrict__ cfac, PipeFuse fz) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  constexpr int W = pipe_width<T>();
-  constexpr int EU = W / kPipeUnits;  // elements of a unit
+  constexpr int W2 = kMaxSubWindow;
+  constexpr int W = pipe_width(UNITS, sizeof(Cx<T>));
+  constexpr int EU = W / UNITS;  // elements of a unit
   constexpr int NW = kPipeCompute;
-  constexpr int R = kPipeMaxRows;
+  constexpr int STEP = pipe_step(UNITS), SWEEPS = pipe_sweeps(UNITS);
+  constexpr int R = STEP * SWEEPS;
+  constexpr bool CONTIG = TST || UNITS < 8;  // rows row0, row0 + 1, ...
+  constexpr int SLOTS = UNITS < 8 ? 1 : kPipeSlots;
   size_t off = 0;
-  Cx<T>* tile = reinterpret_cast<Cx<T>*>(smem_raw);
   u32x4* tile4 = reinterpret_cast<u32x4*>(smem_raw);
-  off += (size_t)(R + kPipeStep) * 128;
+  off += (size_t)(SWEEPS + 1) * 4096;
   int32_t* rslot = reinterpret_cast<int32_t*>(smem_raw + off);
-  if (!TST) off += (size_t)kPipeSlots * R * sizeof(int32_t);
-  GroupSlot* gslot = reinterpret_cast<GroupSlot*>(smem_raw + off);
-  off += (size_t)kMaxLoSlots * sizeof(GroupSlot);
+  if (!CONTIG) off += (size_t)SLOTS * R * sizeof(int32_t);
+  PipeSlot* gslot = reinterpret_cast<PipeSlot*>(smem_raw + off);
+  off += align16((size_t)kPipeMaxLo * sizeof(PipeSlot));
+  uint32_t* goff = reinterpret_cast<uint32_t*>(smem_raw + off);
+  off += align16((size_t)go_cap * sizeof(uint32_t));
   uint32_t* gdesc = reinterpret_cast<uint32_t*>(smem_raw + off);
   off += align16((size_t)gd_cap * sizeof(uint32_t));
-  uint16_t* gmem = reinterpret_cast<uint16_t*>(smem_raw + off);
-  off += align16((size_t)gm_cap * sizeof(uint16_t));
   int32_t* wsched = reinterpret_cast<int32_t*>(smem_raw + off);
-  off += (size_t)kMaxLoSlots * NW * 2 * sizeof(int32_t);
+  off += (size_t)kPipeMaxLo * NW * 2 * sizeof(int32_t);
   uint32_t* wchunks = reinterpret_cast<uint32_t*>(smem_raw + off);
-  off += align16((size_t)gd_cap * sizeof(uint32_t));
+  off += align16((size_t)gc_cap * sizeof(uint32_t));
   // launches that multiply by orbital phases or a fused diagonal
   uint16_t* lbits = reinterpret_cast<uint16_t*>(smem_raw + off);
-  if (DG || FUSE) off += (size_t)kPipeSlots * R * sizeof(uint16_t);
+  if (DG || FUSE) off += (size_t)SLOTS * R * sizeof(uint16_t);
   Cx<double>* ptab = reinterpret_cast<Cx<double>*>(smem_raw + off);  // phases per nibble pattern
   if (DG) off += 64 * sizeof(Cx<double>);
   Cx<double>* pout = reinterpret_cast<Cx<double>*>(smem_raw + off);  // phase outside the window
@@ -113,41 +159,44 @@ __global__ void __launch_bounds__(kPipeThreads)
     const int lane = tid & 63;
     constexpr int NTC = 64 * kPipeCompute;
     auto stage_tables = [&](int kp) {
-      int d_base = 0, m_base = 0, c_base = 0;
-      for (int u = 0; u < los.n; ++u) {
-        const int* ix = ga.index + (kp * ga.n_lo2 + los.lo2[u]) * 4;
-        const int d0 = ix[0], nd = ix[1], m0 = ix[2], nm = ix[3];
-        if (tid == 0) gslot[u] = GroupSlot{d_base, nd, {0, 0}};
-        for (int k = tid; k < nd; k += NTC) {
-          const uint32_t d = ga.desc[d0 + k];
-          gdesc[d_base + k] = ((((d >> 8) - (uint32_t)m0) + (uint32_t)m_base) << 8) | (d & 0xff);
-        }
-        for (int k = tid; k < nm; k += NTC) gmem[m_base + k] = ga.members[m0 + k];
-        const int32_t* wi = ga.wave_idx + ((kp * ga.n_lo2 + los.lo2[u]) * NW) * 2;
+      int d_base = 0, c_base = 0, o_base = 0;
+      for (int u = 0; u < tb.n_slots; ++u) {
+        const int set = kp * tb.n_lo2 + tb.lo2[u];
+        const int d0 = tb.index[2 * set], nd = tb.index[2 * set + 1];
+        if (tid == 0) gslot[u] = PipeSlot{d_base, o_base};
+        for (int k = tid; k < nd; k += NTC) gdesc[d_base + k] = tb.desc[d0 + k];
+        const int32_t* wi = tb.wave_index + (long)set * NW * 2;
         const int first = wi[0];
-        int total = 0;
-        for (int wv = 0; wv < NW; ++wv) total += wi[2 * wv + 1];
+        const int total = wi[2 * (NW - 1)] + wi[2 * (NW - 1) + 1] - first;
         if (tid < NW) {
           wsched[(u * NW + tid) * 2] = c_base + (wi[2 * tid] - first);
           wsched[(u * NW + tid) * 2 + 1] = wi[2 * tid + 1];
         }
-        for (int k = tid; k < total; k += NTC) wchunks[c_base + k] = ga.chunks[first + k];
+        for (int k = tid; k < total; k += NTC) wchunks[c_base + k] = tb.chunks[first + k];
         d_base += nd;
-        m_base += nm;
         c_base += total;
+        o_base += tb.offs_index[2 * tb.lo2[u] + 1];
       }
     };
     int kp = fibers[(int)(t / n_bt)].kp;
-    if (n_sub > 0) stage_tables(kp);
+    if (n_sub > 0) {
+      stage_tables(kp);
+      int o_base = 0;
+      for (int u = 0; u < tb.n_slots; ++u) {
+        const int o0 = tb.offs_index[2 * tb.lo2[u]], no = tb.offs_index[2 * tb.lo2[u] + 1];
+        for (int k = tid; k < no; k += NTC) goff[o_base + k] = tb.offs[o0 + k];
+        o_base += no;
+      }
+    }
     if (FUSE && tid == 0) *arrived = 0;
     __syncthreads();
     bool odd = true;  // where the tile lies (see exchange)
     while (true) {
-      Cx<T>* cur = tile + (odd ? kPipeStep * W : 0);
+      unsigned char* cur = smem_raw + (odd ? 4096 : 0);
       odd = !odd;
       for (int sp = 0; sp < n_sub; ++sp) {
         const SubPass P = subs_g[sp];
-        const GroupSlot gs = gslot[P.slot];
+        const PipeSlot gs = gslot[P.slot];
         const LayerPair* lp = layers_g + P.lp0;
         const int c0 = wsched[(P.slot * NW + wave) * 2];
         const int nc = wsched[(P.slot * NW + wave) * 2 + 1];
@@ -156,11 +205,18 @@ __global__ void __launch_bounds__(kPipeThreads)
           const int gl = lane / W, j = lane % W;
           if (gl < (int)(ch & 0xff)) {
             const uint32_t d = gdesc[gs.d_off + (int)(ch >> 8) + gl];
-            if constexpr (sizeof(T) == 4)
-              group_dispatch<T, W2>(d & 0x7f, (d >> 7) & 1, cur, W, j, gmem + (d >> 8), lp,
-                                    P.n_lp);
-            else
-              group_dispatch<T, W2>(d & 0xff, false, cur, W, j, gmem + (d >> 8), lp, P.n_lp);
+            unsigned char* p = cur + (d >> 16) * (16 * UNITS) + j * (int)sizeof(Cx<T>);
+            const uint32_t* mo = goff + gs.o_off + ((d >> 4) & 0xfff) * 4;
+            const bool flip = (d >> 3) & 1;
+            switch (d & 7) {
+              case 1: pipe_group_apply<T, W2, 1>(p, mo, lp, P.n_lp, flip); break;
+              case 2: pipe_group_apply<T, W2, 2>(p, mo, lp, P.n_lp, flip); break;
+              case 3: pipe_group_apply<T, W2, 3>(p, mo, lp, P.n_lp, flip); break;
+              // complex64 groups of 4 and 5 electrons are complemented ones of 2 and 1
+              case 4: if constexpr (sizeof(T) == 8) pipe_group_apply<T, W2, 4>(p, mo, lp, P.n_lp, flip); break;
+              case 5: if constexpr (sizeof(T) == 8) pipe_group_apply<T, W2, 5>(p, mo, lp, P.n_lp, flip); break;
+              default: break;
+            }
           }
         }
         __syncthreads();
@@ -181,7 +237,7 @@ __global__ void __launch_bounds__(kPipeThreads)
 
   // --------------------------------------------------------- memory waves
   const int m = tid - 64 * kPipeCompute;
-  const int u = m & (kPipeUnits - 1), i0 = m / kPipeUnits;
+  const int u = m & (UNITS - 1), i0 = m / UNITS;
   const int nt = (win_w + 3) >> 2;
   auto cmul = [](const Cx<double>& x, const Cx<double>& y) {
     return Cx<double>{x.re * y.re - x.im * y.im, x.re * y.im + x.im * y.re};
@@ -200,14 +256,14 @@ __global__ void __launch_bounds__(kPipeThreads)
   // what this thread needs of a fiber's strings (i = i0 + 32 k): their rows, and
   // their bits inside the window for the phases
   auto stage_rows = [&](const Fiber& fd, int slot) {
-    if constexpr (!TST || DG || FUSE) {
+    if constexpr (!CONTIG || DG || FUSE) {
 #pragma unroll 1
-      for (int k = 0; k < kPipeSweeps; ++k) {
-        const int i = i0 + k * kPipeStep;
+      for (int k = 0; k < SWEEPS; ++k) {
+        const int i = i0 + k * STEP;
         const int r = row_table[fd.row_off + min(i, fd.n_rows - 1)];
-        if constexpr (!TST) rslot[slot * kPipeMaxRows + i] = r;
+        if constexpr (!CONTIG) rslot[slot * R + i] = r;
         if constexpr (DG || FUSE)
-          lbits[slot * kPipeMaxRows + i] = (uint16_t)((strings[r] & win_mask) >> win_lo);
+          lbits[slot * R + i] = (uint16_t)((strings[r] & win_mask) >> win_lo);
       }
     }
     if constexpr (DG) {
@@ -292,7 +348,7 @@ __global__ void __launch_bounds__(kPipeThreads)
   };
   // memory instructions ahead of the compute waves' arithmetic
   __builtin_amdgcn_s_setprio(3);
-  u32x4 buf[kPipeSweeps];
+  u32x4 buf[SWEEPS];
   // first column of this thread's unit in the tile at column b0 (units that
   // reach past the last column are moved back: they then hold columns that
   // another unit stores, and the store skips those)
@@ -306,8 +362,8 @@ __global__ void __launch_bounds__(kPipeThreads)
     uint32_t row[K1 - K0];
 #pragma unroll
     for (int k = K0; k < K1; ++k)
-      row[k - K0] = TST ? (uint32_t)(row0 + min(first + k * step, nr - 1))
-                        : (uint32_t)rslot[slot * kPipeMaxRows + first + k * step];
+      row[k - K0] = CONTIG ? (uint32_t)(row0 + min(first + k * step, nr - 1))
+                        : (uint32_t)rslot[slot * R + first + k * step];
 #pragma unroll
     for (int k = K0; k < K1; ++k)
       buf[k] = *reinterpret_cast<const u32x4_a8*>(p + (uint64_t)row[k - K0] * (uint32_t)ld_src);
@@ -323,12 +379,12 @@ __global__ void __launch_bounds__(kPipeThreads)
       const int i = first + k * step;
       if (i < nr) {
         const uint32_t row =
-            TST ? (uint32_t)(row0 + i) : (uint32_t)rslot[slot * kPipeMaxRows + i];
+            CONTIG ? (uint32_t)(row0 + i) : (uint32_t)rslot[slot * R + i];
         u32x4 q = buf[k];
         Cx<T> e[EU];
         __builtin_memcpy(e, &q, 16);
         if constexpr (DG || FUSE) {
-          const uint32_t bits = lbits[slot * kPipeMaxRows + i];
+          const uint32_t bits = lbits[slot * R + i];
           Cx<double> Q{1.0, 0.0};
           if constexpr (!FUSE) {
             Q = ptab[bits & 15];
@@ -380,7 +436,7 @@ __global__ void __launch_bounds__(kPipeThreads)
   // sweeps run from the last to the first.
   auto exchange = [&](uint32_t wr, uint32_t rd, int step) {
 #pragma unroll
-    for (int k = 0; k < kPipeSweeps; ++k) {
+    for (int k = 0; k < SWEEPS; ++k) {
       tile4[wr + k * step] = buf[k];
       asm volatile("" ::: "memory");
       buf[k] = tile4[rd + k * step];
@@ -415,16 +471,16 @@ __global__ void __launch_bounds__(kPipeThreads)
     const int f = more ? (int)(t / n_bt) : c_f;
     const int n_b0 = more ? (int)(t % n_bt) * W : c_b0;
     const Fiber fn = fibers[f];
-    int step = up ? -kPipeStep : kPipeStep, mv = m;
+    int step = up ? -STEP : STEP, mv = m;
     // (opaque: the compiler would otherwise keep the loop-invariant addresses
     // of every sweep in registers)
     asm volatile("" : "+s"(step), "+v"(mv));
-    const int first = (mv >> 3) + (up ? kPipeMaxRows - kPipeStep : 0);
-    const int p_first = (mv >> 3) + (up ? 0 : kPipeMaxRows - kPipeStep);
+    const int first = mv / UNITS + (up ? R - STEP : 0);
+    const int p_first = mv / UNITS + (up ? 0 : R - STEP);
     int n_slot = c_slot, n_row0 = c_row0;
     uint64_t n_fixed = c_fixed;
     if (f != c_f) {
-      n_slot = c_slot + 1 == kPipeSlots ? 0 : c_slot + 1;
+      n_slot = c_slot + 1 >= SLOTS ? 0 : c_slot + 1;
       stage_rows(fn, n_slot);
       n_row0 = row_table[fn.row_off];
       if (FUSE) n_fixed = strings[n_row0] & ~win_mask;
@@ -444,16 +500,15 @@ __global__ void __launch_bounds__(kPipeThreads)
     FFSIM_PORTION(4, 8, 2)
     FFSIM_PORTION(8, 12, 3)
     FFSIM_PORTION(12, 16, 4)
-    FFSIM_PORTION(16, 20, 5)
-    FFSIM_PORTION(20, 23, 6)
-    FFSIM_PORTION(23, 26, 7)
-    FFSIM_PORTION(26, 29, 8)
+    FFSIM_PORTION(16, 19, 5)
+    FFSIM_PORTION(19, 22, 6)
+    FFSIM_PORTION(22, 25, 7)
+    FFSIM_PORTION(25, SWEEPS, 8)
 #undef FFSIM_PORTION
     load_bfac(c_b0);
     upto(bars_per_tile);
     write_ffac();
-    exchange(mv + (up ? kPipeMaxRows : 0) * 8, mv + (up ? kPipeMaxRows - kPipeStep : kPipeStep) * 8,
-             step * 8);
+    exchange(mv + (up ? SWEEPS * 256 : 0), mv + (up ? (SWEEPS - 1) * 256 : 256), up ? -256 : 256);
     up = !up;
     __syncthreads();
     p_nr = c_nr;
@@ -471,14 +526,40 @@ __global__ void __launch_bounds__(kPipeThreads)
     bars_per_tile = n_sub;
     if (!more) break;
   }
-  const int step = up ? -kPipeStep : kPipeStep;
-  const int p_first = i0 + (up ? 0 : kPipeMaxRows - kPipeStep);
+  const int step = up ? -STEP : STEP;
+  const int p_first = i0 + (up ? 0 : R - STEP);
   tile_factor();
   store(KC(0), KC(8), p_first, -step, p_nr, p_slot, p_row0, p_b0);
   store(KC(8), KC(16), p_first, -step, p_nr, p_slot, p_row0, p_b0);
-  store(KC(16), KC(23), p_first, -step, p_nr, p_slot, p_row0, p_b0);
-  store(KC(23), KC(29), p_first, -step, p_nr, p_slot, p_row0, p_b0);
+  store(KC(16), KC(22), p_first, -step, p_nr, p_slot, p_row0, p_b0);
+  store(KC(22), KC(SWEEPS), p_first, -step, p_nr, p_slot, p_row0, p_b0);
 #undef KC
 }
+
+// Kernel of a tile geometry and variant (the launching code and the
+// instantiations of each type are compiled apart).
+enum { PIPE_PLAIN = 0, PIPE_PHASES = 1, PIPE_TRANSPOSE = 2, PIPE_TRANSPOSE_PHASES = 3, PIPE_FUSED = 4,
+       PIPE_VARIANTS = 5 };
+template <typename T, int UNITS>
+const void* pipe_kernel_units(int variant) {
+  switch (variant) {
+    case PIPE_PLAIN: return (const void*)fiber_pipe_kernel<T, UNITS, false, false, false>;
+    case PIPE_PHASES: return (const void*)fiber_pipe_kernel<T, UNITS, false, true, false>;
+    case PIPE_TRANSPOSE: return (const void*)fiber_pipe_kernel<T, UNITS, true, false, false>;
+    case PIPE_TRANSPOSE_PHASES: return (const void*)fiber_pipe_kernel<T, UNITS, true, true, false>;
+    default: return (const void*)fiber_pipe_kernel<T, UNITS, true, false, true>;
+  }
+}
+template <typename T>
+const void* pipe_kernel(int units, int variant) {
+  switch (units) {
+    case 8: return pipe_kernel_units<T, 8>(variant);
+    case 4: return pipe_kernel_units<T, 4>(variant);
+    case 2: return pipe_kernel_units<T, 2>(variant);
+    default: return pipe_kernel_units<T, 1>(variant);
+  }
+}
+const void* pipe_kernel_c128(int units, int variant);
+const void* pipe_kernel_c64(int units, int variant);
 
 }  // namespace ffsim_amd

@@ -1,0 +1,6 @@
+// Instantiations of the pipelined window passes, complex64.
+#include "fiber_pipe.hpp"
+
+namespace ffsim_amd {
+const void* pipe_kernel_c64(int units, int variant) { return pipe_kernel<float>(units, variant); }
+}  // namespace ffsim_amd

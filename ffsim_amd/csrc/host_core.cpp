@@ -353,54 +353,173 @@ GroupTables make_group_tables(int w, int w2, bool merge_complements) {
   return T;
 }
 
+namespace {
+// Cuts one (kp, lo2) set of groups (given by their classes) into chunks and
+// deals them to the waves; appends to `chunks` and writes (offset, count) per wave.
+void schedule_groups(const std::vector<int>& classes, int w2, int n_waves, int per_chunk,
+                     std::vector<uint32_t>& chunks, int32_t* index) {
+  const int nd = (int)classes.size(), n_simd = std::min(4, n_waves);
+  struct Ch {
+    int g0, ng;
+    double cost;
+  };
+  std::vector<Ch> chs;
+  for (int g = 0; g < nd;) {
+    const int k2 = classes[g];
+    int e = g;
+    while (e < nd && e - g < per_chunk && classes[e] == k2) ++e;
+    // rotation work per lane ~ pairs per pair position; plus the group's loads/stores
+    const double pairs = (double)binom(w2 - 2, k2 - 1);
+    const double size = (double)binom(w2, k2);
+    chs.push_back({g, e - g, 6.0 * pairs + size});
+    g = e;
+  }
+  std::stable_sort(chs.begin(), chs.end(),
+                   [](const Ch& a, const Ch& b) { return a.cost > b.cost; });
+  std::vector<double> simd_load(n_simd, 0.0), wave_load(n_waves, 0.0);
+  std::vector<std::vector<uint32_t>> per_wave(n_waves);
+  for (const Ch& c : chs) {
+    int s = 0;
+    for (int k = 1; k < n_simd; ++k)
+      if (simd_load[k] < simd_load[s]) s = k;
+    int wv = s;
+    for (int k = s; k < n_waves; k += n_simd)
+      if (wave_load[k] < wave_load[wv]) wv = k;
+    simd_load[s] += c.cost;
+    wave_load[wv] += c.cost;
+    per_wave[wv].push_back(((uint32_t)c.g0 << 8) | (uint32_t)c.ng);
+  }
+  for (int wv = 0; wv < n_waves; ++wv) {
+    index[2 * wv] = (int32_t)chunks.size();
+    index[2 * wv + 1] = (int32_t)per_wave[wv].size();
+    chunks.insert(chunks.end(), per_wave[wv].begin(), per_wave[wv].end());
+  }
+}
+}  // namespace
+
 WaveSchedule make_wave_schedule(const GroupTables& T, int n_waves, int per_chunk) {
   WaveSchedule ws;
   ws.n_waves = n_waves;
   ws.index.assign((size_t)(T.w + 1) * T.n_lo2 * n_waves * 2, 0);
-  const int n_simd = std::min(4, n_waves);
   for (int kp = 0; kp <= T.w; ++kp) {
     for (int lo2 = 0; lo2 < T.n_lo2; ++lo2) {
-      const int* ix = T.index.data() + ((size_t)kp * T.n_lo2 + lo2) * 4;
-      const int d0 = ix[0], nd = ix[1];
-      struct Ch {
-        int g0, ng;
-        double cost;
-      };
-      std::vector<Ch> chs;
-      for (int g = 0; g < nd;) {
-        const int k2 = T.desc[d0 + g] & 0x7f;  // group class (flag bit 7: complemented)
-        int e = g;
-        while (e < nd && e - g < per_chunk && (int)(T.desc[d0 + e] & 0x7f) == k2) ++e;
-        // rotation work per lane ~ pairs per pair position; plus the group's loads/stores
-        const double pairs = (double)binom(T.w2 - 2, k2 - 1);
-        const double size = (double)binom(T.w2, k2);
-        chs.push_back({g, e - g, 6.0 * pairs + size});
-        g = e;
-      }
-      std::stable_sort(chs.begin(), chs.end(),
-                       [](const Ch& a, const Ch& b) { return a.cost > b.cost; });
-      std::vector<double> simd_load(n_simd, 0.0), wave_load(n_waves, 0.0);
-      std::vector<std::vector<uint32_t>> per_wave(n_waves);
-      for (const Ch& c : chs) {
-        int s = 0;
-        for (int k = 1; k < n_simd; ++k)
-          if (simd_load[k] < simd_load[s]) s = k;
-        int wv = s;
-        for (int k = s; k < n_waves; k += n_simd)
-          if (wave_load[k] < wave_load[wv]) wv = k;
-        simd_load[s] += c.cost;
-        wave_load[wv] += c.cost;
-        per_wave[wv].push_back(((uint32_t)c.g0 << 8) | (uint32_t)c.ng);
-      }
-      for (int wv = 0; wv < n_waves; ++wv) {
-        int32_t* out = ws.index.data() + (((size_t)kp * T.n_lo2 + lo2) * n_waves + wv) * 2;
-        out[0] = (int32_t)ws.chunks.size();
-        out[1] = (int32_t)per_wave[wv].size();
-        ws.chunks.insert(ws.chunks.end(), per_wave[wv].begin(), per_wave[wv].end());
-      }
+      const size_t set = (size_t)kp * T.n_lo2 + lo2;
+      const int* ix = T.index.data() + set * 4;
+      std::vector<int> classes;
+      for (int g = 0; g < ix[1]; ++g) classes.push_back(T.desc[ix[0] + g] & 0x7f);
+      schedule_groups(classes, T.w2, n_waves, per_chunk, ws.chunks,
+                      ws.index.data() + set * n_waves * 2);
     }
   }
   return ws;
+}
+
+PipeGroups make_pipe_groups(int w, int kp_lo, int kp_hi, bool merge_complements, int units,
+                            int n_waves, int per_chunk) {
+  if (w < kMaxSubWindow || w > 16 || (units != 1 && units != 2 && units != 4 && units != 8))
+    throw std::invalid_argument("bad pipelined window");
+  PipeGroups T;
+  T.w = w;
+  T.w2 = kMaxSubWindow;
+  T.units = units;
+  const int w2 = T.w2;
+  T.n_lo2 = w - w2 + 1;
+  T.index.assign((size_t)(w + 1) * T.n_lo2 * 2, 0);
+  T.wave_index.assign((size_t)(w + 1) * T.n_lo2 * n_waves * 2, 0);
+  auto reversed = [&](int k2) { return merge_complements && 2 * k2 > w2; };
+  for (int lo2 = 0; lo2 < T.n_lo2; ++lo2) {
+    T.offs_index.push_back((int32_t)T.offs.size());
+    T.offs_index.push_back((lo2 + 1) * kPipeOffStride);
+    for (int kl = 0; kl <= lo2; ++kl) {
+      std::vector<uint32_t> row(kPipeOffStride, 0);
+      for (int k2 = 1; k2 < w2; ++k2) {
+        std::vector<uint64_t> subs = make_strings(w2, k2);
+        if (reversed(k2)) std::reverse(subs.begin(), subs.end());
+        for (size_t m = 0; m < subs.size(); ++m) {
+          uint64_t r = 0;
+          int t = kl;
+          for (uint64_t x = subs[m]; x; x &= x - 1) r += binom(lo2 + __builtin_ctzll(x), ++t);
+          row[kPipeOffStart[k2 - 1] + m] = (uint32_t)(r * 16 * units);
+        }
+      }
+      T.offs.insert(T.offs.end(), row.begin(), row.end());
+    }
+  }
+  const int R = 16 / units;  // strings of one LDS access: bank sets of 16 units bytes
+  for (int kp = std::max(kp_lo, 0); kp <= std::min(kp_hi, w); ++kp) {
+    for (int lo2 = 0; lo2 < T.n_lo2; ++lo2) {
+      struct G {
+        int cls, kl, k2;
+        uint32_t base;
+      };
+      std::vector<G> gs;
+      const int n_out = w - w2;
+      for (uint64_t o = 0; o < (1ull << n_out); ++o) {
+        const uint64_t low = o & ((1ull << lo2) - 1), high = (o >> lo2) << (lo2 + w2);
+        const int kl = __builtin_popcountll(low);
+        const int k2 = kp - kl - __builtin_popcountll(high);
+        if (k2 <= 0 || k2 >= w2) continue;
+        uint64_t base = string_rank(low);
+        int t = kl + k2;
+        for (uint64_t x = high; x; x &= x - 1) base += binom(__builtin_ctzll(x), ++t);
+        gs.push_back({reversed(k2) ? w2 - k2 : k2, kl, k2, (uint32_t)base});
+      }
+      std::stable_sort(gs.begin(), gs.end(), [&](const G& a, const G& b) {
+        const uint64_t sa = binom(w2, a.cls), sb = binom(w2, b.cls);
+        if (sa != sb) return sa > sb;
+        if (a.cls != b.cls) return a.cls < b.cls;
+        if (a.kl != b.kl) return a.kl < b.kl;
+        return a.k2 < b.k2;
+      });
+      // within a class, R groups at a time whose members share the fewest banks
+      std::vector<G> order;
+      const uint32_t* offs = T.offs.data() + T.offs_index[2 * lo2];
+      for (size_t i = 0; i < gs.size();) {
+        size_t j = i;
+        while (j < gs.size() && gs[j].cls == gs[i].cls) ++j;
+        const int N = (int)binom(w2, gs[i].cls);
+        std::vector<char> used(j - i, 0);
+        auto slot = [&](const G& g, int m) {
+          return (g.base + offs[g.kl * kPipeOffStride + kPipeOffStart[g.k2 - 1] + m] /
+                               (16 * units)) % R;
+        };
+        for (size_t n_used = 0; n_used < j - i;) {
+          std::vector<int> occ((size_t)N * R, 0);
+          for (int s = 0; s < R && n_used < j - i; ++s, ++n_used) {
+            size_t best = j;
+            long best_cost = -1;
+            for (size_t b = i; b < j; ++b) {
+              if (used[b - i]) continue;
+              long cost = 0;
+              for (int m = 0; m < N; ++m) cost += occ[(size_t)m * R + slot(gs[b], m)];
+              if (best_cost < 0 || cost < best_cost) {
+                best = b;
+                best_cost = cost;
+                if (cost == 0) break;
+              }
+            }
+            used[best - i] = 1;
+            order.push_back(gs[best]);
+            for (int m = 0; m < N; ++m) ++occ[(size_t)m * R + slot(gs[best], m)];
+          }
+        }
+        i = j;
+      }
+      const size_t set = (size_t)kp * T.n_lo2 + lo2;
+      T.index[2 * set] = (int32_t)T.desc.size();
+      T.index[2 * set + 1] = (int32_t)order.size();
+      std::vector<int> classes;
+      for (const G& g : order) {
+        const uint32_t toff = (uint32_t)(g.kl * kPipeOffStride + kPipeOffStart[g.k2 - 1]) / 4;
+        T.desc.push_back((g.base << 16) | (toff << 4) | (g.cls != g.k2 ? 8u : 0u) |
+                         (uint32_t)g.cls);
+        classes.push_back(g.cls);
+      }
+      schedule_groups(classes, w2, n_waves, per_chunk, T.chunks,
+                      T.wave_index.data() + set * n_waves * 2);
+    }
+  }
+  return T;
 }
 
 // Greedy sub-window schedule: at every step take the sub-window start whose

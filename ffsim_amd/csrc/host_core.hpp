@@ -129,6 +129,34 @@ struct WaveSchedule {
 };
 WaveSchedule make_wave_schedule(const GroupTables& T, int n_waves, int per_chunk);
 
+// Register groups of the pipelined passes.  The colex rank of a string splits
+// into a part fixed by its bits outside the sub-window and a part that depends
+// only on the electrons below the sub-window (kL), the class and the member:
+// so a group is one word (its base rank) and all groups of a window share one
+// small table of member offsets per (lo2, kL), whatever the window's width.
+// offs holds, per sub-window start lo2 and kL in [0, lo2], kPipeOffStride byte
+// offsets into a tile of 16 `units` bytes per string: those of k2 electrons
+// start at kPipeOffStart[k2 - 1], in ascending order of the sub-window bits
+// (descending for k2 > w2 / 2 with merged complements, the order of the
+// complemented class).  Only electron counts kp_lo..kp_hi of the window get
+// groups.  Groups that one LDS access serves together (16 / units of them) are
+// chosen so that their members lie on different banks as often as possible.
+// The wave schedule is make_wave_schedule's.
+constexpr int kPipeOffStride = 68;
+constexpr int kPipeOffStart[5] = {0, 8, 24, 44, 60};
+struct PipeGroups {
+  int w = 0, w2 = 0, n_lo2 = 0, units = 0;
+  // base rank << 16 | (offset in offs of this lo2, in units of 4) << 4 | complemented << 3 | class
+  std::vector<uint32_t> desc;
+  std::vector<int32_t> index;        // [(kp n_lo2 + lo2) 2 + {desc offset, count}]
+  std::vector<uint32_t> offs;
+  std::vector<int32_t> offs_index;   // [lo2 2 + {offset in offs, count}]
+  std::vector<uint32_t> chunks;      // first_group << 8 | n_groups
+  std::vector<int32_t> wave_index;   // [((kp n_lo2 + lo2) n_waves + wave) 2 + {offset, count}]
+};
+PipeGroups make_pipe_groups(int w, int kp_lo, int kp_hi, bool merge_complements, int units,
+                            int n_waves, int per_chunk);
+
 // ------------------------------------------------------ Givens decomposition
 // Exact Clements decomposition U = D G_L^* ... G_1^* with each G acting on
 // adjacent orbitals (i, j) as [[c, s], [-conj(s), c]] (c real), matching the

@@ -194,18 +194,9 @@ __device__ __forceinline__ void slot_apply(Cx<T>* v, const double* c, const doub
   }
 }
 
-// Applies the layer pairs of one sub-pass to one register group (one batch column).
+// Applies the layer pairs of one sub-pass to a group's members in registers.
 template <typename T, int W2, int K2>
-__device__ __forceinline__ void group_apply(Cx<T>* tile, int S, int j,
-                                            const uint16_t* __restrict__ members,
-                                            const LayerPair* lp, int n_lp, bool flip) {
-  constexpr int N = binom_const(W2, K2);
-  Cx<T> v[N];
-  int idx[N];
-#pragma unroll
-  for (int m = 0; m < N; ++m) idx[m] = (int)members[m] * S + j;
-#pragma unroll
-  for (int m = 0; m < N; ++m) v[m] = tile[idx[m]];
+__device__ __forceinline__ void apply_layers(Cx<T>* v, const LayerPair* lp, int n_lp, bool flip) {
   for (int l = 0; l < n_lp; ++l) {
     // one batch of scalar loads for the whole layer pair (uniform over the wave)
     const LayerPair& L = lp[l];
@@ -230,6 +221,21 @@ __device__ __forceinline__ void group_apply(Cx<T>* tile, int S, int j,
     slot_apply<T, W2, K2, 1>(v, c, sr, si, mask, flip);
     slot_apply<T, W2, K2, 3>(v, c, sr, si, mask, flip);
   }
+}
+
+// Applies the layer pairs of one sub-pass to one register group (one batch column).
+template <typename T, int W2, int K2>
+__device__ __forceinline__ void group_apply(Cx<T>* tile, int S, int j,
+                                            const uint16_t* __restrict__ members,
+                                            const LayerPair* lp, int n_lp, bool flip) {
+  constexpr int N = binom_const(W2, K2);
+  Cx<T> v[N];
+  int idx[N];
+#pragma unroll
+  for (int m = 0; m < N; ++m) idx[m] = (int)members[m] * S + j;
+#pragma unroll
+  for (int m = 0; m < N; ++m) v[m] = tile[idx[m]];
+  apply_layers<T, W2, K2>(v, lp, n_lp, flip);
 #pragma unroll
   for (int m = 0; m < N; ++m) tile[idx[m]] = v[m];
 }
