@@ -149,6 +149,7 @@ struct DevWindow {
   Fiber* fibers = nullptr;
   int32_t* rows = nullptr;
   int n_fibers = 0, n_active = 0, max_rows = 0, max_rows_active = 0, lo = 0, w = 0;
+  int whole_kp = 0;  // electrons of the only fiber of a window over all orbitals
   long rows_all = 0, rows_active = 0;  // strings covered by all / by the active fibers
 };
 // Pair tables of one rotation (i, j) for (norb, nocc): the strings with i
@@ -200,9 +201,12 @@ struct ProgramRing {
 // kp_lo..kp_hi electrons.
 struct DevPipe {
   PipeGroups host;
-  uint32_t *desc = nullptr, *offs = nullptr, *chunks = nullptr;
-  int32_t *index = nullptr, *offs_index = nullptr, *wave_index = nullptr;
+  int kp_lo = 0, kp_hi = 0;
+  mutable std::atomic<int> worst_dwords{0};  // image with every sub-window start
+  // staged images per list of sub-window starts (built on first use)
+  std::map<std::vector<int>, PipeTables> images;
 };
+constexpr size_t kMaxPipeImages = 64;
 
 struct Context {
   // rocBLAS handle of the batched small-state path (created on first use;
@@ -394,6 +398,7 @@ const DevWindow& dev_window(Context& ctx, int norb, int nocc, int lo, int w) {
   dw.max_rows_active = L.max_rows_active;
   dw.lo = lo;
   dw.w = w;
+  dw.whole_kp = nocc;
   for (size_t f = 0; f < L.fibers.size(); ++f) {
     dw.rows_all += L.fibers[f].n_rows;
     if ((int)f < L.n_active) dw.rows_active += L.fibers[f].n_rows;
@@ -456,8 +461,7 @@ const DevSchedule& dev_schedule(Context& ctx, const DevGroups& gr, int n_waves, 
   return g.schedules[key] = ds;
 }
 
-const DevPipe& dev_pipe(Context& ctx, int w, int kp_lo, int kp_hi, bool merge, int units,
-                        size_t elem) {
+DevPipe& dev_pipe(Context& ctx, int w, int kp_lo, int kp_hi, bool merge, int units, size_t elem) {
   std::lock_guard<std::mutex> lk(ctx.mu);
   const auto key = std::make_tuple(w, kp_lo, kp_hi, merge, units);
   auto it = ctx.pipe.find(key);
@@ -465,14 +469,62 @@ const DevPipe& dev_pipe(Context& ctx, int w, int kp_lo, int kp_hi, bool merge, i
   auto dp = std::make_unique<DevPipe>();
   dp->host = make_pipe_groups(w, kp_lo, kp_hi, merge, units, kPipeCompute,
                               64 / pipe_width(units, elem));
-  const PipeGroups& T = dp->host;
-  dp->desc = upload_table(T.desc);
-  dp->offs = upload_table(T.offs);
-  dp->chunks = upload_table(T.chunks);
-  dp->index = upload_table(T.index);
-  dp->offs_index = upload_table(T.offs_index);
-  dp->wave_index = upload_table(T.wave_index);
+  dp->kp_lo = kp_lo;
+  dp->kp_hi = kp_hi;
   return *(ctx.pipe[key] = std::move(dp));
+}
+
+// The images (see PipeTables) of a list of sub-window starts, kp_lo..kp_hi.
+std::vector<uint32_t> pipe_image(const DevPipe& dp, const std::vector<int>& lo2, PipeTables& tb) {
+  const PipeGroups& T = dp.host;
+  const int n = (int)lo2.size();
+  int groups = 0, chunks = 0, offsets = 0;
+  auto set_of = [&](int kp, int u) { return (size_t)kp * T.n_lo2 + lo2[u]; };
+  auto n_chunks = [&](size_t set) {
+    const int32_t* wi = T.wave_index.data() + set * kPipeCompute * 2;
+    return wi[2 * kPipeCompute - 2] + wi[2 * kPipeCompute - 1] - wi[0];
+  };
+  for (int kp = dp.kp_lo; kp <= dp.kp_hi; ++kp) {
+    int nd = 0, nc = 0;
+    for (int u = 0; u < n; ++u) {
+      nd += T.index[2 * set_of(kp, u) + 1];
+      nc += n_chunks(set_of(kp, u));
+    }
+    groups = std::max(groups, nd);
+    chunks = std::max(chunks, nc);
+  }
+  for (int u = 0; u < n; ++u) offsets += T.offs_index[2 * lo2[u] + 1];
+  auto up4 = [](int x) { return (x + 3) / 4 * 4; };
+  tb.kp_lo = dp.kp_lo;
+  tb.desc = kPipeImageOffs + up4(offsets);
+  tb.sched = tb.desc + up4(groups);
+  tb.chunks = tb.sched + 2 * kPipeCompute * n;
+  tb.dwords = up4(tb.chunks + chunks);
+  std::vector<uint32_t> img((size_t)tb.dwords * (dp.kp_hi - dp.kp_lo + 1), 0);
+  for (int kp = dp.kp_lo; kp <= dp.kp_hi; ++kp) {
+    uint32_t* im = img.data() + (size_t)(kp - dp.kp_lo) * tb.dwords;
+    int d = 0, o = 0, c = 0;
+    for (int u = 0; u < n; ++u) {
+      const size_t set = set_of(kp, u);
+      im[2 * u] = (uint32_t)d;
+      im[2 * u + 1] = (uint32_t)o;
+      const int o0 = T.offs_index[2 * lo2[u]], no = T.offs_index[2 * lo2[u] + 1];
+      std::copy(T.offs.begin() + o0, T.offs.begin() + o0 + no, im + kPipeImageOffs + o);
+      const int d0 = T.index[2 * set], nd = T.index[2 * set + 1];
+      std::copy(T.desc.begin() + d0, T.desc.begin() + d0 + nd, im + tb.desc + d);
+      const int32_t* wi = T.wave_index.data() + set * kPipeCompute * 2;
+      for (int wv = 0; wv < kPipeCompute; ++wv) {
+        im[tb.sched + 2 * (kPipeCompute * u + wv)] = (uint32_t)(c + wi[2 * wv] - wi[0]);
+        im[tb.sched + 2 * (kPipeCompute * u + wv) + 1] = (uint32_t)wi[2 * wv + 1];
+      }
+      const int nc = n_chunks(set);
+      std::copy(T.chunks.begin() + wi[0], T.chunks.begin() + wi[0] + nc, im + tb.chunks + c);
+      d += nd;
+      o += no;
+      c += nc;
+    }
+  }
+  return img;
 }
 
 size_t pow2_ceil(size_t x) {
@@ -698,28 +750,21 @@ size_t fiber_lds_bytes(size_t elem, int W, bool cols, int n_waves, int rows, int
          align16((size_t)gd_cap * 4) + diag_lds_bytes(diag, fuse, n_diag, rows, W, n_fac, win);
 }
 
-// mt: several states of one shape (in place: src and dst unused; no
-// transposing store, no fused diagonal), their tiles in one persistent
-// launch; null for one state.
-template <typename T, int W, int MODE, int W2, int NTHR, bool FUSE = false, bool MULTI = false>
+template <typename T, int W, int MODE, int W2, int NTHR, bool FUSE = false>
 void launch_fiber_t(const void* src, void* dst, long ld_src, long ld_dst, int n_batch, bool tstore,
                     const DevWindow& win, bool all_fibers, const DevGroups& gr, const LoSlots& los,
                     int gd_cap, int gm_cap, const SubPass* d_subs, int n_sub,
                     const LayerPair* d_layers, int n_layers, const double* d_diag,
                     const uint64_t* d_strings, int n_diag, size_t lds_max, hipStream_t stream,
-                    const DiagFuse& fz = DiagFuse{}, const MultiTiles* mt = nullptr) {
-  static_assert(!(MULTI && FUSE), "the multi-state pass has no fused diagonal");
-  require(MULTI == (mt != nullptr) && (!MULTI || !tstore), FFSIM_ERR_VALUE,
-          "fiber launch: inconsistent multi-state arguments");
-  const int n_states = MULTI ? mt->n_states : 1;
+                    const DiagFuse& fz = DiagFuse{}) {
   const int n_f = all_fibers ? win.n_fibers : win.n_active;
-  if (n_f == 0 || n_batch == 0 || n_states == 0) return;
+  if (n_f == 0 || n_batch == 0) return;
   const int rows = all_fibers ? win.max_rows : win.max_rows_active;
   const size_t lds = fiber_lds_bytes(sizeof(Cx<T>), W, MODE == MODE_COLS, NTHR / 64, rows,
                                      gd_cap, gm_cap, d_diag != nullptr, FUSE, n_diag, fz.n_fac,
                                      fz.win);
   require(lds <= lds_max, FFSIM_ERR_VALUE, "fiber tile exceeds LDS");
-  auto kern = fiber_kernel<T, W, MODE, NTHR, W2, FUSE, MULTI>;
+  auto kern = fiber_kernel<T, W, MODE, NTHR, W2, FUSE>;
   const DevSchedule& sched = dev_schedule(context(), gr, NTHR / 64, W);
   static bool attr_set = false;
   if (!attr_set) {
@@ -728,7 +773,7 @@ void launch_fiber_t(const void* src, void* dst, long ld_src, long ld_dst, int n_
     attr_set = true;
   }
   const int n_bt = (n_batch + W - 1) / W;
-  const long n_tiles = (long)n_bt * n_f * n_states;
+  const long n_tiles = (long)n_bt * n_f;
   require(n_tiles < (1l << 40), FFSIM_ERR_VALUE, "grid too large");
   // persistent grid: as many blocks as fit on the device at once
   int occ = 0;
@@ -736,55 +781,16 @@ void launch_fiber_t(const void* src, void* dst, long ld_src, long ld_dst, int n_
   const long per_cu = std::max(1, occ);
   const long grid = std::min<long>(n_tiles, per_cu * g_n_cu);
   // algorithmic bytes: every element of every launched fiber read once and written once
-  const double moved = 2.0 * (double)sizeof(Cx<T>) * (double)n_batch * (double)n_states *
+  const double moved = 2.0 * (double)sizeof(Cx<T>) * (double)n_batch *
                        (double)(all_fibers ? win.rows_all : win.rows_active);
   const long pk = prof_start(PROF_FIBER, moved, stream);
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NTHR), lds, stream,
                      reinterpret_cast<const Cx<T>*>(src), reinterpret_cast<Cx<T>*>(dst), ld_src,
                      ld_dst, n_batch, tstore ? 1 : 0, win.fibers, n_f, win.rows, gr.args(sched), los,
                      d_subs, n_sub, d_layers, n_layers, d_diag, d_strings, n_diag, rows, gd_cap,
-                     gm_cap, fz, MULTI ? *mt : MultiTiles{nullptr, 1, 0, 0});
+                     gm_cap, fz);
   HIP_CHECK(hipGetLastError());
   prof_stop(pk, stream);
-}
-
-// Entries of a pipelined pass's tables in LDS, over the window's electron
-// counts: groups, member offsets and chunks of the given sub-window starts.
-struct PipeCaps {
-  int groups = 0, offsets = 0, chunks = 0;
-};
-PipeCaps pipe_caps(const PipeGroups& T, const int* lo2, int n) {
-  PipeCaps c;
-  for (int kp = 0; kp <= T.w; ++kp) {
-    int nd = 0, nc = 0;
-    for (int u = 0; u < n; ++u) {
-      const size_t set = (size_t)kp * T.n_lo2 + lo2[u];
-      nd += T.index[2 * set + 1];
-      for (int wv = 0; wv < kPipeCompute; ++wv)
-        nc += T.wave_index[(set * kPipeCompute + wv) * 2 + 1];
-    }
-    c.groups = std::max(c.groups, nd);
-    c.chunks = std::max(c.chunks, nc);
-  }
-  for (int u = 0; u < n; ++u) c.offsets += T.offs_index[2 * lo2[u] + 1];
-  return c;
-}
-
-// LDS of a pipelined launch, following the kernel's layout.
-size_t pipe_lds_bytes(int units, size_t elem, const PipeCaps& c, bool tstore, bool diag,
-                      int n_fac, int win) {
-  const size_t R = pipe_max_rows(units), W = pipe_width(units, elem);
-  const size_t slots = units < 8 ? 1 : kPipeSlots;
-  size_t b = (size_t)(pipe_sweeps(units) + 1) * 4096 + (tstore || units < 8 ? 0 : slots * R * 4) +
-             align16(kPipeMaxLo * sizeof(PipeSlot)) + align16((size_t)c.offsets * 4) +
-             align16((size_t)c.groups * 4) + (size_t)kPipeMaxLo * kPipeCompute * 8 +
-             align16((size_t)c.chunks * 4);
-  if (diag || n_fac) b += slots * R * 2;
-  if (n_fac)
-    b += 16 + (W * n_fac + (size_t)fuse_nibble_entries(win, (int)W)) * sizeof(Cx<double>);
-  else if (diag)
-    b += 68 * sizeof(Cx<double>);
-  return b;
 }
 
 // How the passes of a sector with strings on rows run: the window width, and
@@ -799,9 +805,65 @@ size_t pipe_lds_bytes(int units, size_t elem, const PipeCaps& c, bool tstore, bo
 // 107 us, norb=14 (3432, 2 columns) 449 -> 281 us, norb=15 (6435, 1 column)
 // 1614 -> 945 us; complex64 153 -> 81, 324 -> 220 and 1080 -> 810 us.
 struct SectorGeom {
-  int w = 0, units = 0;
+  int w = 0, units = 0, sweeps = 0;
   bool whole = false;  // a tile holds every string of the sector (one pass)
+  bool small = false;  // in place, several states (norb <= 12)
 };
+
+// LDS of a pipelined launch, following the kernel's layout.
+size_t pipe_lds_bytes(const SectorGeom& g, size_t elem, int image_dwords, int variant, int n_fac,
+                      int win) {
+  const int units = g.units;
+  const bool small = variant >= PIPE_SMALL_ROWS;
+  const bool whole = small || units < 8;
+  const bool tstore = variant == PIPE_TRANSPOSE || variant == PIPE_TRANSPOSE_PHASES ||
+                      variant == PIPE_FUSED;
+  const bool dg = variant == PIPE_PHASES || variant == PIPE_TRANSPOSE_PHASES || small;
+  const size_t R = pipe_max_rows(units, g.sweeps), W = pipe_width(units, elem);
+  const size_t slots = whole ? 1 : kPipeSlots;
+  size_t b = (size_t)(g.sweeps + 1) * 4096 + (tstore || whole ? 0 : slots * R * 4) +
+             align16((size_t)image_dwords * 4);
+  if (dg || variant == PIPE_FUSED) b += slots * R * 2;
+  if (dg) b += 68 * sizeof(Cx<double>);
+  if (variant == PIPE_FUSED || small) b += 16;
+  if (variant == PIPE_FUSED)
+    b += (W * n_fac + (size_t)fuse_nibble_entries(win, (int)W)) * sizeof(Cx<double>);
+  return b;
+}
+
+// Geometry of the in-place whole-sector passes of norb 6 to 12 (units 0: none):
+// the least tile that holds the sector's strings.  A tile's time is the chain
+// of its sub-passes (one chunk each of 6-orbital groups: 25 to 40 us at norb
+// 10 to 12), not its width, so the width is chosen for the number of tiles:
+// - 64-byte rows where a sector of norb 12 alone would leave CUs without a
+//   tile (924 x 924 complex128: 231 tiles instead of 116, 50 -> 41 us);
+// - 256-byte rows for sectors of at most 464 strings once 128-byte rows would
+//   give a CU a second tile: half as many tiles, whose chunks are fuller (norb
+//   10: 3 of 5 chunks of 8 groups have no more than half their lanes).  32 states of
+//   norb 10: complex128 81 -> 51 us, complex64 48 -> 33; 8 states of norb 11:
+//   complex128 62 -> 54, complex64 54 -> 36.
+SectorGeom small_geom(int dtype, int norb, int nocc, long n_batch, int n_states) {
+  SectorGeom g;
+  g.w = norb;
+  const size_t elem = elem_bytes(dtype);
+  if (norb < kMaxSubWindow || norb > std::min(window_cap(), 12) || n_batch > (1l << 30) ||
+      tile_width(dtype) != (dtype == FFSIM_C64 ? 4 : 8) || n_batch < (long)(16 / elem))
+    return g;
+  const long rows = (long)binom(norb, nocc), W = pipe_width(8, elem);
+  if (rows == 0 || rows > pipe_max_rows(8, 29)) return g;
+  g.whole = g.small = true;
+  g.units = 8;
+  g.sweeps = rows <= pipe_max_rows(8, 8) ? 8 : rows <= pipe_max_rows(8, 15) ? 15 : 29;
+  const long tiles = (long)((n_batch + W - 1) / W) * n_states;
+  if (g.sweeps == 29 && tiles < g_n_cu) {
+    g.units = 4;
+    g.sweeps = 15;
+  } else if (rows <= pipe_max_rows(16, 29) && tiles > g_n_cu) {
+    g.units = 16;
+    g.sweeps = rows <= pipe_max_rows(16, 16) ? 16 : 29;
+  }
+  return g;
+}
 int choose_window(Context& ctx, int norb, int nocc, int dtype);
 SectorGeom sector_geom(Context& ctx, int dtype, int norb, int nocc, long n_batch) {
   SectorGeom g;
@@ -814,10 +876,14 @@ SectorGeom sector_geom(Context& ctx, int dtype, int norb, int nocc, long n_batch
           n_batch >= pipe_width(units, elem)) {
         g.w = norb;
         g.units = units;
+        g.sweeps = pipe_sweeps(units);
         g.whole = true;
         return g;
       }
-  if (g.w >= kMaxSubWindow && g.w <= 16 && n_batch >= pipe_width(8, elem)) g.units = 8;
+  if (g.w >= kMaxSubWindow && g.w <= 16 && n_batch >= pipe_width(8, elem)) {
+    g.units = 8;
+    g.sweeps = pipe_sweeps(8);
+  }
   return g;
 }
 
@@ -849,9 +915,35 @@ bool pipe_applies(Context& ctx, int dtype, const SectorGeom& g, const DevWindow&
          (c128 ? 21.0 * rounds(8, 1) : 21.5 * rounds(4, 3));
 }
 
-const DevPipe& sector_pipe(Context& ctx, int dtype, int norb, int nocc, const SectorGeom& g) {
-  return dev_pipe(ctx, g.w, std::max(1, nocc - (norb - g.w)), std::min(nocc, g.w - 1),
+DevPipe& sector_pipe(Context& ctx, int dtype, int norb, int nocc, const SectorGeom& g) {
+  return dev_pipe(ctx, g.w, std::max(0, nocc - (norb - g.w)), std::min(nocc, g.w),
                   dtype == FFSIM_C64, g.units, elem_bytes(dtype));
+}
+
+// The tables of one pass: its sub-window starts' images, kept on the device
+// (the plan of a generic rotation is the same at every call), or in the call's
+// program once kMaxPipeImages lists have been seen; then *prog_off is their
+// offset there.
+PipeTables pass_tables(Context& ctx, DevPipe& dp, const std::vector<SubPass>& subs, Program& prog,
+                       size_t* prog_off) {
+  std::vector<int> lo2;
+  for (const SubPass& sp : subs) {
+    require(sp.slot < kPipeMaxLo, FFSIM_ERR_VALUE, "too many sub-window starts");
+    if ((int)lo2.size() <= sp.slot) lo2.resize(sp.slot + 1, 0);
+    lo2[sp.slot] = sp.lo2;
+  }
+  std::lock_guard<std::mutex> lk(ctx.mu);
+  auto it = dp.images.find(lo2);
+  if (it != dp.images.end()) return it->second;
+  PipeTables tb{};
+  const std::vector<uint32_t> img = pipe_image(dp, lo2, tb);
+  if (dp.images.size() < kMaxPipeImages) {
+    tb.image = upload_table(img);
+    dp.images[lo2] = tb;
+  } else {
+    *prog_off = prog.append(img.data(), img.size() * sizeof(uint32_t));
+  }
+  return tb;
 }
 
 struct PipeLaunch {
@@ -868,73 +960,55 @@ struct PipeLaunch {
   const uint64_t* strings;
   const Cx<double>* cfac;
   PipeFuse fz;
+  bool small, cols;
+  PipeStates ms;
 };
 
-void pipe_pass(int dtype, int units, PipeLaunch L, const DevWindow& win, PipeTables tb,
-               const PipeCaps& caps, size_t lds_max, hipStream_t stream) {
+void pipe_pass(int dtype, const SectorGeom& g, PipeLaunch L, const DevWindow& win, PipeTables tb,
+               size_t lds_max, hipStream_t stream) {
   const size_t elem = elem_bytes(dtype);
-  const int W = pipe_width(units, elem);
+  const int units = g.units, W = pipe_width(units, elem);
   int n_f = L.all_fibers ? win.n_fibers : win.n_active;
-  if (n_f == 0 || L.n_batch == 0) return;
+  if (n_f == 0 || L.n_batch == 0 || L.ms.n_states == 0) return;
   const bool fuse = L.fz.bfac != nullptr;
   const bool dg = !fuse && L.diag != nullptr;
-  require(L.n_batch >= W && (L.all_fibers ? win.max_rows : win.max_rows_active) <=
-                                pipe_max_rows(units),
+  const bool whole = L.small || units < 8;
+  int rows = L.all_fibers ? win.max_rows : win.max_rows_active;
+  require(L.n_batch >= (L.small ? (int)(16 / elem) : W) && rows <= pipe_max_rows(units, g.sweeps),
           FFSIM_ERR_VALUE, "pipelined pass: shape");
-  require((!L.tstore && units == 8) || (win.lo == 0 && (units == 8 || win.n_fibers == 1)),
+  require((!L.tstore && !whole) || (win.lo == 0 && (!whole || win.n_fibers == 1)),
           FFSIM_ERR_VALUE, "pipelined pass: rows not contiguous");
   require(!fuse || L.tstore, FFSIM_ERR_VALUE, "pipelined pass: fused diagonal without transposition");
   require(!L.cfac || (L.tstore && dg), FFSIM_ERR_VALUE, "pipelined pass: column factors");
-  const size_t lds = pipe_lds_bytes(units, elem, caps, L.tstore, dg, L.fz.n_fac, win.w);
+  require(L.small || (!L.cols && L.ms.n_states == 1), FFSIM_ERR_VALUE, "pipelined pass: states");
+  const int variant = L.small ? (L.cols ? PIPE_SMALL_COLS : PIPE_SMALL_ROWS)
+                      : fuse  ? PIPE_FUSED
+                              : 2 * L.tstore + dg;
+  const size_t lds = pipe_lds_bytes(g, elem, tb.dwords, variant, L.fz.n_fac, win.w);
   require(lds <= lds_max, FFSIM_ERR_VALUE, "pipelined tile exceeds LDS");
-  const int variant = fuse ? PIPE_FUSED : 2 * L.tstore + dg;
-  const void* kern = dtype == FFSIM_C128 ? pipe_kernel_c128(units, variant)
-                                         : pipe_kernel_c64(units, variant);
-  static std::atomic<bool> attr_set[2][9][PIPE_VARIANTS] = {};
-  if (!attr_set[dtype][units][variant]) {
+  const void* kern = dtype == FFSIM_C128 ? pipe_kernel_c128(units, g.sweeps, variant)
+                                         : pipe_kernel_c64(units, g.sweeps, variant);
+  require(kern != nullptr, FFSIM_ERR_VALUE, "pipelined pass: no such tile geometry");
+  static std::atomic<bool> attr_set[2][17][32][PIPE_VARIANTS] = {};
+  std::atomic<bool>& attr = attr_set[dtype][units][g.sweeps][variant];
+  if (!attr) {
     HIP_CHECK(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max));
-    attr_set[dtype][units][variant] = true;
+    attr = true;
   }
-  const long n_tiles = (long)((L.n_batch + W - 1) / W) * n_f;
+  const long n_tiles = (long)((L.n_batch + W - 1) / W) * (whole ? L.ms.n_states : n_f);
+  require(n_tiles < (1l << 40), FFSIM_ERR_VALUE, "grid too large");
   const long grid = std::min<long>(n_tiles, g_n_cu);
-  const double moved = 2.0 * (double)elem * (double)L.n_batch *
+  const double moved = 2.0 * (double)elem * (double)L.n_batch * (double)L.ms.n_states *
                        (double)(L.all_fibers ? win.rows_all : win.rows_active);
   const long pk = prof_start(PROF_FIBER, moved, stream);
-  int lo = win.lo, w = win.w, gd = caps.groups, go = caps.offsets, gc = caps.chunks;
+  int lo = win.lo, w = win.w, kp = win.whole_kp;
   const Fiber* fibers = win.fibers;
-  const int32_t* rows = win.rows;
-  void* args[] = {&L.src,   &L.dst,      &L.ld_src, &L.ld_dst,  &L.n_batch, &fibers, &n_f, &rows,
-                  &tb,      &L.subs,     &L.n_sub,  &L.layers,  &L.n_layers, &L.diag, &L.strings,
-                  &lo,      &w,          &gd,       &go,        &gc,        &L.cfac, &L.fz};
+  const int32_t* row_table = win.rows;
+  void* args[] = {&L.src, &L.dst,  &L.ld_src, &L.ld_dst, &L.n_batch,  &fibers, &n_f,
+                  &row_table, &tb, &L.subs,   &L.n_sub,  &L.layers,   &L.n_layers, &L.diag,
+                  &L.strings, &lo, &w,        &rows,     &kp,         &L.cfac, &L.fz, &L.ms};
   HIP_CHECK(hipLaunchKernel(kern, dim3((unsigned)grid), dim3(kPipeThreads), args, lds, stream));
   prof_stop(pk, stream);
-}
-
-template <typename T>
-void launch_fiber_multi(int mode, const MultiTiles& mt, long ld, int n_batch,
-                        const DevWindow& win, bool all_fibers, const DevGroups& gr,
-                        const LoSlots& los, int gd_cap, int gm_cap, const SubPass* d_subs,
-                        int n_sub, const LayerPair* d_layers, int n_layers, const double* d_diag,
-                        const uint64_t* d_strings, int n_diag, size_t lds_max, int W,
-                        hipStream_t stream) {
-  require(gr.w2 == kMaxSubWindow && W == (std::is_same<T, double>::value ? 8 : 4),
-          FFSIM_ERR_VALUE, "multi-state pass: unsupported shape");
-  constexpr int WW = std::is_same<T, double>::value ? 8 : 4;
-  const int rows_l = all_fibers ? win.max_rows : win.max_rows_active;
-  const size_t lds_l = fiber_lds_bytes(sizeof(Cx<T>), WW, mode == MODE_COLS, 16, rows_l, gd_cap,
-                                       gm_cap, d_diag != nullptr, false, n_diag, 0, 0);
-  const bool wide = 2 * lds_l > lds_max;
-#define FFSIM_MULTI_LAUNCH(MM, NT)                                                           \
-  launch_fiber_t<T, WW, MM, kMaxSubWindow, NT, false, true>(                                 \
-      nullptr, nullptr, ld, ld, n_batch, false, win, all_fibers, gr, los, gd_cap, gm_cap,      \
-      d_subs, n_sub, d_layers, n_layers, d_diag, d_strings, n_diag, lds_max, stream,           \
-      DiagFuse{}, &mt)
-  if (mode == MODE_ROWS) {
-    if (wide) FFSIM_MULTI_LAUNCH(MODE_ROWS, 512); else FFSIM_MULTI_LAUNCH(MODE_ROWS, 256);
-  } else {
-    if (wide) FFSIM_MULTI_LAUNCH(MODE_COLS, 512); else FFSIM_MULTI_LAUNCH(MODE_COLS, 256);
-  }
-#undef FFSIM_MULTI_LAUNCH
 }
 
 template <typename T>
@@ -1184,10 +1258,11 @@ void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, l
                 const FuseTables* fuse = nullptr, bool* fused = nullptr,
                 const size_t* cfac_off = nullptr) {
   if (fused) *fused = false;
-  SectorGeom geom;
-  if (mode == MODE_ROWS) geom = sector_geom(ctx, dtype, norb, nocc, n_batch);
-  const int w = std::max(1, mode == MODE_COLS ? norb : geom.w);
   const bool tstore = tstore_dst != nullptr;
+  SectorGeom geom;
+  if (!tstore) geom = small_geom(dtype, norb, nocc, n_batch, 1);
+  if (!geom.small && mode == MODE_ROWS) geom = sector_geom(ctx, dtype, norb, nocc, n_batch);
+  const int w = std::max(1, mode == MODE_COLS ? norb : geom.w);
   std::vector<PlannedPass> passes = plan_passes(rot.steps, norb, w, tstore, -1);
   const DevStrings& ds = dev_strings(ctx, norb, nocc);
   const bool need_diag = !rot.trivial_diag;
@@ -1217,16 +1292,10 @@ void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, l
     void* dst = ts ? tstore_dst : state;
     const long ld_dst = ts ? ld_t : ld;
     const bool all = ts || dg;
-    if (mode == MODE_ROWS && pipe_applies(ctx, dtype, geom, win, all, n_batch)) {
-      const DevPipe& dp = sector_pipe(ctx, dtype, norb, nocc, geom);
-      PipeTables tb{dp.desc,   dp.index,      dp.offs,       dp.offs_index,
-                    dp.chunks, dp.wave_index, dp.host.n_lo2, 0, {}};
-      for (const SubPass& sp : subs) {
-        require(sp.slot < kPipeMaxLo, FFSIM_ERR_VALUE, "too many sub-window starts");
-        tb.lo2[sp.slot] = sp.lo2;
-        tb.n_slots = std::max(tb.n_slots, sp.slot + 1);
-      }
-      const PipeCaps caps = pipe_caps(dp.host, tb.lo2, tb.n_slots);
+    if (geom.small || (mode == MODE_ROWS && pipe_applies(ctx, dtype, geom, win, all, n_batch))) {
+      size_t img_off = 0;
+      const PipeTables tb0 =
+          pass_tables(ctx, sector_pipe(ctx, dtype, norb, nocc, geom), subs, prog, &img_off);
       const bool fz_pipe = ts && fuse && fuse->columns_later;
       if (fz_pipe && fused) *fused = true;
       const FuseTables fp = fz_pipe ? *fuse : FuseTables{};
@@ -1239,9 +1308,12 @@ void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, l
       launches.push_back([=, &ctx, &prog, &win, &ds]() {
         PipeLaunch L{state, dst, ld, ld_dst, n_batch, ts, all, prog.dev<SubPass>(poff), n_sub,
                      prog.dev<LayerPair>(soff), n_layers, ph ? prog.dev<double>(doff) : nullptr,
-                     ds.d, cf ? prog.scratch<Cx<double>>(coff) : nullptr, PipeFuse{nullptr, 0}};
+                     ds.d, cf ? prog.scratch<Cx<double>>(coff) : nullptr, PipeFuse{nullptr, 0},
+                     geom.small, mode == MODE_COLS, PipeStates{nullptr, 1, 0, 0}};
         if (fz_pipe) L.fz = PipeFuse{prog.scratch<Cx<double>>(fp.bfac_off), fp.n_fac};
-        pipe_pass(dtype, geom.units, L, win, tb, caps, ctx.lds_max, stream);
+        PipeTables tb = tb0;
+        if (!tb.image) tb.image = prog.dev<uint32_t>(img_off);
+        pipe_pass(dtype, geom, L, win, tb, ctx.lds_max, stream);
       });
       continue;
     }
@@ -1302,15 +1374,20 @@ bool pipe_fuse_applies(Context& ctx, int dtype, int norb, int na, int nb, int n_
       !pipe_applies(ctx, dtype, gb, dev_window(ctx, norb, nb, 0, gb.w), true, da))
     return false;
   const size_t elem = elem_bytes(dtype);
-  int lo2[kPipeMaxLo];
-  for (int k = 0; k < kPipeMaxLo; ++k) lo2[k] = k;
-  auto caps = [&](int nocc, const SectorGeom& g) {
-    const PipeGroups& T = sector_pipe(ctx, dtype, norb, nocc, g).host;
-    return pipe_caps(T, lo2, T.n_lo2);
+  auto fits = [&](int nocc, const SectorGeom& g, int variant, int fac) {
+    const DevPipe& dp = sector_pipe(ctx, dtype, norb, nocc, g);
+    std::vector<int> lo2;
+    for (int k = 0; k < dp.host.n_lo2; ++k) lo2.push_back(k);
+    PipeTables tb{};
+    if (dp.worst_dwords == 0) {
+      pipe_image(dp, lo2, tb);
+      dp.worst_dwords = tb.dwords;
+    }
+    return pipe_lds_bytes(g, elem, dp.worst_dwords, variant, fac, g.w) <=
+           ctx.lds_max;
   };
-  return pipe_width(gb.units, elem) * n_fac <= 512 &&
-         pipe_lds_bytes(ga.units, elem, caps(na, ga), true, true, 0, ga.w) <= ctx.lds_max &&
-         pipe_lds_bytes(gb.units, elem, caps(nb, gb), true, true, n_fac, gb.w) <= ctx.lds_max;
+  return pipe_width(gb.units, elem) * n_fac <= 512 && fits(na, ga, PIPE_TRANSPOSE_PHASES, 0) &&
+         fits(nb, gb, PIPE_FUSED, n_fac);
 }
 
 // Full spinful orbital rotation (both sectors) on a dim_a x dim_b state.
@@ -1916,38 +1993,34 @@ bool plan_multi_sector(const std::vector<const SectorRotation*>& rots, int norb,
   return true;
 }
 
-// Queues the passes of a planned multi-state sector rotation: one fiber
-// launch per window pass over the tiles of every state (`states`, a device
-// array of the m state addresses in the call's program).
+// Queues the passes of a planned multi-state sector rotation: one launch per
+// pass over the tiles of every state (`states`, a device array of the m state
+// addresses in the call's program).
 void queue_multi_sector(Context& ctx, Program& prog, const MultiSector& ms, int dtype, int mode,
-                        size_t states_off, int m, long ld, int n_batch, int norb, int nocc, int w,
+                        size_t states_off, int m, long ld, int n_batch, int norb, int nocc,
                         hipStream_t stream, std::vector<std::function<void()>>& launches) {
   const DevStrings& ds = dev_strings(ctx, norb, nocc);
-  const DevGroups& gr = dev_groups(ctx, w, dtype == FFSIM_C64);
+  const SectorGeom geom = small_geom(dtype, norb, nocc, n_batch, m);
+  require(geom.small, FFSIM_ERR_VALUE, "multi-state pass: unsupported shape");
   size_t diag_off = 0;
   if (ms.need_diag) diag_off = prog.append(ms.diag.data(), ms.diag.size() * sizeof(double));
   for (const MultiSector::Pass& P : ms.passes) {
     const size_t soff = prog.append(P.layers.data(), P.layers.size() * sizeof(LayerPair));
     const size_t poff = prog.append(P.subs.data(), P.subs.size() * sizeof(SubPass));
-    LoSlots los{};
-    int gd_cap = 0, gm_cap = 0;
-    pass_slots(gr, P.subs, los, gd_cap, gm_cap);
-    const DevWindow& win = dev_window(ctx, norb, nocc, P.lo, w);
+    size_t img_off = 0;
+    const PipeTables tb0 =
+        pass_tables(ctx, sector_pipe(ctx, dtype, norb, nocc, geom), P.subs, prog, &img_off);
+    const DevWindow& win = dev_window(ctx, norb, nocc, P.lo, norb);
     const int n_sub = (int)P.subs.size(), n_layers = P.n_layers;
     const bool dg = P.dg;
-    launches.push_back([=, &ctx, &prog, &win, &gr, &ds]() {
-      const MultiTiles mt{prog.dev<void*>(states_off), m, (long)n_layers, 2l * norb};
-      const double* d_diag = dg ? prog.dev<double>(diag_off) : nullptr;
-      if (dtype == FFSIM_C128)
-        launch_fiber_multi<double>(mode, mt, ld, n_batch, win, dg, gr, los, gd_cap, gm_cap,
-                                   prog.dev<SubPass>(poff), n_sub, prog.dev<LayerPair>(soff),
-                                   n_layers, d_diag, ds.d, norb, ctx.lds_max, tile_width(dtype),
-                                   stream);
-      else
-        launch_fiber_multi<float>(mode, mt, ld, n_batch, win, dg, gr, los, gd_cap, gm_cap,
-                                  prog.dev<SubPass>(poff), n_sub, prog.dev<LayerPair>(soff),
-                                  n_layers, d_diag, ds.d, norb, ctx.lds_max, tile_width(dtype),
-                                  stream);
+    launches.push_back([=, &ctx, &prog, &win, &ds]() {
+      PipeLaunch L{nullptr, nullptr, ld, ld, n_batch, false, dg, prog.dev<SubPass>(poff), n_sub,
+                   prog.dev<LayerPair>(soff), n_layers, dg ? prog.dev<double>(diag_off) : nullptr,
+                   ds.d, nullptr, PipeFuse{nullptr, 0}, true, mode == MODE_COLS,
+                   PipeStates{prog.dev<void*>(states_off), m, (long)n_layers, 2l * norb}};
+      PipeTables tb = tb0;
+      if (!tb.image) tb.image = prog.dev<uint32_t>(img_off);
+      pipe_pass(dtype, geom, L, win, tb, ctx.lds_max, stream);
     });
   }
 }
@@ -1955,22 +2028,12 @@ void queue_multi_sector(Context& ctx, Program& prog, const MultiSector& ms, int 
 // States per program of the multi-state path.
 constexpr int kMultiChunk = 256;
 
-// The window widths of the multi-state path for this shape; false where it
-// does not apply: a beta vector must fit one tile (the beta sector runs in
-// place with strings on columns, its window all norb orbitals), both windows
-// must hold a full register sub-window, and the tiles must have the
-// production width.
-bool multi_windows(Context& ctx, int dtype, int n, int na, int nb, int& w_a, int& w_b) {
-  const int ww = dtype == FFSIM_C128 ? 8 : 4;
-  const long db = (long)binom(n, nb);
-  if (n < kMaxSubWindow || n > kMaxDiagOrbitals || tile_width(dtype) != ww ||
-      !beta_in_columns(n, db, dtype, ctx))
-    return false;
-  w_a = choose_window(ctx, n, na, dtype);
-  w_b = n;
-  if (w_a < kMaxSubWindow) return false;
-  return dev_groups(ctx, w_a, dtype == FFSIM_C64).w2 == kMaxSubWindow &&
-         dev_groups(ctx, w_b, dtype == FFSIM_C64).w2 == kMaxSubWindow;
+// Whether the multi-state path applies to this shape: both sectors in place on
+// whole-sector tiles (norb 6 to 12).
+bool multi_applies(Context& ctx, int dtype, int n, int na, int nb) {
+  const long da = (long)binom(n, na), db = (long)binom(n, nb);
+  return beta_in_columns(n, db, dtype, ctx) && small_geom(dtype, n, na, db, 1).small &&
+         small_geom(dtype, n, nb, da, 1).small;
 }
 
 // One orbital rotation per state, planned for multi-state passes.
@@ -1983,41 +2046,38 @@ struct MultiRotation {
 // is not rotated (then every entry is null).  The beta sector reuses the
 // alpha decomposition where ffsim_apply_orbital_rotation does.  False when
 // the states' pass structures differ.
-bool plan_multi_rotation(int n, int w_a, int w_b, const std::vector<const cdouble*>& mats_a,
+bool plan_multi_rotation(int n, const std::vector<const cdouble*>& mats_a,
                          const std::vector<const cdouble*>& mats_b, MultiRotation& mr) {
   const size_t m = mats_a.size();
   mr.has_a = mats_a[0] != nullptr;
   mr.has_b = mats_b[0] != nullptr;
-  const bool same_order = triangle_order(n, w_a) == triangle_order(n, w_b);
   std::vector<SectorRotation> ra(m), rb(m);
   std::vector<const SectorRotation*> pa(m), pb(m);
   for (size_t i = 0; i < m; ++i) {
-    if (mr.has_a) ra[i] = prepare_rotation(mats_a[i], n, w_a);
+    if (mr.has_a) ra[i] = prepare_rotation(mats_a[i], n, n);
     if (mr.has_b) {
-      if (mr.has_a && same_order &&
-          std::memcmp(mats_a[i], mats_b[i], sizeof(cdouble) * n * n) == 0)
+      if (mr.has_a && std::memcmp(mats_a[i], mats_b[i], sizeof(cdouble) * n * n) == 0)
         rb[i] = ra[i];
       else
-        rb[i] = prepare_rotation(mats_b[i], n, w_b);
+        rb[i] = prepare_rotation(mats_b[i], n, n);
     }
     pa[i] = &ra[i];
     pb[i] = &rb[i];
   }
-  return (!mr.has_a || plan_multi_sector(pa, n, w_a, mr.a)) &&
-         (!mr.has_b || plan_multi_sector(pb, n, w_b, mr.b));
+  return (!mr.has_a || plan_multi_sector(pa, n, n, mr.a)) &&
+         (!mr.has_b || plan_multi_sector(pb, n, n, mr.b));
 }
 
 // Queues a planned multi-state rotation: the alpha sector's passes (strings on
 // rows), then the beta sector's (strings on columns), in place.
 void queue_multi_rotation(Context& ctx, Program& prog, const MultiRotation& mr, int dtype,
-                          size_t states_off, int m, int n, int na, int nb, int w_a, int w_b,
-                          hipStream_t stream, std::vector<std::function<void()>>& launches) {
+                          size_t states_off, int m, int n, int na, int nb, hipStream_t stream, std::vector<std::function<void()>>& launches) {
   const long da = (long)binom(n, na), db = (long)binom(n, nb);
   if (mr.has_a)
-    queue_multi_sector(ctx, prog, mr.a, dtype, MODE_ROWS, states_off, m, db, (int)db, n, na, w_a,
+    queue_multi_sector(ctx, prog, mr.a, dtype, MODE_ROWS, states_off, m, db, (int)db, n, na,
                        stream, launches);
   if (mr.has_b)
-    queue_multi_sector(ctx, prog, mr.b, dtype, MODE_COLS, states_off, m, db, (int)da, n, nb, w_b,
+    queue_multi_sector(ctx, prog, mr.b, dtype, MODE_COLS, states_off, m, db, (int)da, n, nb,
                        stream, launches);
 }
 
@@ -2037,8 +2097,7 @@ bool ucj_batched_multi(Context& ctx, int n_states, void* const* vecs, int dtype,
                        const double* orbital_rotations, const double* final_rots,
                        hipStream_t stream) {
   const long da = (long)binom(n, na), db = (long)binom(n, nb);
-  int w_a = 0, w_b = 0;
-  if (!multi_windows(ctx, dtype, n, na, nb, w_a, w_b)) return false;
+  if (!multi_applies(ctx, dtype, n, na, nb)) return false;
   require(diag_grid(da, db).y <= 65535, FFSIM_ERR_VALUE, "too many columns");
   const size_t nn = (size_t)n * n;
   const int n_steps = n_reps + 1;
@@ -2057,7 +2116,7 @@ bool ucj_batched_multi(Context& ctx, int n_states, void* const* vecs, int dtype,
     for (int r = 0; r < n_steps; ++r) {
       std::vector<const cdouble*> pm(m);
       for (int i = 0; i < m; ++i) pm[i] = V[i][r].data();
-      if (!plan_multi_rotation(n, w_a, w_b, pm, pm, mr[r])) {
+      if (!plan_multi_rotation(n, pm, pm, mr[r])) {
         if (i0 == 0) return false;
         // earlier chunks are queued: the rest state by state (the beta sector
         // runs in place, no work buffer)
@@ -2098,8 +2157,7 @@ bool ucj_batched_multi(Context& ctx, int n_states, void* const* vecs, int dtype,
             FFSIM_ERR_VALUE, "batched UCJ: column factors exceed the program scratch");
     std::vector<std::function<void()>> launches;
     for (int r = 0; r < n_steps; ++r) {
-      queue_multi_rotation(ctx, prog, mr[r], dtype, states_off, m, n, na, nb, w_a, w_b, stream,
-                           launches);
+      queue_multi_rotation(ctx, prog, mr[r], dtype, states_off, m, n, na, nb, stream, launches);
       if (r == n_reps) break;
       const size_t hoff = hoffs[r], coff = coffs[r];
       launches.push_back([=, &prog, &sa, &sb]() {
@@ -2136,8 +2194,7 @@ void orbital_rotation_batched_impl(Context& ctx, int n_states, void* const* vecs
   const long da = (long)binom(n, na), db = (long)binom(n, nb);
   if (da == 0 || db == 0 || n == 0 || (!mats_a && !mats_b)) return;
   const size_t nn = (size_t)n * n;
-  int w_a = 0, w_b = 0;
-  const bool multi = n_states >= 2 && multi_windows(ctx, dtype, n, na, nb, w_a, w_b);
+  const bool multi = n_states >= 2 && multi_applies(ctx, dtype, n, na, nb);
   for (int i0 = 0; i0 < n_states; i0 += kMultiChunk) {
     const int m = std::min(kMultiChunk, n_states - i0);
     std::vector<const cdouble*> pa(m), pb(m);
@@ -2146,13 +2203,12 @@ void orbital_rotation_batched_impl(Context& ctx, int n_states, void* const* vecs
       pb[i] = mats_b ? mats_b + (size_t)(i0 + i) * nn : nullptr;
     }
     MultiRotation mr;
-    if (multi && m >= 2 && plan_multi_rotation(n, w_a, w_b, pa, pb, mr)) {
+    if (multi && m >= 2 && plan_multi_rotation(n, pa, pb, mr)) {
       Program prog(ctx, stream);
       std::vector<const void*> ptrs(vecs + i0, vecs + i0 + m);
       const size_t states_off = prog.append(ptrs.data(), m * sizeof(void*));
       std::vector<std::function<void()>> launches;
-      queue_multi_rotation(ctx, prog, mr, dtype, states_off, m, n, na, nb, w_a, w_b, stream,
-                           launches);
+      queue_multi_rotation(ctx, prog, mr, dtype, states_off, m, n, na, nb, stream, launches);
       prog.commit();
       for (auto& f : launches) f();
       prog.finish();

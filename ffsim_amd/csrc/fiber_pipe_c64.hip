@@ -2,5 +2,7 @@
 #include "fiber_pipe.hpp"
 
 namespace ffsim_amd {
-const void* pipe_kernel_c64(int units, int variant) { return pipe_kernel<float>(units, variant); }
+const void* pipe_kernel_c64(int units, int sweeps, int variant) {
+  return pipe_kernel<float>(units, sweeps, variant);
+}
 }  // namespace ffsim_amd

@@ -416,7 +416,8 @@ WaveSchedule make_wave_schedule(const GroupTables& T, int n_waves, int per_chunk
 
 PipeGroups make_pipe_groups(int w, int kp_lo, int kp_hi, bool merge_complements, int units,
                             int n_waves, int per_chunk) {
-  if (w < kMaxSubWindow || w > 16 || (units != 1 && units != 2 && units != 4 && units != 8))
+  if (w < kMaxSubWindow || w > 16 || (units != 1 && units != 2 && units != 4 && units != 8 &&
+                                 units != 16))
     throw std::invalid_argument("bad pipelined window");
   PipeGroups T;
   T.w = w;

@@ -311,18 +311,6 @@ __host__ __device__ constexpr int fuse_nibble_entries(int win, int W) {
   return (((win + 3) >> 2) * 16 + 1) * W;
 }
 
-// Several states of one shape in one launch (the batched Givens path): tile t
-// covers fiber t / (n_states n_bt) of state (t / n_bt) % n_states, so the
-// tiles of one fiber stay together across states and share the staged
-// tables.  Each state is rotated in place at its own address, with its own
-// layer-pair coefficients and orbital phases at the given strides.
-struct MultiTiles {
-  void* const* states;  // device array of the states' addresses
-  int n_states;
-  long layer_stride;  // LayerPairs between consecutive states' coefficients
-  long diag_stride;   // doubles between consecutive states' phases
-};
-
 // Element (string i, batch j) of a fiber tile lives at
 //   MODE_ROWS: state[row_table[i] * ld + b0 + j]   (strings index rows)
 //   MODE_COLS: state[(b0 + j) * ld + row_table[i]] (strings index columns)
@@ -335,7 +323,7 @@ struct MultiTiles {
 // LDS, the next tile's loads are already in flight into registers.
 //
 // LDS: tile[max_rows * S] | rows[max_rows] | slots | desc | members | wave schedule
-template <typename T, int W, int MODE, int NTHR, int W2, bool FUSE = false, bool MULTI = false>
+template <typename T, int W, int MODE, int NTHR, int W2, bool FUSE = false>
 __global__ void __launch_bounds__(NTHR)
     fiber_kernel(const Cx<T>* src, Cx<T>* dst, long ld_src, long ld_dst, int n_batch, int tstore,
                  const Fiber* __restrict__ fibers, int n_fibers,
@@ -343,7 +331,7 @@ __global__ void __launch_bounds__(NTHR)
                  const SubPass* __restrict__ subs_g, int n_sub,
                  const LayerPair* __restrict__ layers_g, int n_layers,
                  const double* __restrict__ diag, const uint64_t* __restrict__ strings,
-                 int n_diag, int max_rows, int gd_cap, int gm_cap, DiagFuse fz, MultiTiles mt) {
+                 int n_diag, int max_rows, int gd_cap, int gm_cap, DiagFuse fz) {
   static_assert(!FUSE || MODE == MODE_ROWS, "the fused diagonal store is a row-mode store");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   // LDS stride of one string's batch.  Row mode: unpadded (the register
@@ -388,20 +376,7 @@ __global__ void __launch_bounds__(NTHR)
 
   const int tid = threadIdx.x;
   const int n_bt = (n_batch + W - 1) / W;
-  const int NS = MULTI ? mt.n_states : 1;
-  const long per_f = (long)n_bt * NS;  // tiles of one fiber (over all states)
-  const long n_tiles = per_f * n_fibers;
-  // the state of tile t and its address (one state: the src / dst arguments)
-  auto state_of = [&](long tt) -> int { return MULTI ? (int)((tt / n_bt) % NS) : 0; };
-  auto src_of = [&](int st) -> const Cx<T>* {
-    if constexpr (MULTI) return reinterpret_cast<const Cx<T>*>(mt.states[st]);
-    else return src;
-  };
-  auto dst_of = [&](int st) -> Cx<T>* {
-    if constexpr (MULTI) return reinterpret_cast<Cx<T>*>(mt.states[st]);
-    else return dst;
-  };
-
+  const long n_tiles = (long)n_bt * n_fibers;
 
   // stage the row addresses and group tables of fiber f
   // The group tables and wave schedule depend only on the fiber's electron count
@@ -468,7 +443,7 @@ __global__ void __launch_bounds__(NTHR)
   // and waiting for those (vmcnt) would also drain the stores in flight.
   // All row addresses are read first and the element loads issued after them, so
   // the global-table case waits once for its addresses instead of once per row.
-  auto load_regs = [&](Cx<T>* buf, int nr, int b0, int nb, const int32_t* rt, const Cx<T>* sp) {
+  auto load_regs = [&](Cx<T>* buf, int nr, int b0, int nb, const int32_t* rt) {
     int ra[CH];
     if (MODE == MODE_ROWS) {
       const int j = tid % W, i0 = tid / W;
@@ -480,7 +455,7 @@ __global__ void __launch_bounds__(NTHR)
 #pragma unroll
       for (int k = 0; k < CH; ++k) {
         buf[k] = Cx<T>{T(0), T(0)};
-        if (ra[k] >= 0) buf[k] = sp[(long)ra[k] * ld_src + b0 + j];
+        if (ra[k] >= 0) buf[k] = src[(long)ra[k] * ld_src + b0 + j];
       }
     } else {
 #pragma unroll
@@ -492,7 +467,7 @@ __global__ void __launch_bounds__(NTHR)
       for (int k = 0; k < CH; ++k) {
         const int j = k % W;
         buf[k] = Cx<T>{T(0), T(0)};
-        if (ra[k] >= 0) buf[k] = sp[(long)(b0 + j) * ld_src + ra[k]];
+        if (ra[k] >= 0) buf[k] = src[(long)(b0 + j) * ld_src + ra[k]];
       }
     }
   };
@@ -514,17 +489,17 @@ __global__ void __launch_bounds__(NTHR)
   };
   // rows [first, nr) straight from global memory into LDS
   constexpr int kCovered = (MODE == MODE_ROWS) ? CH * RSTEP : (CH / W) * NTHR;
-  auto load_rows = [&](int first, int nr, int b0, int nb, const Cx<T>* sp) {
+  auto load_rows = [&](int first, int nr, int b0, int nb) {
     if (nr <= first) return;
     if (MODE == MODE_ROWS) {
       const int j = tid % W, i0 = tid / W;
 #pragma unroll 4
       for (int i = first + i0; i < nr; i += RSTEP)
-        tile[i * S + j] = (j < nb) ? sp[(long)rows[i] * ld_src + b0 + j] : Cx<T>{T(0), T(0)};
+        tile[i * S + j] = (j < nb) ? src[(long)rows[i] * ld_src + b0 + j] : Cx<T>{T(0), T(0)};
     } else {
       for (int i = first + tid; i < nr; i += NTHR)
         for (int j = 0; j < W; ++j)
-          tile[i * S + j] = (j < nb) ? sp[(long)(b0 + j) * ld_src + rows[i]] : Cx<T>{T(0), T(0)};
+          tile[i * S + j] = (j < nb) ? src[(long)(b0 + j) * ld_src + rows[i]] : Cx<T>{T(0), T(0)};
     }
   };
   auto row_phase = [&](int i, T& pr, T& pim) {
@@ -541,7 +516,7 @@ __global__ void __launch_bounds__(NTHR)
     pr = (T)re;
     pim = (T)im;
   };
-  auto store_tile = [&](int nr, int b0, int nb, Cx<T>* dp) {
+  auto store_tile = [&](int nr, int b0, int nb) {
     if (MODE == MODE_ROWS && !tstore) {
       const int j = tid % W, i0 = tid / W;
       if (j < nb) {
@@ -555,7 +530,7 @@ __global__ void __launch_bounds__(NTHR)
             v.im = v.re * pim + v.im * pr;
             v.re = t;
           }
-          dp[(long)rows[i] * ld_dst + b0 + j] = v;
+          dst[(long)rows[i] * ld_dst + b0 + j] = v;
         }
       }
     } else if (FUSE) {
@@ -611,7 +586,7 @@ __global__ void __launch_bounds__(NTHR)
             const T t = v.re * (T)P[j].re - v.im * (T)P[j].im;
             v.im = v.re * (T)P[j].im + v.im * (T)P[j].re;
             v.re = t;
-            dp[(long)(b0 + j) * ld_dst + r] = v;
+            dst[(long)(b0 + j) * ld_dst + r] = v;
           }
         }
       }
@@ -629,7 +604,7 @@ __global__ void __launch_bounds__(NTHR)
               v.im = v.re * pim + v.im * pr;
               v.re = t;
             }
-            dp[(long)(b0 + j) * ld_dst + r] = v;
+            dst[(long)(b0 + j) * ld_dst + r] = v;
           }
         }
       }
@@ -667,8 +642,8 @@ __global__ void __launch_bounds__(NTHR)
   if (t >= n_tiles) return;
   if (diag)
     for (int k = tid; k < 2 * n_diag; k += NTHR)
-      dph[k] = diag[(MULTI ? (long)state_of(t) * mt.diag_stride : 0) + k];
-  int f = (int)(t / per_f);
+      dph[k] = diag[k];
+  int f = (int)(t / n_bt);
   Fiber fd = fibers[f];
   stage_fiber(fd, true);
   __syncthreads();
@@ -677,7 +652,7 @@ __global__ void __launch_bounds__(NTHR)
   {
     const int b0 = (int)(t % n_bt) * W;
     const int nb = min(W, n_batch - b0);
-    load_rows(0, fd.n_rows, b0, nb, src_of(state_of(t)));
+    load_rows(0, fd.n_rows, b0, nb);
     if (FUSE) bfac_to_lds(load_bfac(b0), b0);
   }
   while (true) {
@@ -685,9 +660,7 @@ __global__ void __launch_bounds__(NTHR)
     const int b0 = (int)(t % n_bt) * W;
     const int nb = min(W, n_batch - b0);
     const long tn = t + gridDim.x;
-    const int fn = tn < n_tiles ? (int)(tn / per_f) : -1;
-    const int st = state_of(t);
-    const int stn = tn < n_tiles ? state_of(tn) : st;
+    const int fn = tn < n_tiles ? (int)(tn / n_bt) : -1;
     const bool same_fiber = (fn == f);
     // the next tile is prefetched also when it starts a new fiber: its rows then
     // come from the global row table (one more dependent load, hidden by the
@@ -701,9 +674,9 @@ __global__ void __launch_bounds__(NTHR)
     // around the loop: a loop-carried buf makes the compiler copy it at the back
     // edge behind a vmcnt(0) that would also drain this tile's stores
     if (same_fiber)
-      load_regs(buf, nrn, b0n, nbn, rows, src_of(stn));
+      load_regs(buf, nrn, b0n, nbn, rows);
     else
-      load_regs(buf, nrn, b0n, nbn, row_table + fdn.row_off, src_of(stn));
+      load_regs(buf, nrn, b0n, nbn, row_table + fdn.row_off);
     if (FUSE) bfn = load_bfac(b0n);
 
     // ---- register sub-passes on the current tile
@@ -714,7 +687,7 @@ __global__ void __launch_bounds__(NTHR)
       // the pass program is uniform: scalar loads straight from device memory
       const SubPass P = subs_g[sp];
       const GroupSlot gs = gslot[P.slot];
-      const LayerPair* lp = layers_g + (MULTI ? (long)st * mt.layer_stride : 0) + P.lp0;
+      const LayerPair* lp = layers_g + P.lp0;
       const int c0 = wsched[(P.slot * NW + wave) * 2];
       const int nc = wsched[(P.slot * NW + wave) * 2 + 1];
       for (int c = 0; c < nc; ++c) {
@@ -736,13 +709,9 @@ __global__ void __launch_bounds__(NTHR)
     // (vmcnt counts stores too: a wait placed after them would drain them).
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), expcnt/lgkmcnt unchanged
     __syncthreads();
-    store_tile(nr, b0, nb, dst_of(st));
+    store_tile(nr, b0, nb);
     __syncthreads();
     if (tn >= n_tiles) break;
-    // the next tile's state: its orbital phases (read by the next store, after
-    // several barriers)
-    if (MULTI && diag && stn != st)
-      for (int k = tid; k < 2 * n_diag; k += NTHR) dph[k] = diag[(long)stn * mt.diag_stride + k];
     if (!same_fiber) {
       f = fn;
       const bool tables = fdn.kp != fd.kp;
@@ -752,7 +721,7 @@ __global__ void __launch_bounds__(NTHR)
     }
     regs_to_lds(buf, nrn);
     if (FUSE) bfac_to_lds(bfn, b0n);
-    load_rows(kCovered, nrn, b0n, nbn, src_of(stn));
+    load_rows(kCovered, nrn, b0n, nbn);
     t = tn;
   }
 }

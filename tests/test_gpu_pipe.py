@@ -66,3 +66,35 @@ def test_ansatz_equals_its_gates(norb, nelec, dtype):
     err = (got - want).abs().max().item()
     assert err <= (TOL[dtype] if dtype == "complex128"
                    else TOL[dtype] * want.abs().max().item())
+
+
+# (norb, nelec, states): one workgroup's tile holds every string of a sector.  Each
+# tile size (256, 480 and 928 strings of 128 bytes, 960 of 64, 256 and 464 of
+# 256) with full and with ragged columns, down to a single one.
+SMALL = [(6, (3, 1), 1), (7, (6, 3), 3), (10, (5, 3), 2), (10, (5, 3), 40), (11, (5, 2), 1),
+         (11, (4, 6), 12), (12, (6, 1), 1), (12, (6, 4), 1), (12, (4, 6), 6)]
+
+
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("norb,nelec,n_states", SMALL)
+def test_small_sectors_in_place(norb, nelec, n_states, dtype):
+    """Whole-sector passes in place, both orientations, on states that lie one
+    element apart (8-byte alignment in complex64) with a guard between them."""
+    from ffsim_amd.gates.orbital_rotation import orbital_rotations_in_place
+
+    rng = np.random.default_rng(norb * 1000 + n_states)
+    dim = ffsim_amd.dim(norb, nelec)
+    facs = [O.random_state_vector(ffsim_amd.dim(norb, n), rng) for n in nelec]
+    buf = torch.full((n_states * (dim + 1) + 1,), 7.0, dtype=getattr(torch, dtype), device="cuda")
+    states = [buf[1 + i * (dim + 1):][:dim] for i in range(n_states)]
+    start = torch.from_numpy(np.kron(*facs).astype(dtype)).cuda()
+    mats = [tuple(ffsim_amd.random.random_unitary(norb, seed=rng) for _ in nelec)
+            for _ in range(n_states)]
+    for s in states:
+        s.copy_(start)
+    orbital_rotations_in_place(states, mats, norb, nelec)
+    assert torch.all(buf[:: dim + 1] == 7.0)
+    for i in {0, n_states // 2, n_states - 1}:
+        want = np.kron(*[_rotated(f, m, norb, n) for f, m, n in zip(facs, mats[i], nelec)])
+        bound = TOL[dtype] * (1.0 if dtype == "complex128" else np.abs(want).max())
+        assert np.abs(states[i].cpu().numpy() - want).max() <= bound

@@ -20,7 +20,8 @@ def lib(tmp_path_factory):
 
 # (window, electrons, 16-byte units per string)
 CASES = [(6, 3, 8), (7, 2, 8), (12, 6, 8), (12, 4, 8), (13, 7, 4), (13, 6, 4), (14, 7, 2),
-         (14, 5, 2), (15, 8, 1), (15, 7, 1), (16, 5, 1), (16, 1, 8), (16, 15, 8), (14, 14, 8)]
+         (14, 5, 2), (15, 8, 1), (15, 7, 1), (16, 5, 1), (16, 1, 8), (16, 15, 8), (14, 14, 8),
+         (10, 5, 16), (11, 6, 16), (6, 1, 16)]
 
 
 @pytest.mark.parametrize("merge", [0, 1])
