@@ -229,7 +229,7 @@ struct Context {
   // once (created on first use, default priority)
   std::vector<hipStream_t> aux;
   std::map<int, std::pair<uint32_t*, int32_t*>> ob_links;
-  std::map<std::tuple<int, int, int, bool, int>, std::unique_ptr<DevPipe>> pipe;
+  std::map<std::tuple<int, int, int, bool, int, int>, std::unique_ptr<DevPipe>> pipe;
   ProgramRing ring;
 };
 
@@ -461,14 +461,14 @@ const DevSchedule& dev_schedule(Context& ctx, const DevGroups& gr, int n_waves, 
   return g.schedules[key] = ds;
 }
 
-DevPipe& dev_pipe(Context& ctx, int w, int kp_lo, int kp_hi, bool merge, int units, size_t elem) {
+DevPipe& dev_pipe(Context& ctx, int w, int kp_lo, int kp_hi, bool merge, int units,
+                  int per_chunk) {
   std::lock_guard<std::mutex> lk(ctx.mu);
-  const auto key = std::make_tuple(w, kp_lo, kp_hi, merge, units);
+  const auto key = std::make_tuple(w, kp_lo, kp_hi, merge, units, per_chunk);
   auto it = ctx.pipe.find(key);
   if (it != ctx.pipe.end()) return *it->second;
   auto dp = std::make_unique<DevPipe>();
-  dp->host = make_pipe_groups(w, kp_lo, kp_hi, merge, units, kPipeCompute,
-                              64 / pipe_width(units, elem));
+  dp->host = make_pipe_groups(w, kp_lo, kp_hi, merge, units, kPipeCompute, per_chunk);
   dp->kp_lo = kp_lo;
   dp->kp_hi = kp_hi;
   return *(ctx.pipe[key] = std::move(dp));
@@ -806,6 +806,7 @@ void launch_fiber_t(const void* src, void* dst, long ld_src, long ld_dst, int n_
 // 1614 -> 945 us; complex64 153 -> 81, 324 -> 220 and 1080 -> 810 us.
 struct SectorGeom {
   int w = 0, units = 0, sweeps = 0;
+  int cols = 1;        // columns of a compute lane
   bool whole = false;  // a tile holds every string of the sector (one pass)
   bool small = false;  // in place, several states (norb <= 12)
 };
@@ -849,19 +850,23 @@ SectorGeom small_geom(int dtype, int norb, int nocc, long n_batch, int n_states)
   if (norb < kMaxSubWindow || norb > std::min(window_cap(), 12) || n_batch > (1l << 30) ||
       tile_width(dtype) != (dtype == FFSIM_C64 ? 4 : 8) || n_batch < (long)(16 / elem))
     return g;
-  const long rows = (long)binom(norb, nocc), W = pipe_width(8, elem);
+  const long rows = (long)binom(norb, nocc);
   if (rows == 0 || rows > pipe_max_rows(8, 29)) return g;
   g.whole = g.small = true;
   g.units = 8;
   g.sweeps = rows <= pipe_max_rows(8, 8) ? 8 : rows <= pipe_max_rows(8, 15) ? 15 : 29;
-  const long tiles = (long)((n_batch + W - 1) / W) * n_states;
-  if (g.sweeps == 29 && tiles < g_n_cu) {
+  auto tiles = [&]() {
+    const long w = pipe_width(g.units, elem);
+    return (n_batch + w - 1) / w * n_states;
+  };
+  if (g.sweeps == 29 && tiles() < g_n_cu) {
     g.units = 4;
     g.sweeps = 15;
-  } else if (rows <= pipe_max_rows(16, 29) && tiles > g_n_cu) {
+  } else if (rows <= pipe_max_rows(16, 29) && tiles() > g_n_cu) {
     g.units = 16;
     g.sweeps = rows <= pipe_max_rows(16, 16) ? 16 : 29;
   }
+  if (tiles() > g_n_cu && g.sweeps == 29) g.cols = pipe_cols(g.units, elem);
   return g;
 }
 int choose_window(Context& ctx, int norb, int nocc, int dtype);
@@ -877,12 +882,14 @@ SectorGeom sector_geom(Context& ctx, int dtype, int norb, int nocc, long n_batch
         g.w = norb;
         g.units = units;
         g.sweeps = pipe_sweeps(units);
+        g.cols = pipe_cols(units, elem);
         g.whole = true;
         return g;
       }
   if (g.w >= kMaxSubWindow && g.w <= 16 && n_batch >= pipe_width(8, elem)) {
     g.units = 8;
     g.sweeps = pipe_sweeps(8);
+    g.cols = pipe_cols(8, elem);
   }
   return g;
 }
@@ -892,7 +899,7 @@ SectorGeom sector_geom(Context& ctx, int dtype, int norb, int nocc, long n_batch
 // in rounds over the CUs, one pipelined tile per CU against one plain
 // complex128 tile or three plain complex64 tiles of a quarter of the columns.
 // Measured on the 12-orbital passes of norb 13 to 16: a round takes about 17.6
-// / 21 us (complex128) and 25.6 / 21.5 us (complex64), and a pipelined launch
+// / 21 us (complex128) and 24 / 21.5 us (complex64), and a pipelined launch
 // 16 us more to fill and drain, so it wins from 5 rounds on in complex128 (25
 // rounds: 482 against 538 us per launch; 2 rounds: 58 against 53).  Fibers
 // whose plain tiles leave room for a second workgroup per CU gain nothing from
@@ -911,13 +918,14 @@ bool pipe_applies(Context& ctx, int dtype, const SectorGeom& g, const DevWindow&
     const long tiles = (n_batch + width - 1) / width * n_f;
     return (double)((tiles + per_cu * g_n_cu - 1) / (per_cu * g_n_cu));
   };
-  return (c128 ? 17.6 : 25.6) * rounds(pipe_width(8, elem_bytes(dtype)), 1) + 16.0 <
+  return (c128 ? 17.6 : 24.0) * rounds(pipe_width(8, elem_bytes(dtype)), 1) + 16.0 <
          (c128 ? 21.0 * rounds(8, 1) : 21.5 * rounds(4, 3));
 }
 
 DevPipe& sector_pipe(Context& ctx, int dtype, int norb, int nocc, const SectorGeom& g) {
   return dev_pipe(ctx, g.w, std::max(0, nocc - (norb - g.w)), std::min(nocc, g.w),
-                  dtype == FFSIM_C64, g.units, elem_bytes(dtype));
+                  dtype == FFSIM_C64, g.units,
+                  64 / (pipe_width(g.units, elem_bytes(dtype)) / g.cols));
 }
 
 // The tables of one pass: its sub-window starts' images, kept on the device
@@ -986,11 +994,11 @@ void pipe_pass(int dtype, const SectorGeom& g, PipeLaunch L, const DevWindow& wi
                               : 2 * L.tstore + dg;
   const size_t lds = pipe_lds_bytes(g, elem, tb.dwords, variant, L.fz.n_fac, win.w);
   require(lds <= lds_max, FFSIM_ERR_VALUE, "pipelined tile exceeds LDS");
-  const void* kern = dtype == FFSIM_C128 ? pipe_kernel_c128(units, g.sweeps, variant)
-                                         : pipe_kernel_c64(units, g.sweeps, variant);
+  const void* kern = dtype == FFSIM_C128 ? pipe_kernel_c128(units, g.sweeps, g.cols, variant)
+                                         : pipe_kernel_c64(units, g.sweeps, g.cols, variant);
   require(kern != nullptr, FFSIM_ERR_VALUE, "pipelined pass: no such tile geometry");
-  static std::atomic<bool> attr_set[2][17][32][PIPE_VARIANTS] = {};
-  std::atomic<bool>& attr = attr_set[dtype][units][g.sweeps][variant];
+  static std::atomic<bool> attr_set[2][17][32][3][PIPE_VARIANTS] = {};
+  std::atomic<bool>& attr = attr_set[dtype][units][g.sweeps][g.cols][variant];
   if (!attr) {
     HIP_CHECK(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max));
     attr = true;

@@ -14,16 +14,14 @@
 // barriers, so the traffic is spread evenly over the sub-passes (all of it
 // before the first barrier instead: 2.27 ms per launch).
 //
-// Rows of 128 bytes for both types: 8 complex128 or 16 complex64 columns.  16
-// columns fill the complex64 chunks (4 groups x 16 columns: 20 groups of the
-// largest class are exactly 5 chunks), 23% fewer wave instructions than the 4
-// columns of fiber_kernel.
+// Rows of 128 bytes for both types: 8 complex128 or 16 complex64 columns, one
+// 16-byte unit to a compute lane (see pipe_cols).
 //
 // Measured at norb=16 (12870 x 12870, LUCJ n_reps=4, average launch): complex128
-// 2.28 -> 1.72 ms (3.1 TB/s algorithmic), complex64 1.49 -> 1.19 ms.  What bounds
-// it: without the memory waves' traffic and exchange a launch takes 1.47 / 1.13
-// ms, without the rotations 1.38 / 0.83 ms; the VALU is busy 49% / 60% of the
-// time, the rest of a sub-pass goes to its LDS reads and writes and the barrier.
+// 2.28 -> 1.72 ms (3.1 TB/s algorithmic), complex64 1.49 -> 1.12 ms.  What bounds
+// it: without the memory waves' traffic and exchange a complex128 launch takes
+// 1.47 ms, without the rotations 1.38; the VALU is busy 49% of the time, the rest
+// of a sub-pass goes to its LDS reads and writes and the barrier.
 //
 // SMALL launches rotate whole sectors in place (norb 6 to 12, one or several
 // states, strings on rows or on columns).  One tile per CU or few, so what
@@ -59,6 +57,14 @@ constexpr int pipe_sweeps(int units) { return units == 8 ? 29 : units == 1 ? 26 
 constexpr int pipe_max_rows(int units, int sweeps) { return pipe_step(units) * sweeps; }
 constexpr int pipe_max_rows(int units) { return pipe_max_rows(units, pipe_sweeps(units)); }
 constexpr int pipe_width(int units, size_t elem) { return units * 16 / (int)elem; }
+// Columns that a compute lane rotates together: complex64 passes with several
+// tiles per CU take both columns of a 16-byte unit, which halves the LDS
+// instructions, address and coefficient work of a rotation (norb 16 1.19 ->
+// 1.12 ms a launch, norb 15 0.79 -> 0.65, norb 14 0.197 -> 0.174).  A launch of
+// one tile per CU waits for one chunk's chain of instructions, which that doubles
+// (norb 12 39 -> 48 us, norb 13 69 -> 71): one column there, and for sectors of
+// at most 256 strings (64 states of norb 10: 58 us against 69).
+constexpr int pipe_cols(int units, size_t elem) { return units == 4 ? 1 : 16 / (int)elem; }
 
 // Tables of a pipelined pass: one image per electron count kp of the window,
 // laid out as the workgroup keeps it in LDS (dword offsets): PipeSlot per
@@ -86,21 +92,31 @@ struct PipeStates {
   long diag_stride;   // doubles
 };
 
-// Applies the layer pairs of one sub-pass to one register group (one batch
-// column): p is the group's base address in the tile, off its members' offsets.
-template <typename T, int W2, int K2>
+// Applies the layer pairs of one sub-pass to one register group (NC batch
+// columns): p is the group's base address in the tile, off its members' offsets.
+template <typename T, int W2, int K2, int NC>
 __device__ __forceinline__ void pipe_group_apply(unsigned char* p, const uint32_t* __restrict__ off,
                                                  const LayerPair* lp, int n_lp, bool flip) {
   constexpr int N = binom_const(W2, K2);
-  Cx<T> v[N];
-  Cx<T>* at[N];
+  struct alignas(NC * sizeof(Cx<T>)) Unit { Cx<T> c[NC]; };
+  Cx<T> v[NC * N];  // column-major
+  Unit* at[N];
 #pragma unroll
-  for (int m = 0; m < N; ++m) at[m] = reinterpret_cast<Cx<T>*>(p + off[m]);
+  for (int m = 0; m < N; ++m) at[m] = reinterpret_cast<Unit*>(p + off[m]);
 #pragma unroll
-  for (int m = 0; m < N; ++m) v[m] = *at[m];
-  apply_layers<T, W2, K2>(v, lp, n_lp, flip);
+  for (int m = 0; m < N; ++m) {
+    const Unit x = *at[m];
 #pragma unroll
-  for (int m = 0; m < N; ++m) *at[m] = v[m];
+    for (int k = 0; k < NC; ++k) v[k * N + m] = x.c[k];
+  }
+  apply_layers<T, W2, K2, NC>(v, lp, n_lp, flip);
+#pragma unroll
+  for (int m = 0; m < N; ++m) {
+    Unit x;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) x.c[k] = v[k * N + m];
+    *at[m] = x;
+  }
 }
 
 // A diagonal Coulomb evolution fused into the store of a transposing pass,
@@ -119,7 +135,7 @@ struct PipeFuse {
 // rows or (COLS) on columns, with phases if diag is given.  Tiles of fewer
 // than 8 units and SMALL ones hold a whole sector (rows 0, 1, ..., one fiber
 // of whole_rows strings with whole_kp electrons).
-template <typename T, int UNITS, int SWEEPS, bool TST, bool DG, bool FUSE, bool SMALL, bool COLS>
+template <typename T, int UNITS, int SWEEPS, int NC, bool TST, bool DG, bool FUSE, bool SMALL, bool COLS>
 __global__ void __launch_bounds__(kPipeThreads)
     fiber_pipe_kernel(const Cx<T>* src, Cx<T>* dst, long ld_src, long ld_dst, int n_batch,
                       const Fiber* __restrict__ fibers, int n_fibers,
@@ -225,19 +241,19 @@ __global__ void __launch_bounds__(kPipeThreads)
         const int nc = (int)wsched[(P.slot * NW + wave) * 2 + 1];
         for (int c = 0; c < nc; ++c) {
           const uint32_t ch = wchunks[c0 + c];
-          const int gl = lane / W, j = lane % W;
+          const int gl = lane / (W / NC), j = lane % (W / NC);
           if (gl < (int)(ch & 0xff)) {
             const uint32_t d = gdesc[gs.d_off + (int)(ch >> 8) + gl];
-            unsigned char* p = cur + (d >> 16) * (16 * UNITS) + j * (int)sizeof(Cx<T>);
+            unsigned char* p = cur + (d >> 16) * (16 * UNITS) + j * (int)(NC * sizeof(Cx<T>));
             const uint32_t* mo = goff + gs.o_off + ((d >> 4) & 0xfff) * 4;
             const bool flip = (d >> 3) & 1;
             switch (d & 7) {
-              case 1: pipe_group_apply<T, W2, 1>(p, mo, lp, P.n_lp, flip); break;
-              case 2: pipe_group_apply<T, W2, 2>(p, mo, lp, P.n_lp, flip); break;
-              case 3: pipe_group_apply<T, W2, 3>(p, mo, lp, P.n_lp, flip); break;
+              case 1: pipe_group_apply<T, W2, 1, NC>(p, mo, lp, P.n_lp, flip); break;
+              case 2: pipe_group_apply<T, W2, 2, NC>(p, mo, lp, P.n_lp, flip); break;
+              case 3: pipe_group_apply<T, W2, 3, NC>(p, mo, lp, P.n_lp, flip); break;
               // complex64 groups of 4 and 5 electrons are complemented ones of 2 and 1
-              case 4: if constexpr (sizeof(T) == 8) pipe_group_apply<T, W2, 4>(p, mo, lp, P.n_lp, flip); break;
-              case 5: if constexpr (sizeof(T) == 8) pipe_group_apply<T, W2, 5>(p, mo, lp, P.n_lp, flip); break;
+              case 4: if constexpr (sizeof(T) == 8) pipe_group_apply<T, W2, 4, NC>(p, mo, lp, P.n_lp, flip); break;
+              case 5: if constexpr (sizeof(T) == 8) pipe_group_apply<T, W2, 5, NC>(p, mo, lp, P.n_lp, flip); break;
               default: break;
             }
           }
@@ -618,48 +634,56 @@ __global__ void __launch_bounds__(kPipeThreads)
 // instantiations of each type are compiled apart).
 enum { PIPE_PLAIN = 0, PIPE_PHASES = 1, PIPE_TRANSPOSE = 2, PIPE_TRANSPOSE_PHASES = 3, PIPE_FUSED = 4,
        PIPE_SMALL_ROWS = 5, PIPE_SMALL_COLS = 6, PIPE_VARIANTS = 7 };
-template <typename T, int UNITS>
+template <typename T, int UNITS, int NC>
 const void* pipe_kernel_units(int variant) {
   constexpr int S = pipe_sweeps(UNITS);
   switch (variant) {
     case PIPE_PLAIN:
-      return (const void*)fiber_pipe_kernel<T, UNITS, S, false, false, false, false, false>;
+      return (const void*)fiber_pipe_kernel<T, UNITS, S, NC, false, false, false, false, false>;
     case PIPE_PHASES:
-      return (const void*)fiber_pipe_kernel<T, UNITS, S, false, true, false, false, false>;
+      return (const void*)fiber_pipe_kernel<T, UNITS, S, NC, false, true, false, false, false>;
     case PIPE_TRANSPOSE:
-      return (const void*)fiber_pipe_kernel<T, UNITS, S, true, false, false, false, false>;
+      return (const void*)fiber_pipe_kernel<T, UNITS, S, NC, true, false, false, false, false>;
     case PIPE_TRANSPOSE_PHASES:
-      return (const void*)fiber_pipe_kernel<T, UNITS, S, true, true, false, false, false>;
-    default: return (const void*)fiber_pipe_kernel<T, UNITS, S, true, false, true, false, false>;
+      return (const void*)fiber_pipe_kernel<T, UNITS, S, NC, true, true, false, false, false>;
+    default: return (const void*)fiber_pipe_kernel<T, UNITS, S, NC, true, false, true, false, false>;
   }
 }
-template <typename T, int UNITS, int SWEEPS>
+template <typename T, int UNITS, int SWEEPS, int NC>
 const void* pipe_kernel_small(int variant) {
   return variant == PIPE_SMALL_ROWS
-             ? (const void*)fiber_pipe_kernel<T, UNITS, SWEEPS, false, true, false, true, false>
-             : (const void*)fiber_pipe_kernel<T, UNITS, SWEEPS, false, true, false, true, true>;
+             ? (const void*)fiber_pipe_kernel<T, UNITS, SWEEPS, NC, false, true, false, true, false>
+             : (const void*)fiber_pipe_kernel<T, UNITS, SWEEPS, NC, false, true, false, true, true>;
 }
 template <typename T>
-const void* pipe_kernel(int units, int sweeps, int variant) {
+const void* pipe_kernel(int units, int sweeps, int cols, int variant) {
+  constexpr int EU = 16 / (int)sizeof(Cx<T>);  // columns of a unit
+  if (cols != 1 && cols != EU) return nullptr;
   if (variant >= PIPE_SMALL_ROWS) {
-    if (units == 4 && sweeps == 15) return pipe_kernel_small<T, 4, 15>(variant);
-    if (units == 8 && sweeps == 8) return pipe_kernel_small<T, 8, 8>(variant);
-    if (units == 8 && sweeps == 15) return pipe_kernel_small<T, 8, 15>(variant);
-    if (units == 8 && sweeps == 29) return pipe_kernel_small<T, 8, 29>(variant);
-    if (units == 16 && sweeps == 16) return pipe_kernel_small<T, 16, 16>(variant);
-    if (units == 16 && sweeps == 29) return pipe_kernel_small<T, 16, 29>(variant);
+    if (cols == 1) {
+      if (units == 4 && sweeps == 15) return pipe_kernel_small<T, 4, 15, 1>(variant);
+      if (units == 8 && sweeps == 8) return pipe_kernel_small<T, 8, 8, 1>(variant);
+      if (units == 8 && sweeps == 15) return pipe_kernel_small<T, 8, 15, 1>(variant);
+      if (units == 16 && sweeps == 16) return pipe_kernel_small<T, 16, 16, 1>(variant);
+    }
+    if (units == 8 && sweeps == 29)
+      return cols == 1 ? pipe_kernel_small<T, 8, 29, 1>(variant)
+                       : pipe_kernel_small<T, 8, 29, EU>(variant);
+    if (units == 16 && sweeps == 29)
+      return cols == 1 ? pipe_kernel_small<T, 16, 29, 1>(variant)
+                       : pipe_kernel_small<T, 16, 29, EU>(variant);
     return nullptr;
   }
-  if (sweeps != pipe_sweeps(units)) return nullptr;
+  if (sweeps != pipe_sweeps(units) || cols != pipe_cols(units, sizeof(Cx<T>))) return nullptr;
   switch (units) {
-    case 8: return pipe_kernel_units<T, 8>(variant);
-    case 4: return pipe_kernel_units<T, 4>(variant);
-    case 2: return pipe_kernel_units<T, 2>(variant);
-    case 1: return pipe_kernel_units<T, 1>(variant);
+    case 8: return pipe_kernel_units<T, 8, EU>(variant);
+    case 4: return pipe_kernel_units<T, 4, 1>(variant);
+    case 2: return pipe_kernel_units<T, 2, EU>(variant);
+    case 1: return pipe_kernel_units<T, 1, EU>(variant);
     default: return nullptr;
   }
 }
-const void* pipe_kernel_c128(int units, int sweeps, int variant);
-const void* pipe_kernel_c64(int units, int sweeps, int variant);
+const void* pipe_kernel_c128(int units, int sweeps, int cols, int variant);
+const void* pipe_kernel_c64(int units, int sweeps, int cols, int variant);
 
 }  // namespace ffsim_amd

@@ -2,7 +2,7 @@
 #include "fiber_pipe.hpp"
 
 namespace ffsim_amd {
-const void* pipe_kernel_c64(int units, int sweeps, int variant) {
-  return pipe_kernel<float>(units, sweeps, variant);
+const void* pipe_kernel_c64(int units, int sweeps, int cols, int variant) {
+  return pipe_kernel<float>(units, sweeps, cols, variant);
 }
 }  // namespace ffsim_amd

@@ -179,23 +179,27 @@ __device__ __forceinline__ void rot_sub_vsr(Cx<T>* v, T c, T sr, T si) {
 // x' = c x + s y, y' = c y - conj(s) x with x <-> y is the same update with
 // s -> -conj(s).  Self-complementary classes (2 K2 == W2) are never flipped,
 // and c128 tables have no complemented groups (Re(sigma) stays in SGPRs).
-template <typename T, int W2, int K2, int P>
+template <typename T, int W2, int K2, int P, int NC>
 __device__ __forceinline__ void slot_apply(Cx<T>* v, const double* c, const double* sr,
                                            const double* si, int mask, bool flip) {
   if constexpr (P + 1 < W2) {
     if (mask & (1 << P)) {
+      constexpr int N = binom_const(W2, K2);
       if constexpr (2 * K2 == W2 || sizeof(T) == 8) {
-        rot_sub<T, W2, K2, P>(v, (T)c[P], (T)sr[P], (T)si[P]);
+#pragma unroll
+        for (int k = 0; k < NC; ++k)
+          rot_sub<T, W2, K2, P>(v + k * N, (T)c[P], (T)sr[P], (T)si[P]);
       } else {
         const T s = flip ? -(T)sr[P] : (T)sr[P];
-        rot_sub_vsr<T, W2, K2, P>(v, (T)c[P], s, (T)si[P]);
+#pragma unroll
+        for (int k = 0; k < NC; ++k) rot_sub_vsr<T, W2, K2, P>(v + k * N, (T)c[P], s, (T)si[P]);
       }
     }
   }
 }
 
 // Applies the layer pairs of one sub-pass to a group's members in registers.
-template <typename T, int W2, int K2>
+template <typename T, int W2, int K2, int NC = 1>
 __device__ __forceinline__ void apply_layers(Cx<T>* v, const LayerPair* lp, int n_lp, bool flip) {
   for (int l = 0; l < n_lp; ++l) {
     // one batch of scalar loads for the whole layer pair (uniform over the wave)
@@ -215,11 +219,11 @@ __device__ __forceinline__ void apply_layers(Cx<T>* v, const LayerPair* lp, int 
     asm volatile("" ::"s"(c[0]), "s"(sr[0]), "s"(si[0]), "s"(c[1]), "s"(sr[1]), "s"(si[1]),
                  "s"(c[2]), "s"(sr[2]), "s"(si[2]), "s"(c[3]), "s"(sr[3]), "s"(si[3]),
                  "s"(c[4]), "s"(sr[4]), "s"(si[4]));
-    slot_apply<T, W2, K2, 0>(v, c, sr, si, mask, flip);
-    slot_apply<T, W2, K2, 2>(v, c, sr, si, mask, flip);
-    slot_apply<T, W2, K2, 4>(v, c, sr, si, mask, flip);
-    slot_apply<T, W2, K2, 1>(v, c, sr, si, mask, flip);
-    slot_apply<T, W2, K2, 3>(v, c, sr, si, mask, flip);
+    slot_apply<T, W2, K2, 0, NC>(v, c, sr, si, mask, flip);
+    slot_apply<T, W2, K2, 2, NC>(v, c, sr, si, mask, flip);
+    slot_apply<T, W2, K2, 4, NC>(v, c, sr, si, mask, flip);
+    slot_apply<T, W2, K2, 1, NC>(v, c, sr, si, mask, flip);
+    slot_apply<T, W2, K2, 3, NC>(v, c, sr, si, mask, flip);
   }
 }
 

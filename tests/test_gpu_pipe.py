@@ -72,7 +72,7 @@ def test_ansatz_equals_its_gates(norb, nelec, dtype):
 # tile size (256, 480 and 928 strings of 128 bytes, 960 of 64, 256 and 464 of
 # 256) with full and with ragged columns, down to a single one.
 SMALL = [(6, (3, 1), 1), (7, (6, 3), 3), (10, (5, 3), 2), (10, (5, 3), 40), (11, (5, 2), 1),
-         (11, (4, 6), 12), (12, (6, 1), 1), (12, (6, 4), 1), (12, (4, 6), 6)]
+         (11, (4, 6), 12), (11, (4, 6), 20), (12, (6, 1), 1), (12, (6, 4), 1), (12, (4, 6), 6)]
 
 
 @pytest.mark.parametrize("dtype", ["complex128", "complex64"])
