@@ -809,18 +809,37 @@ __global__ void __launch_bounds__(256)
   const double* lin_row = coef + 3 * n * n;
   const int tid = threadIdx.x;
 
+  struct Col {
+    Cx<T> v[R];
+    uint64_t bits;
+    double g0, g1;  // evolution: column factor (cos, sin); else gamma, unused
+  };
+  auto load = [&](int c, Col& k) {
+    const int cc = min(c, c_hi - 1);
+    k.bits = col_str[cc];
+    if (MODE == DIAG_EVOLVE) {
+      k.g0 = colv ? colv[2 * cc] : 1.0;
+      k.g1 = colv ? colv[2 * cc + 1] : 0.0;
+    } else {
+      k.g0 = colv ? colv[cc] : 0.0;
+      k.g1 = 0.0;
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int rr = min(r0 + r, n_rows - 1);
+      k.v[r] = src[(long)rr * ld + cc];
+    }
+  };
   // cross vectors w_a[q] (rows beyond n_rows get zeros and are never stored)
   for (int t = tid; t < R * n; t += NT) {
     const int r = t / n, q = t % n;
     double acc = 0.0;
     if (r0 + r < n_rows && (flags & DF_CROSS)) {
       const uint64_t bits = row_str[r0 + r];
+#pragma unroll 8
       for (int i = 0; i < n; ++i) {
-        const int occ = (bits >> i) & 1;
-        if (z)
-          acc += (occ ? -1.0 : 1.0) * X[i * n + q];
-        else if (occ)
-          acc += X[i * n + q];
+        const double x = X[i * n + q];
+        acc += ((bits >> i) & 1) ? (z ? -x : x) : (z ? x : 0.0);
       }
     }
     w_row[r][q] = acc;
@@ -832,15 +851,15 @@ __global__ void __launch_bounds__(256)
     if (r0 + r < n_rows) {
       const uint64_t bits = row_str[r0 + r];
       if (flags & DF_QUAD) {
+#pragma unroll 4
         for (int p = l; p < n * n; p += LPR) {
           const int j = p / n, k = p % n;
-          if (k < j) continue;
+          const double x = A_row[p];
           const int oj = (bits >> j) & 1, ok = (bits >> k) & 1;
-          if (z) {
-            if (k > j) acc += ((oj ^ ok) ? -1.0 : 1.0) * A_row[j * n + k];
-          } else if (oj && ok) {
-            acc += A_row[j * n + k];
-          }
+          if (z)
+            acc += k > j ? ((oj ^ ok) ? -x : x) : 0.0;
+          else
+            acc += (k >= j && oj && ok) ? x : 0.0;
         }
       }
       if (flags & DF_LIN)
@@ -851,6 +870,10 @@ __global__ void __launch_bounds__(256)
     for (int o = LPR / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, LPR);
     if (l == 0) rho[r] = acc;
   }
+  // the first columns come in while the row factors are formed
+  Col A, B;
+  int c = c_lo + tid;
+  if (c < c_hi) load(c, A);
   __syncthreads();
   if (MODE == DIAG_EVOLVE) {
     // per-orbital factors and row factors, angle = -scale * term
@@ -880,27 +903,6 @@ __global__ void __launch_bounds__(256)
   }
   __syncthreads();
 
-  struct Col {
-    Cx<T> v[R];
-    uint64_t bits;
-    double g0, g1;  // evolution: column factor (cos, sin); else gamma, unused
-  };
-  auto load = [&](int c, Col& k) {
-    const int cc = min(c, c_hi - 1);
-    k.bits = col_str[cc];
-    if (MODE == DIAG_EVOLVE) {
-      k.g0 = colv ? colv[2 * cc] : 1.0;
-      k.g1 = colv ? colv[2 * cc + 1] : 0.0;
-    } else {
-      k.g0 = colv ? colv[cc] : 0.0;
-      k.g1 = 0.0;
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int rr = min(r0 + r, n_rows - 1);
-      k.v[r] = src[(long)rr * ld + cc];
-    }
-  };
   auto form = [&](int c, const Col& k) {
     if (c >= c_hi) return;
     if (MODE == DIAG_EVOLVE) {
@@ -965,9 +967,6 @@ __global__ void __launch_bounds__(256)
   };
   // two columns per step: B's loads are in flight while A is formed, and A's
   // next loads while B is formed
-  Col A, B;
-  int c = c_lo + tid;
-  if (c < c_hi) load(c, A);
   for (; c < c_hi; c += 2 * NT) {
     load(c + NT, B);
     form(c, A);
