@@ -1207,6 +1207,7 @@ SectorRotation prepare_rotation(const cdouble* mat, int norb, int w) {
   SectorRotation r;
   GivensDecomposition g = triangle_order(norb, w) ? triangle_decomposition(mat, norb, 1e-12)
                                                   : givens_decomposition(mat, norb, 1e-12);
+  r.steps.reserve(g.rotations.size());
   for (const auto& rot : g.rotations) r.steps.push_back(kernel_step_from_rotation(rot));
   r.diag = g.diag;
   for (const auto& d : g.diag)
@@ -2010,20 +2011,35 @@ bool plan_multi_sector(const std::vector<const SectorRotation*>& rots, int norb,
   return true;
 }
 
+// Offsets of a planned sector rotation in the call's program.
+struct MultiUpload {
+  size_t diag_off = 0;
+  std::vector<std::pair<size_t, size_t>> passes;  // (layer pairs, sub-passes)
+};
+MultiUpload upload_multi_sector(Program& prog, const MultiSector& ms) {
+  MultiUpload up;
+  if (ms.need_diag) up.diag_off = prog.append(ms.diag.data(), ms.diag.size() * sizeof(double));
+  for (const MultiSector::Pass& P : ms.passes) {
+    const size_t soff = prog.append(P.layers.data(), P.layers.size() * sizeof(LayerPair));
+    up.passes.emplace_back(soff, prog.append(P.subs.data(), P.subs.size() * sizeof(SubPass)));
+  }
+  return up;
+}
+
 // Queues the passes of a planned multi-state sector rotation: one launch per
 // pass over the tiles of every state (`states`, a device array of the m state
 // addresses in the call's program).
-void queue_multi_sector(Context& ctx, Program& prog, const MultiSector& ms, int dtype, int mode,
+void queue_multi_sector(Context& ctx, Program& prog, const MultiSector& ms,
+                        const MultiUpload& up, int dtype, int mode,
                         size_t states_off, int m, long ld, int n_batch, int norb, int nocc,
                         hipStream_t stream, std::vector<std::function<void()>>& launches) {
   const DevStrings& ds = dev_strings(ctx, norb, nocc);
   const SectorGeom geom = small_geom(dtype, norb, nocc, n_batch, m);
   require(geom.small, FFSIM_ERR_VALUE, "multi-state pass: unsupported shape");
-  size_t diag_off = 0;
-  if (ms.need_diag) diag_off = prog.append(ms.diag.data(), ms.diag.size() * sizeof(double));
-  for (const MultiSector::Pass& P : ms.passes) {
-    const size_t soff = prog.append(P.layers.data(), P.layers.size() * sizeof(LayerPair));
-    const size_t poff = prog.append(P.subs.data(), P.subs.size() * sizeof(SubPass));
+  const size_t diag_off = up.diag_off;
+  for (size_t k = 0; k < ms.passes.size(); ++k) {
+    const MultiSector::Pass& P = ms.passes[k];
+    const size_t soff = up.passes[k].first, poff = up.passes[k].second;
     size_t img_off = 0;
     const PipeTables tb0 =
         pass_tables(ctx, sector_pipe(ctx, dtype, norb, nocc, geom), P.subs, prog, &img_off);
@@ -2057,6 +2073,7 @@ bool multi_applies(Context& ctx, int dtype, int n, int na, int nb) {
 struct MultiRotation {
   MultiSector a, b;
   bool has_a = false, has_b = false;
+  bool same = false;  // both sectors by the same matrices: one plan (a), uploaded once
 };
 
 // mats_a[i], mats_b[i]: state i's matrices; a sector whose first entry is null
@@ -2068,34 +2085,45 @@ bool plan_multi_rotation(int n, const std::vector<const cdouble*>& mats_a,
   const size_t m = mats_a.size();
   mr.has_a = mats_a[0] != nullptr;
   mr.has_b = mats_b[0] != nullptr;
-  std::vector<SectorRotation> ra(m), rb(m);
+  mr.same = mr.has_a && mr.has_b;
+  for (size_t i = 0; i < m && mr.same; ++i)
+    mr.same = std::memcmp(mats_a[i], mats_b[i], sizeof(cdouble) * n * n) == 0;
+  std::vector<SectorRotation> ra(m), rb(mr.same ? 0 : m);
   std::vector<const SectorRotation*> pa(m), pb(m);
   for (size_t i = 0; i < m; ++i) {
     if (mr.has_a) ra[i] = prepare_rotation(mats_a[i], n, n);
+    pa[i] = &ra[i];
+    if (mr.same) continue;
     if (mr.has_b) {
       if (mr.has_a && std::memcmp(mats_a[i], mats_b[i], sizeof(cdouble) * n * n) == 0)
         rb[i] = ra[i];
       else
         rb[i] = prepare_rotation(mats_b[i], n, n);
     }
-    pa[i] = &ra[i];
     pb[i] = &rb[i];
   }
   return (!mr.has_a || plan_multi_sector(pa, n, n, mr.a)) &&
-         (!mr.has_b || plan_multi_sector(pb, n, n, mr.b));
+         (!mr.has_b || mr.same || plan_multi_sector(pb, n, n, mr.b));
 }
 
 // Queues a planned multi-state rotation: the alpha sector's passes (strings on
 // rows), then the beta sector's (strings on columns), in place.
 void queue_multi_rotation(Context& ctx, Program& prog, const MultiRotation& mr, int dtype,
-                          size_t states_off, int m, int n, int na, int nb, hipStream_t stream, std::vector<std::function<void()>>& launches) {
+                          size_t states_off, int m, int n, int na, int nb, hipStream_t stream,
+                          std::vector<std::function<void()>>& launches) {
   const long da = (long)binom(n, na), db = (long)binom(n, nb);
-  if (mr.has_a)
-    queue_multi_sector(ctx, prog, mr.a, dtype, MODE_ROWS, states_off, m, db, (int)db, n, na,
+  MultiUpload up;
+  if (mr.has_a) {
+    up = upload_multi_sector(prog, mr.a);
+    queue_multi_sector(ctx, prog, mr.a, up, dtype, MODE_ROWS, states_off, m, db, (int)db, n, na,
                        stream, launches);
-  if (mr.has_b)
-    queue_multi_sector(ctx, prog, mr.b, dtype, MODE_COLS, states_off, m, db, (int)da, n, nb,
+  }
+  if (mr.has_b) {
+    const MultiSector& b = mr.same ? mr.a : mr.b;
+    if (!mr.same) up = upload_multi_sector(prog, b);
+    queue_multi_sector(ctx, prog, b, up, dtype, MODE_COLS, states_off, m, db, (int)da, n, nb,
                        stream, launches);
+  }
 }
 
 // A batch of spin-balanced UCJ applications of one shape on the Givens path

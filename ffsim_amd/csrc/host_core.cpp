@@ -799,21 +799,44 @@ namespace {
 // Rotation that zeroes b against a: returns (c, s) with c real such that
 // c*b - conj(s)*a == 0 for the column/row updates below (BLAS zrotg
 // convention with thresholds, as the decomposition contract requires).
-void zrotg_tol(cdouble a, cdouble b, double tol, double& c, cdouble& s) {
-  double aa = std::abs(a), ab = std::abs(b);
-  if (ab <= tol) {
-    c = 1.0;
-    s = 0.0;
-    return;
+// The moduli are formed in extended precision, without hypot's scaling (the
+// squares of doubles neither overflow nor vanish there).  False where |b| is not
+// above tol: nothing to rotate, c = 1, or c = s = NaN for a NaN.
+bool zrotg_tol(cdouble a, cdouble b, double tol, double& c, cdouble& s) {
+  typedef long double ld;
+  const ld ar = a.real(), ai = a.imag(), br = b.real(), bi = b.imag();
+  const ld na = ar * ar + ai * ai, nb = br * br + bi * bi, t2 = (ld)tol * tol;
+  if (!(nb > t2)) {
+    c = nb <= t2 ? 1.0 : (double)nb;
+    s = nb <= t2 ? 0.0 : (double)nb;
+    return false;
   }
-  if (aa <= tol) {
+  if (na <= t2) {
     c = 0.0;
     s = 1.0;
-    return;
+    return true;
   }
-  double r = std::hypot(aa, ab);
-  c = std::min(1.0, std::max(-1.0, aa / r));
-  s = (a / aa) * std::conj(b) / r;
+  const ld aa = std::sqrt(na), r = std::sqrt(na + nb), f = 1 / (aa * r);
+  c = std::min(1.0, (double)(na * f));
+  s = cdouble((double)((ar * br + ai * bi) * f), (double)((ai * br - ar * bi) * f));
+  return true;
+}
+
+// x <- c x + s y, y <- c y - conj(s) x over n elements `stride` apart, in the
+// products' own terms: std::complex multiplications test every result for NaN
+// (a 10 x 10 decomposition 4.4 -> 3.6 us; 2.0 with zrotg_tol's moduli and
+// without the nulled elements).
+void rotate_pair(cdouble* x, cdouble* y, int n, size_t stride, double c, cdouble s) {
+  const double sr = s.real(), si = s.imag();
+  double* px = reinterpret_cast<double*>(x);
+  double* py = reinterpret_cast<double*>(y);
+  for (int k = 0; k < n; ++k, px += 2 * stride, py += 2 * stride) {
+    const double xr = px[0], xi = px[1], yr = py[0], yi = py[1];
+    px[0] = c * xr + (sr * yr - si * yi);
+    px[1] = c * xi + (sr * yi + si * yr);
+    py[0] = c * yr - (sr * xr + si * xi);
+    py[1] = c * yi - (sr * xi - si * xr);
+  }
 }
 }  // namespace
 
@@ -821,46 +844,38 @@ GivensDecomposition givens_decomposition(const cdouble* mat, int n, double tol) 
   GivensDecomposition out;
   std::vector<cdouble> M(mat, mat + (size_t)n * n);
   auto at = [&](int r, int c) -> cdouble& { return M[(size_t)r * n + c]; };
-  // column update on (x, y): x <- c x + s y, y <- c y - conj(s) x  (M <- M G^T)
-  auto rot_cols = [&](int x, int y, double c, cdouble s) {
-    for (int r = 0; r < n; ++r) {
-      cdouble xo = at(r, x), yo = at(r, y);
-      at(r, x) = c * xo + s * yo;
-      at(r, y) = c * yo - std::conj(s) * xo;
-    }
+  // M <- M G^T on columns (x, y) down to the row of the nulled element, M <- G M
+  // on rows from its column on, with the same 2x2: both are nulled beyond
+  auto rot_cols = [&](int x, int y, int row, double c, cdouble s) {
+    rotate_pair(&at(0, x), &at(0, y), row + 1, n, c, s);
   };
-  // row update on (x, y) with the same 2x2 (M <- G M)
-  auto rot_rows = [&](int x, int y, double c, cdouble s) {
-    for (int k = 0; k < n; ++k) {
-      cdouble xo = at(x, k), yo = at(y, k);
-      at(x, k) = c * xo + s * yo;
-      at(y, k) = c * yo - std::conj(s) * xo;
-    }
+  auto rot_rows = [&](int x, int y, int col, double c, cdouble s) {
+    rotate_pair(&at(x, col), &at(y, col), n - col, 1, c, s);
   };
   std::vector<GivensRotation> right, left;
+  right.reserve((size_t)n * (n - 1) / 2);
+  left.reserve((size_t)n * (n - 1) / 2);
   // Clements et al., Optica 3, 1460 (2016): alternate nulling anti-diagonals
   // from the right (column rotations) and from the left (row rotations).
   for (int d = 0; d + 1 < n; ++d) {
     if (d % 2 == 0) {
       for (int t = 0; t <= d; ++t) {
         int col = d - t, row = n - 1 - t;
-        if (std::abs(at(row, col)) > tol) {
-          double c;
-          cdouble s;
-          zrotg_tol(at(row, col + 1), at(row, col), tol, c, s);
+        double c;
+        cdouble s;
+        if (zrotg_tol(at(row, col + 1), at(row, col), tol, c, s)) {
           right.push_back({c, s, col + 1, col});
-          rot_cols(col + 1, col, c, s);
+          rot_cols(col + 1, col, row, c, s);
         }
       }
     } else {
       for (int t = 0; t <= d; ++t) {
         int row = n - 1 - d + t, col = t;
-        if (std::abs(at(row, col)) > tol) {
-          double c;
-          cdouble s;
-          zrotg_tol(at(row - 1, col), at(row, col), tol, c, s);
+        double c;
+        cdouble s;
+        if (zrotg_tol(at(row - 1, col), at(row, col), tol, c, s)) {
           left.push_back({c, s, row - 1, row});
-          rot_rows(row - 1, row, c, s);
+          rot_rows(row - 1, row, col, c, s);
         }
       }
     }
@@ -870,7 +885,7 @@ GivensDecomposition givens_decomposition(const cdouble* mat, int n, double tol) 
   // diagonal: L^H diag(d) = diag(d) G'^* with G' = (c, -conj(s) d_i conj(d_j)).
   std::vector<cdouble> d(n);
   for (int k = 0; k < n; ++k) d[k] = at(k, k);
-  out.rotations = right;
+  out.rotations = std::move(right);
   for (auto it = left.rbegin(); it != left.rend(); ++it) {
     const GivensRotation& g = *it;
     cdouble sp = -std::conj(g.s) * d[g.i] * std::conj(d[g.j]);
@@ -890,16 +905,11 @@ GivensDecomposition triangle_decomposition(const cdouble* mat, int n, double tol
   // with no rotation moved through the diagonal.
   for (int row = n - 1; row >= 1; --row) {
     for (int col = 0; col < row; ++col) {
-      if (std::abs(at(row, col)) <= tol) continue;
       double c;
       cdouble s;
-      zrotg_tol(at(row, col + 1), at(row, col), tol, c, s);
+      if (!zrotg_tol(at(row, col + 1), at(row, col), tol, c, s) && c == 1.0) continue;
       out.rotations.push_back({c, s, col + 1, col});
-      for (int r = 0; r < n; ++r) {
-        const cdouble xo = at(r, col + 1), yo = at(r, col);
-        at(r, col + 1) = c * xo + s * yo;
-        at(r, col) = c * yo - std::conj(s) * xo;
-      }
+      rotate_pair(&at(0, col + 1), &at(0, col), row + 1, n, c, s);
     }
   }
   out.diag.resize(n);
