@@ -1408,10 +1408,48 @@ bool pipe_fuse_applies(Context& ctx, int dtype, int norb, int na, int nb, int n_
          fits(nb, gb, PIPE_FUSED, n_fac);
 }
 
+// Queues a diagonal operator (its column terms and the elementwise pass) in a
+// call's program; false, with nothing queued, if its scratch does not fit there.
+bool queue_diag(Context& ctx, Program& prog, int op, const void* src, void* dst, int dtype,
+                int norb, int nrow_occ, int ncol_occ, const DiagSpec& spec, hipStream_t stream,
+                std::vector<std::function<void()>>& launches) {
+  const long n_rows = (long)binom(norb, nrow_occ), n_cols = (long)binom(norb, ncol_occ);
+  require(norb <= 63, FFSIM_ERR_VALUE, "norb > 63 unsupported");
+  require(spec.norb == norb, FFSIM_ERR_VALUE, "diagonal operator of another norb");
+  require(diag_grid(n_rows, n_cols).y <= 65535, FFSIM_ERR_VALUE, "too many columns");
+  const DevStrings& rs = dev_strings(ctx, norb, nrow_occ);
+  const DevStrings& cs = dev_strings(ctx, norb, ncol_occ);
+  // per column: gamma (contractions) or its phase factor (cos, sin) (evolution)
+  const int evolve = op == DIAG_EVOLVE ? 1 : 0;
+  size_t goff = 0;
+  if (!prog.reserve((size_t)n_cols * (evolve ? 2 : 1) * sizeof(double), &goff)) return false;
+  const std::pair<size_t, size_t> par = append_diag_params(prog, spec);
+  const size_t hoff = par.first, coff = par.second;
+  launches.push_back([=, &prog, &rs, &cs]() {
+    const DiagHeader* dh = prog.dev<DiagHeader>(hoff);
+    const double* dc = prog.dev<double>(coff);
+    double* dg = prog.scratch<double>(goff);
+    launch_diag_col_term(n_cols, cs.d, dh, dc, dg, evolve, stream);
+    HIP_CHECK(hipGetLastError());
+    const double moved = (double)elem_bytes(dtype) * (double)n_rows * (double)n_cols *
+                         (op == DIAG_CONTRACT_ACC ? 3.0 : 2.0);
+    const long pk = prof_start(PROF_DIAG, moved, stream);
+    if (dtype == FFSIM_C128)
+      launch_diag_pass_t<double>(op, src, dst, n_rows, n_cols, rs.d, cs.d, dg, dh, dc, stream);
+    else
+      launch_diag_pass_t<float>(op, src, dst, n_rows, n_cols, rs.d, cs.d, dg, dh, dc, stream);
+    HIP_CHECK(hipGetLastError());
+    prof_stop(pk, stream);
+  });
+  return true;
+}
+
 // Full spinful orbital rotation (both sectors) on a dim_a x dim_b state.
 // With `then_diag`, the diagonal Coulomb evolution that follows the rotation is
-// fused into the final pass when that pass is a transposing c128 row pass and
-// everything fits; says whether it was (the caller applies it otherwise).  With
+// fused into the final pass when that pass is a transposing row pass and
+// everything fits, or else follows in the same program (a program of its own cost
+// 7 us: norb 12 LUCJ n_reps=4 552 -> 523 us); says whether it was applied (the
+// caller applies it otherwise: no scratch left).  With
 // may_leave_columns (the caller's next gate is a rotation of both sectors) it
 // may leave out the factor of the beta strings alone: the next call then gets
 // the same spec as left_columns.
@@ -1508,44 +1546,28 @@ Fused orbital_rotation_impl(Context& ctx, void* vec, void* work, int dtype, int 
                  stream, launches, want_fuse ? &ft : nullptr, &fused);
     }
   }
+  // a diagonal that no pass took follows in the same program: one upload less
+  const bool columns_left = fused && ft.columns_later;
+  if (then_diag && then_diag->flags && !fused)
+    fused = queue_diag(ctx, prog, DIAG_EVOLVE, vec, vec, dtype, norb, na, nb, *then_diag, stream,
+                       launches);
   prog.commit();
   for (auto& f : launches) f();
   prog.finish();
-  return !fused ? Fused::kNo : ft.columns_later ? Fused::kAllButColumns : Fused::kYes;
+  return !fused ? Fused::kNo : columns_left ? Fused::kAllButColumns : Fused::kYes;
 }
 
 
 void diag_impl(Context& ctx, int op, const void* src, void* dst, int dtype, int norb, int nrow_occ,
                int ncol_occ, const DiagSpec& spec, hipStream_t stream) {
-  const long n_rows = (long)binom(norb, nrow_occ), n_cols = (long)binom(norb, ncol_occ);
-  if (n_rows == 0 || n_cols == 0) return;
-  require(norb <= 63, FFSIM_ERR_VALUE, "norb > 63 unsupported");
-  const DevStrings& rs = dev_strings(ctx, norb, nrow_occ);
-  const DevStrings& cs = dev_strings(ctx, norb, ncol_occ);
+  if (binom(norb, nrow_occ) == 0 || binom(norb, ncol_occ) == 0) return;
   Program prog(ctx, stream);
-  require(spec.norb == norb, FFSIM_ERR_VALUE, "diagonal operator of another norb");
-  const auto [hoff, coff] = append_diag_params(prog, spec);
-  // per column: gamma (contractions) or its phase factor (cos, sin) (evolution)
-  const int evolve = op == DIAG_EVOLVE ? 1 : 0;
-  size_t goff = 0;
-  require(prog.reserve((size_t)n_cols * (evolve ? 2 : 1) * sizeof(double), &goff),
+  std::vector<std::function<void()>> launches;
+  require(queue_diag(ctx, prog, op, src, dst, dtype, norb, nrow_occ, ncol_occ, spec, stream,
+                     launches),
           FFSIM_ERR_VALUE, "diagonal operator: too many columns");
   prog.commit();
-  const DiagHeader* dh = prog.dev<DiagHeader>(hoff);
-  const double* dc = prog.dev<double>(coff);
-  double* dg = prog.scratch<double>(goff);
-  require(diag_grid(n_rows, n_cols).y <= 65535, FFSIM_ERR_VALUE, "too many columns");
-  launch_diag_col_term(n_cols, cs.d, dh, dc, dg, evolve, stream);
-  HIP_CHECK(hipGetLastError());
-  const double moved = (double)elem_bytes(dtype) * (double)n_rows * (double)n_cols *
-                       (op == DIAG_CONTRACT_ACC ? 3.0 : 2.0);
-  const long pk = prof_start(PROF_DIAG, moved, stream);
-  if (dtype == FFSIM_C128)
-    launch_diag_pass_t<double>(op, src, dst, n_rows, n_cols, rs.d, cs.d, dg, dh, dc, stream);
-  else
-    launch_diag_pass_t<float>(op, src, dst, n_rows, n_cols, rs.d, cs.d, dg, dh, dc, stream);
-  HIP_CHECK(hipGetLastError());
-  prof_stop(pk, stream);
+  for (auto& f : launches) f();
   prog.finish();
 }
 
