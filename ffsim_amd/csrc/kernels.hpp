@@ -1065,90 +1065,99 @@ __device__ __forceinline__ uint64_t colex_rank_dev(uint64_t s, const uint64_t* b
   return r;
 }
 
-// Transition one-body RDM of one spin sector, one 4-wave block per string S
-// of the sector (its links dealt round-robin to the waves, so that a small
-// sector still puts several waves on every SIMD): for q in S and p = q or p
-// not in S, T = S - q + p and
-//   part[(p norb + q) 2 + c][S - s_begin] = sign * sum_o conj(lam(T, o)) psi(S, o)
-// (c: re, im) for the strings s_begin <= S < s_begin + n_chunk, where (S, o)
-// addresses row S of an n_str x n_other row-major matrix (COLS = false) or
-// column S of an n_other x n_str one (COLS = true).  The links of S run in a
-// wave-uniform loop, each dot product is reduced across the wave, and every
-// (pair, string) entry is written by exactly one wave, so trdm_reduce_kernel
-// sums them in a fixed order (deterministic results).  part must be zero where
-// S has no link (p, q).
-template <typename T, bool COLS>
+// Transition one-body RDM of one spin sector, its strings on the rows of
+// n_str x n_other matrices lam and psi, from the strings R of one electron less:
+// every pair of orbitals (p, q) that R leaves empty adds
+//   sign_p sign_q sum_o conj(lam(R + p, o)) psi(R + q, o),
+// so R's u = norb - (k - 1) rows of each state give u^2 products, a small
+// matrix product.  A wave forms a 4 x 4 block of them in registers (grid.y:
+// groups of 4 blocks) and reduces its 32 sums across the lanes together, 31
+// exchanges instead of 192.  (p, q) of R - r_begin goes to
+//   part[(p norb + q) 2 + c][R - r_begin]   (c: re, im),
+// which must be zero elsewhere: trdm_reduce_kernel sums it in a fixed order.
+// Bound by reading the rows through L2: a wave's 8 rows serve 16 products,
+// where one row of lam for each product, string by string, read 574 MB at norb
+// 12.  Per launch, complex128: norb 10 18.9 -> 9.7 us, norb 12 33 -> 17 (77 -> 32
+// between the gates of a gradient), norb 13 321 -> 86, norb 14 1566 -> 418, norb
+// 16 with 2 electrons 487 -> 109; complex64 norb 12 75 -> 30.
+constexpr int kMinorTile = 4;
+template <typename T>
 __global__ void __launch_bounds__(256)
-    trdm_links_kernel(const Cx<T>* __restrict__ lam, const Cx<T>* __restrict__ psi, int n_str,
-                      int n_other, int norb, const uint64_t* __restrict__ strings,
-                      const uint64_t* __restrict__ binom_tab, int s_begin, int n_chunk,
-                      double* __restrict__ part) {
+    trdm_minors_kernel(const Cx<T>* __restrict__ lam, const Cx<T>* __restrict__ psi, int n_other,
+                       int norb, const uint64_t* __restrict__ minors,
+                       const uint64_t* __restrict__ binom_tab, long r_begin, int n_chunk,
+                       double* __restrict__ part) {
+  constexpr int M = kMinorTile;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int s_loc = blockIdx.x;
-  const int s_idx = s_begin + s_loc;
-  if (s_loc >= n_chunk || s_idx >= n_str) return;
-  const uint64_t S = strings[s_idx];
+  const int r_loc = blockIdx.x;
+  const uint64_t R = minors[r_begin + r_loc];
+  const uint64_t empty = ~R & ((1ull << norb) - 1);
+  const int u = __popcll(empty), nt = (u + M - 1) / M;
+  const int t = blockIdx.y * 4 + wave;
+  if (t >= nt * nt) return;
   const int stride = norb + 1;
-  auto at = [&](const Cx<T>* m, long str, int o) -> Cx<T> {
-    return COLS ? m[(long)o * n_str + str] : m[str * n_other + o];
-  };
-  // psi's row in registers when it is at most 16 values per lane (row-major
-  // sectors): each link then reads only lam's row
-  constexpr int XR = 16;
-  const bool xreg = !COLS && n_other <= 64 * XR;
-  Cx<T> xr[XR];
+  // the M empty orbitals from the i0-th on (the last one again past the end)
+  int orb[2][M];
+  const Cx<T>* row[2][M];
 #pragma unroll
-  for (int k = 0; k < XR; ++k) {
-    const int o = lane + 64 * k;
-    xr[k] = (xreg && o < n_other) ? psi[(long)s_idx * n_other + o] : Cx<T>{T(0), T(0)};
-  }
-  uint64_t qbits = S;
-  int link = 0;  // the string's links in (q, p) order, dealt round-robin to the 4 waves
-  while (qbits) {
-    const int q = __builtin_ctzll(qbits);
-    qbits &= qbits - 1;
-    const uint64_t S0 = S & ~(1ull << q);
-    const int sign_q = __popcll(S & ((1ull << q) - 1)) & 1;
-    for (int p = 0; p < norb; ++p) {
-      if (p != q && ((S >> p) & 1)) continue;
-      if ((link++ & 3) != wave) continue;
-      const uint64_t S1 = S0 | (1ull << p);
-      const int sign_p = __popcll(S0 & ((1ull << p) - 1)) & 1;
-      const double sgn = ((sign_q ^ sign_p) & 1) ? -1.0 : 1.0;
-      const long t_idx = (long)colex_rank_dev(S1, binom_tab, stride);
-      double re = 0.0, im = 0.0;
-      if (xreg) {
-        // the same terms in the same order as the loop below
+  for (int h = 0; h < 2; ++h) {
+    const int i0 = M * (h == 0 ? t / nt : t % nt);
+    uint64_t e = empty;
+    for (int i = 0; i < i0; ++i) e &= e - 1;
 #pragma unroll
-        for (int k = 0; k < XR; ++k) {
-          const int o = lane + 64 * k;
-          if (o < n_other) {
-            const Cx<T> l = lam[t_idx * n_other + o], x = xr[k];
-            re += (double)l.re * (double)x.re + (double)l.im * (double)x.im;
-            im += (double)l.re * (double)x.im - (double)l.im * (double)x.re;
-          }
-        }
-      } else {
-#pragma unroll 4
-        for (int o = lane; o < n_other; o += 64) {
-          const Cx<T> l = at(lam, t_idx, o), x = at(psi, s_idx, o);
-          // conj(l) * x
-          re += (double)l.re * (double)x.re + (double)l.im * (double)x.im;
-          im += (double)l.re * (double)x.im - (double)l.im * (double)x.re;
-        }
-      }
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) {
-        re += __shfl_xor(re, off);
-        im += __shfl_xor(im, off);
-      }
-      if (lane == 0) {
-        const long e = 2l * (p * norb + q);
-        part[e * n_chunk + s_loc] = sgn * re;
-        part[(e + 1) * n_chunk + s_loc] = sgn * im;
-      }
+    for (int i = 0; i < M; ++i) {
+      const int q = __builtin_ctzll(e);
+      if (e & (e - 1)) e &= e - 1;
+      orb[h][i] = q;
+      row[h][i] = (h == 0 ? lam : psi) +
+                  (long)colex_rank_dev(R | (1ull << q), binom_tab, stride) * n_other;
     }
+  }
+  double acc[2 * M * M];
+#pragma unroll
+  for (int k = 0; k < 2 * M * M; ++k) acc[k] = 0.0;
+  for (int o = lane; o < n_other; o += 64) {
+    Cx<T> l[M], x[M];
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      l[i] = row[0][i][o];
+      x[i] = row[1][i][o];
+    }
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+#pragma unroll
+      for (int j = 0; j < M; ++j) {
+        double& re = acc[2 * (i * M + j)];
+        double& im = acc[2 * (i * M + j) + 1];
+        re += (double)l[i].re * (double)x[j].re + (double)l[i].im * (double)x[j].im;
+        im += (double)l[i].re * (double)x[j].im - (double)l[i].im * (double)x[j].re;
+      }
+  }
+  // lanes exchange halves of their sums: after the step of distance d, lane bit d
+  // tells which half this lane keeps, and sum k of the 32 ends in lanes 2 k, 2 k + 1
+#pragma unroll
+  for (int d = 32, n = M * M; d > 1; d >>= 1, n >>= 1) {
+    const bool up = (lane & d) != 0;
+#pragma unroll
+    for (int k = 0; k < n; ++k) {
+      const double mine = up ? acc[k + n] : acc[k], theirs = up ? acc[k] : acc[k + n];
+      acc[k] = mine + __shfl_xor(theirs, d);
+    }
+  }
+  const double sum = acc[0] + __shfl_xor(acc[0], 1);
+  const int k = lane >> 1, i = k / (2 * M), j = (k >> 1) % M;
+  const int ip = M * (t / nt) + i, jq = M * (t % nt) + j;
+  if ((lane & 1) == 0 && ip < u && jq < u) {
+    int p = orb[0][0], q = orb[1][0];
+#pragma unroll
+    for (int m = 1; m < M; ++m) {
+      if (i == m) p = orb[0][m];
+      if (j == m) q = orb[1][m];
+    }
+    const int sgn = (__popcll(R & ((1ull << p) - 1)) ^ __popcll(R & ((1ull << q) - 1))) & 1;
+    const long e = 2l * (p * norb + q) + (k & 1);
+    part[e * n_chunk + r_loc] = sgn ? -sum : sum;
   }
 }
 
