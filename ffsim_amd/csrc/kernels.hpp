@@ -870,10 +870,6 @@ __global__ void __launch_bounds__(256)
     for (int o = LPR / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, LPR);
     if (l == 0) rho[r] = acc;
   }
-  // the first columns come in while the row factors are formed
-  Col A, B;
-  int c = c_lo + tid;
-  if (c < c_hi) load(c, A);
   __syncthreads();
   if (MODE == DIAG_EVOLVE) {
     // per-orbital factors and row factors, angle = -scale * term
@@ -967,6 +963,9 @@ __global__ void __launch_bounds__(256)
   };
   // two columns per step: B's loads are in flight while A is formed, and A's
   // next loads while B is formed
+  Col A, B;
+  int c = c_lo + tid;
+  if (c < c_hi) load(c, A);
   for (; c < c_hi; c += 2 * NT) {
     load(c + NT, B);
     form(c, A);
