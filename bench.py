@@ -843,7 +843,7 @@ def main() -> int:
     achieved = bytes_per_launch / (avg_ms * 1e-3) / 1e9 if avg_ms > 0 else 0.0
     roofline = {
         "bound": "hbm",
-        "kernel": "fiber_kernel (fused Givens window pass)",
+        "kernel": "fiber_pipe_kernel (fused Givens window pass)",
         "achieved": round(achieved, 1),
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",
@@ -862,7 +862,7 @@ def main() -> int:
     roofline["copy_GBs"] = round(copy_gbs, 1)
     roofline["frac_of_copy"] = round(achieved / copy_gbs, 4)
     log(f"device copy: {copy_gbs:.1f} GB/s")
-    tr = measured_traffic("fiber_kernel", f"lucj_norb{norb}_nreps{args.n_reps}", args.dtype)
+    tr = measured_traffic("fiber_pipe_kernel", f"lucj_norb{norb}_nreps{args.n_reps}", args.dtype)
     if tr is not None:
         roofline["traffic"] = tr["bytes_per_launch"]
         roofline["traffic_source"] = tr["source"]
