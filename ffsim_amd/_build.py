@@ -15,7 +15,8 @@ LIB_PATH = PKG_DIR / "libffsim_amd.so"
 
 SOURCES = ["ffsim_amd.hip", "fiber_pipe_c128.hip", "fiber_pipe_c64.hip", "noalloc.hip",
            "host_core.cpp"]
-HEADERS = ["kernels.hpp", "fiber_pipe.hpp", "host_core.hpp", "status.hpp", "diag_params.hpp"]
+HEADERS = ["kernels.hpp", "pass_rules.hpp", "fiber_pipe.hpp", "host_core.hpp", "status.hpp",
+           "diag_params.hpp"]
 
 
 def hipcc() -> str:

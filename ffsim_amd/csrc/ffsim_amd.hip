@@ -32,6 +32,7 @@
 #include "host_core.hpp"
 #include "fiber_pipe.hpp"
 #include "kernels.hpp"
+#include "pass_rules.hpp"
 #include "status.hpp"
 
 namespace ffsim_amd {
@@ -224,7 +225,8 @@ struct Context {
   std::mutex blas_mu;
   int device = -1;
   size_t lds_max = 65536;
-  int n_cu = 0;
+  int n_cu = 1;
+  PassLimits limits() const { return {lds_max, n_cu}; }
   std::mutex mu;
   std::map<std::pair<int, int>, DevStrings> strings;
   std::map<std::pair<int, int>, DevLinks> links;
@@ -296,8 +298,7 @@ Context& context() {
   hipDeviceProp_t prop;
   HIP_CHECK(hipGetDeviceProperties(&prop, dev));
   ctx->lds_max = prop.sharedMemPerBlock;
-  ctx->n_cu = prop.multiProcessorCount;
-  g_n_cu = std::max(1, prop.multiProcessorCount);
+  ctx->n_cu = g_n_cu = std::max(1, prop.multiProcessorCount);
   for (int k = 0; k < ProgramRing::kSlots; ++k)
     HIP_CHECK(hipEventCreateWithFlags(&ctx->ring.ev[k], hipEventDisableTiming));
   Context& ref = *ctx;
@@ -674,70 +675,6 @@ struct Program {
   }
 };
 
-size_t elem_bytes(int dtype) { return dtype == FFSIM_C64 ? 8 : 16; }
-
-// LDS kept free for the staged program of a pass (sub-passes + steps).
-constexpr size_t kProgramLdsReserve = 20480;
-// LDS kept free beside the tile, row indices and row strings of a window pass.
-constexpr size_t kGroupLdsReserve = 16384;
-
-int tile_width(int dtype) {
-  static int env_w = [] {
-    const char* e = std::getenv("FFSIM_AMD_TILE_W");
-    return e ? std::atoi(e) : 0;
-  }();
-  if (env_w == 4 || env_w == 8 || env_w == 16) return env_w;
-  // c128: 8 columns (128-byte row segments, one tile per CU).  c64: 4 columns,
-  // so that several independent tiles share a CU and one tile's barrier waits
-  // overlap another's work (measured 8% faster than 8 columns, 20% than 16).
-  return dtype == FFSIM_C64 ? 4 : 8;
-}
-
-// The beta rotation runs in place with strings on columns when a whole beta
-// vector fits one tile and its window (all norb orbitals) is no wider than
-// the row-mode window cap, whose group tables the LDS reserve is sized for.
-int window_cap();
-bool beta_in_columns(int norb, long dim_b, int dtype, const Context& ctx) {
-  return norb <= window_cap() &&
-         (size_t)dim_b * (tile_width(dtype) + 1) * elem_bytes(dtype) + kProgramLdsReserve <=
-             ctx.lds_max &&
-         dim_b < 65536;
-}
-
-// Largest fiber of a window of width w for nocc electrons on norb orbitals.
-int max_fiber(int norb, int nocc, int w) {
-  int lo_k = std::max(0, nocc - (norb - w)), hi_k = std::min(nocc, w);
-  uint64_t m = 0;
-  for (int kp = lo_k; kp <= hi_k; ++kp) m = std::max(m, binom(w, kp));
-  return (int)m;
-}
-
-int window_cap() {
-  static int cap = [] {
-    const char* e = std::getenv("FFSIM_AMD_MAX_WINDOW");
-    const int v = e ? std::atoi(e) : 0;
-    return (v >= 2 && v <= 16) ? v : 12;
-  }();
-  return cap;
-}
-
-// Largest window (up to the cap) whose fiber tiles fit in LDS.
-int choose_window(Context& ctx, int norb, int nocc, int dtype) {
-  const int W = tile_width(dtype);
-  // tile row + row index + row string (phase passes); the reserve holds the group
-  // tables, wave schedule and orbital phases
-  const size_t per_row = (size_t)(W + 1) * elem_bytes(dtype) + 4 + (norb <= 32 ? 4 : 8);
-  int best = std::min(norb, 2);
-  for (int w = std::min(norb, window_cap()); w >= 2; --w) {
-    if ((size_t)max_fiber(norb, nocc, w) * per_row + kGroupLdsReserve <= ctx.lds_max) {
-      best = w;
-      break;
-    }
-  }
-  if (norb <= 1) best = std::max(norb, 1);
-  return best;
-}
-
 // LDS of a phase pass beyond the tile: orbital phases and one string per row,
 // and with a fused diagonal the batch columns' factors and the store's tables.
 size_t diag_lds_bytes(bool diag, bool fuse, int n_diag, int rows, int W, int n_fac, int win) {
@@ -802,133 +739,11 @@ void launch_fiber_t(const void* src, void* dst, long ld_src, long ld_dst, int n_
   prof_stop(pk, stream);
 }
 
-// How the passes of a sector with strings on rows run: the window width, and
-// the 16-byte units per string of a pipelined tile (0: plain passes).
-//
-// Up to norb 16, a sector whose strings all fit one tile at some tile width
-// runs as one pass over all orbitals instead of three over 12-orbital windows:
-// a third of the traffic and of the launches, and 8 to 10 register sub-passes
-// instead of 10 to 12, for narrower segments in memory (64, 32 or 16 bytes of
-// a row; neighbouring tiles run on one XCD and share its L2).  Measured per
-// sector rotation, LUCJ: norb=13 (1716 strings, 4 complex128 columns) 160 ->
-// 107 us, norb=14 (3432, 2 columns) 449 -> 281 us, norb=15 (6435, 1 column)
-// 1614 -> 945 us; complex64 153 -> 81, 324 -> 220 and 1080 -> 810 us.
-struct SectorGeom {
-  int w = 0, units = 0, sweeps = 0;
-  int cols = 1;        // columns of a compute lane
-  bool whole = false;  // a tile holds every string of the sector (one pass)
-  bool small = false;  // in place, several states (norb <= 12)
-};
-
-// LDS of a pipelined launch, following the kernel's layout.
-size_t pipe_lds_bytes(const SectorGeom& g, size_t elem, int image_dwords, int variant, int n_fac,
-                      int win) {
-  const int units = g.units;
-  const bool small = variant >= PIPE_SMALL_ROWS;
-  const bool whole = small || units < 8;
-  const bool tstore = variant == PIPE_TRANSPOSE || variant == PIPE_TRANSPOSE_PHASES ||
-                      variant == PIPE_FUSED;
-  const bool dg = variant == PIPE_PHASES || variant == PIPE_TRANSPOSE_PHASES || small;
-  const size_t R = pipe_max_rows(units, g.sweeps), W = pipe_width(units, elem);
-  const size_t slots = whole ? 1 : kPipeSlots;
-  size_t b = (size_t)(g.sweeps + 1) * 4096 + (tstore || whole ? 0 : slots * R * 4) +
-             align16((size_t)image_dwords * 4);
-  if (dg || variant == PIPE_FUSED) b += slots * R * 2;
-  if (dg) b += 68 * sizeof(Cx<double>);
-  if (variant == PIPE_FUSED || small) b += 16;
-  if (variant == PIPE_FUSED)
-    b += (W * n_fac + (size_t)fuse_nibble_entries(win, (int)W)) * sizeof(Cx<double>);
-  return b;
-}
-
-// Geometry of the in-place whole-sector passes of norb 6 to 12 (units 0: none):
-// the least tile that holds the sector's strings.  A tile's time is the chain
-// of its sub-passes (one chunk each of 6-orbital groups: 25 to 40 us at norb
-// 10 to 12), not its width, so the width is chosen for the number of tiles:
-// - 64-byte rows where a sector of norb 12 alone would leave CUs without a
-//   tile (924 x 924 complex128: 231 tiles instead of 116, 50 -> 41 us);
-// - 256-byte rows for sectors of at most 464 strings once 128-byte rows would
-//   give a CU a second tile: half as many tiles, whose chunks are fuller (norb
-//   10: 3 of 5 chunks of 8 groups have no more than half their lanes).  32 states of
-//   norb 10: complex128 81 -> 51 us, complex64 48 -> 33; 8 states of norb 11:
-//   complex128 62 -> 54, complex64 54 -> 36.
-SectorGeom small_geom(int dtype, int norb, int nocc, long n_batch, int n_states) {
-  SectorGeom g;
-  g.w = norb;
-  const size_t elem = elem_bytes(dtype);
-  if (norb < kMaxSubWindow || norb > std::min(window_cap(), 12) || n_batch > (1l << 30) ||
-      tile_width(dtype) != (dtype == FFSIM_C64 ? 4 : 8) || n_batch < (long)(16 / elem))
-    return g;
-  const long rows = (long)binom(norb, nocc);
-  if (rows == 0 || rows > pipe_max_rows(8, 29)) return g;
-  g.whole = g.small = true;
-  g.units = 8;
-  g.sweeps = rows <= pipe_max_rows(8, 8) ? 8 : rows <= pipe_max_rows(8, 15) ? 15 : 29;
-  auto tiles = [&]() {
-    const long w = pipe_width(g.units, elem);
-    return (n_batch + w - 1) / w * n_states;
-  };
-  if (g.sweeps == 29 && tiles() < g_n_cu) {
-    g.units = 4;
-    g.sweeps = 15;
-  } else if (rows <= pipe_max_rows(16, 29) && tiles() > g_n_cu) {
-    g.units = 16;
-    g.sweeps = rows <= pipe_max_rows(16, 16) ? 16 : 29;
-  }
-  if (tiles() > g_n_cu && g.sweeps == 29) g.cols = pipe_cols(g.units, elem);
-  return g;
-}
-int choose_window(Context& ctx, int norb, int nocc, int dtype);
-SectorGeom sector_geom(Context& ctx, int dtype, int norb, int nocc, long n_batch) {
-  SectorGeom g;
-  g.w = choose_window(ctx, norb, nocc, dtype);
-  const size_t elem = elem_bytes(dtype);
-  if (n_batch > (1l << 30) || tile_width(dtype) != (dtype == FFSIM_C64 ? 4 : 8)) return g;
-  if (norb > window_cap() && norb >= kMaxSubWindow && norb <= 16)
-    for (int units : {8, 4, 2, 1})
-      if ((long)binom(norb, nocc) <= pipe_max_rows(units) &&
-          n_batch >= pipe_width(units, elem)) {
-        g.w = norb;
-        g.units = units;
-        g.sweeps = pipe_sweeps(units);
-        g.cols = pipe_cols(units, elem);
-        g.whole = true;
-        return g;
-      }
-  if (g.w >= kMaxSubWindow && g.w <= 16 && n_batch >= pipe_width(8, elem)) {
-    g.units = 8;
-    g.sweeps = pipe_sweeps(8);
-    g.cols = pipe_cols(8, elem);
-  }
-  return g;
-}
-
-// Whether a row pass over these fibers runs pipelined (fiber_pipe_kernel).
-// Whole-sector tiles always do.  For the others, both kernels walk their tiles
-// in rounds over the CUs, one pipelined tile per CU against one plain
-// complex128 tile or three plain complex64 tiles of a quarter of the columns.
-// Measured on the 12-orbital passes of norb 13 to 16: a round takes about 17.6
-// / 21 us (complex128) and 24 / 21.5 us (complex64), and a pipelined launch
-// 16 us more to fill and drain, so it wins from 5 rounds on in complex128 (25
-// rounds: 482 against 538 us per launch; 2 rounds: 58 against 53).  Fibers
-// whose plain tiles leave room for a second workgroup per CU gain nothing from
-// it in complex128 (norb=16 (4,4) in 12-orbital windows, 495 strings: 180
-// against 126 us).
-bool pipe_applies(Context& ctx, int dtype, const SectorGeom& g, const DevWindow& win,
+// Whether a pass over the window's fibers runs pipelined.
+bool pipe_applies(const Context& ctx, int dtype, const SectorGeom& g, const DevWindow& win,
                   bool all_fibers, long n_batch) {
-  if (g.units == 0) return false;
-  if (g.whole) return true;
-  const int rows = all_fibers ? win.max_rows : win.max_rows_active;
-  const long n_f = all_fibers ? win.n_fibers : win.n_active;
-  if (rows > pipe_max_rows(8)) return false;
-  const bool c128 = dtype == FFSIM_C128;
-  if (c128 ? 2 * (size_t)rows * 128 <= ctx.lds_max : rows < 400) return false;
-  auto rounds = [&](int width, long per_cu) {
-    const long tiles = (n_batch + width - 1) / width * n_f;
-    return (double)((tiles + per_cu * g_n_cu - 1) / (per_cu * g_n_cu));
-  };
-  return (c128 ? 17.6 : 24.0) * rounds(pipe_width(8, elem_bytes(dtype)), 1) + 16.0 <
-         (c128 ? 21.0 * rounds(8, 1) : 21.5 * rounds(4, 3));
+  return pipe_applies(ctx.limits(), dtype, g, all_fibers ? win.max_rows : win.max_rows_active,
+                      all_fibers ? win.n_fibers : win.n_active, n_batch);
 }
 
 DevPipe& sector_pipe(Context& ctx, int dtype, int norb, int nocc, const SectorGeom& g) {
@@ -1278,8 +1093,8 @@ void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, l
   if (fused) *fused = false;
   const bool tstore = tstore_dst != nullptr;
   SectorGeom geom;
-  if (!tstore) geom = small_geom(dtype, norb, nocc, n_batch, 1);
-  if (!geom.small && mode == MODE_ROWS) geom = sector_geom(ctx, dtype, norb, nocc, n_batch);
+  if (!tstore) geom = small_geom(ctx.limits(), dtype, norb, nocc, n_batch, 1);
+  if (!geom.small && mode == MODE_ROWS) geom = sector_geom(ctx.limits(), dtype, norb, nocc, n_batch);
   const int w = std::max(1, mode == MODE_COLS ? norb : geom.w);
   std::vector<PlannedPass> passes = plan_passes(rot.steps, norb, w, tstore, -1);
   const DevStrings& ds = dev_strings(ctx, norb, nocc);
@@ -1386,8 +1201,8 @@ enum class Fused { kNo, kYes, kAllButColumns };
 // room for their tables whatever sub-windows a rotation uses.
 bool pipe_fuse_applies(Context& ctx, int dtype, int norb, int na, int nb, int n_fac) {
   const long da = (long)binom(norb, na), db = (long)binom(norb, nb);
-  const SectorGeom ga = sector_geom(ctx, dtype, norb, na, db);
-  const SectorGeom gb = sector_geom(ctx, dtype, norb, nb, da);
+  const SectorGeom ga = sector_geom(ctx.limits(), dtype, norb, na, db);
+  const SectorGeom gb = sector_geom(ctx.limits(), dtype, norb, nb, da);
   if (!pipe_applies(ctx, dtype, ga, dev_window(ctx, norb, na, 0, ga.w), true, db) ||
       !pipe_applies(ctx, dtype, gb, dev_window(ctx, norb, nb, 0, gb.w), true, da))
     return false;
@@ -1463,9 +1278,9 @@ Fused orbital_rotation_impl(Context& ctx, void* vec, void* work, int dtype, int 
   const long dim_a = (long)binom(norb, na), dim_b = (long)binom(norb, nb);
   if (dim_a == 0 || dim_b == 0 || norb == 0) return Fused::kNo;
   require(dim_a < (1l << 31) && dim_b < (1l << 31), FFSIM_ERR_VALUE, "dimension too large");
-  const bool beta_cols = beta_in_columns(norb, dim_b, dtype, ctx);
-  const int w_a = sector_geom(ctx, dtype, norb, na, dim_b).w;
-  const int w_b = beta_cols ? norb : sector_geom(ctx, dtype, norb, nb, dim_a).w;
+  const bool beta_cols = beta_in_columns(norb, dim_b, dtype, ctx.limits());
+  const int w_a = sector_geom(ctx.limits(), dtype, norb, na, dim_b).w;
+  const int w_b = beta_cols ? norb : sector_geom(ctx.limits(), dtype, norb, nb, dim_a).w;
   if (ld_w == 0) ld_w = transposed_ld(dtype, dim_a);
   require(ld_w >= dim_a, FFSIM_ERR_VALUE, "work row pitch below dim_a");
   SectorRotation ra, rb;
@@ -2056,7 +1871,7 @@ void queue_multi_sector(Context& ctx, Program& prog, const MultiSector& ms,
                         size_t states_off, int m, long ld, int n_batch, int norb, int nocc,
                         hipStream_t stream, std::vector<std::function<void()>>& launches) {
   const DevStrings& ds = dev_strings(ctx, norb, nocc);
-  const SectorGeom geom = small_geom(dtype, norb, nocc, n_batch, m);
+  const SectorGeom geom = small_geom(ctx.limits(), dtype, norb, nocc, n_batch, m);
   require(geom.small, FFSIM_ERR_VALUE, "multi-state pass: unsupported shape");
   const size_t diag_off = up.diag_off;
   for (size_t k = 0; k < ms.passes.size(); ++k) {
@@ -2087,8 +1902,8 @@ constexpr int kMultiChunk = 256;
 // whole-sector tiles (norb 6 to 12).
 bool multi_applies(Context& ctx, int dtype, int n, int na, int nb) {
   const long da = (long)binom(n, na), db = (long)binom(n, nb);
-  return beta_in_columns(n, db, dtype, ctx) && small_geom(dtype, n, na, db, 1).small &&
-         small_geom(dtype, n, nb, da, 1).small;
+  return beta_in_columns(n, db, dtype, ctx.limits()) && small_geom(ctx.limits(), dtype, n, na, db, 1).small &&
+         small_geom(ctx.limits(), dtype, n, nb, da, 1).small;
 }
 
 // One orbital rotation per state, planned for multi-state passes.
@@ -2508,7 +2323,7 @@ int64_t ffsim_orbital_rotation_work_elements(int dtype, int norb, int n_alpha, i
     check_sizes(norb, n_alpha, n_beta);
     Context& ctx = context();
     const long dim_a = (long)binom(norb, n_alpha), dim_b = (long)binom(norb, n_beta);
-    const bool beta_cols = beta_in_columns(norb, dim_b, dtype, ctx);
+    const bool beta_cols = beta_in_columns(norb, dim_b, dtype, ctx.limits());
     out = beta_cols ? 0 : (int64_t)transposed_ld(dtype, dim_a) * dim_b;
   });
   return rc == FFSIM_OK ? out : rc;
@@ -3053,7 +2868,7 @@ int ffsim_apply_givens_layer(void* vec, int dtype, int norb, int nocc, int64_t n
     // as independent launches over the same rows.  The window passes apply them
     // in one fused pass; where those cannot run in place (strings on columns
     // with a string vector too long for one tile) each rotation is one launch.
-    const bool fused = strings_on_rows || beta_in_columns(norb, dim, dtype, ctx);
+    const bool fused = strings_on_rows || beta_in_columns(norb, dim, dtype, ctx.limits());
     if (fused) {
       SectorRotation rot;
       for (int r = 0; r < n_rot; ++r) {

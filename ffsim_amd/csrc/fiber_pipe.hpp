@@ -35,36 +35,13 @@
 #pragma once
 
 #include "kernels.hpp"
+#include "pass_rules.hpp"
 
 namespace ffsim_amd {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // a 16-byte access to memory that is only 8-byte aligned (complex64 rows)
 typedef u32x4 u32x4_a8 __attribute__((aligned(8)));
-
-constexpr int kPipeCompute = 8;  // compute waves
-constexpr int kPipeMemory = 4;   // memory waves
-constexpr int kPipeThreads = 64 * (kPipeCompute + kPipeMemory);
-constexpr int kPipeSlots = 3;    // fibers whose rows are in LDS at once
-constexpr int kPipeMaxLo = 11;   // sub-window starts of a 16-orbital window
-
-// Geometry of a tile with `units` 16-byte units per string: 8 for windows of
-// part of the orbitals (128-byte segments), and fewer where that lets a tile
-// hold every string of a sector, whose rotation is then a single pass.
-// A sweep is one 16-byte access of every memory lane.
-constexpr int pipe_step(int units) { return 64 * kPipeMemory / units; }  // strings per sweep
-constexpr int pipe_sweeps(int units) { return units == 8 ? 29 : units == 1 ? 26 : 27; }
-constexpr int pipe_max_rows(int units, int sweeps) { return pipe_step(units) * sweeps; }
-constexpr int pipe_max_rows(int units) { return pipe_max_rows(units, pipe_sweeps(units)); }
-constexpr int pipe_width(int units, size_t elem) { return units * 16 / (int)elem; }
-// Columns that a compute lane rotates together: complex64 passes with several
-// tiles per CU take both columns of a 16-byte unit, which halves the LDS
-// instructions, address and coefficient work of a rotation (norb 16 1.19 ->
-// 1.12 ms a launch, norb 15 0.79 -> 0.65, norb 14 0.197 -> 0.174).  A launch of
-// one tile per CU waits for one chunk's chain of instructions, which that doubles
-// (norb 12 39 -> 48 us, norb 13 69 -> 71): one column there, and for sectors of
-// at most 256 strings (64 states of norb 10: 58 us against 69).
-constexpr int pipe_cols(int units, size_t elem) { return units == 4 ? 1 : 16 / (int)elem; }
 
 // Tables of a pipelined pass: one image per electron count kp of the window,
 // laid out as the workgroup keeps it in LDS (dword offsets): PipeSlot per
@@ -632,8 +609,6 @@ __global__ void __launch_bounds__(kPipeThreads)
 
 // Kernel of a tile geometry and variant (the launching code and the
 // instantiations of each type are compiled apart).
-enum { PIPE_PLAIN = 0, PIPE_PHASES = 1, PIPE_TRANSPOSE = 2, PIPE_TRANSPOSE_PHASES = 3, PIPE_FUSED = 4,
-       PIPE_SMALL_ROWS = 5, PIPE_SMALL_COLS = 6, PIPE_VARIANTS = 7 };
 template <typename T, int UNITS, int NC>
 const void* pipe_kernel_units(int variant) {
   constexpr int S = pipe_sweeps(UNITS);

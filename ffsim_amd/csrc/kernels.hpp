@@ -19,6 +19,7 @@
 #include <stdint.h>
 
 #include "host_core.hpp"
+#include "pass_rules.hpp"
 
 namespace ffsim_amd {
 
@@ -294,8 +295,6 @@ struct GroupSlot {
   int pad[2];
 };
 
-__host__ __device__ constexpr size_t align16(size_t x) { return (x + 15) & ~size_t(15); }
-
 // A diagonal Coulomb evolution fused into the store of a transposing pass
 // (the last pass of the second sector's rotation).  Element (tile string i,
 // batch string j) is multiplied by exp(-i t E) formed from complex FP64
@@ -307,13 +306,6 @@ struct DiagFuse {
   int n_fac;               // norb + 1 (at most 64)
   int win;                 // the pass's window is orbitals [0, win), win <= 16
 };
-// LDS of the fused store's per-tile tables: for every 4-orbital nibble t of the
-// window and every occupation pattern p of it, the product of the batch
-// columns' factors over p; then one factor per column for the batch term and
-// the fiber's orbitals outside the window (the same for every tile string).
-__host__ __device__ constexpr int fuse_nibble_entries(int win, int W) {
-  return (((win + 3) >> 2) * 16 + 1) * W;
-}
 
 // Element (string i, batch j) of a fiber tile lives at
 //   MODE_ROWS: state[row_table[i] * ld + b0 + j]   (strings index rows)
