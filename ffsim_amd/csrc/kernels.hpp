@@ -439,7 +439,10 @@ __global__ void __launch_bounds__(NTHR)
   // and waiting for those (vmcnt) would also drain the stores in flight.
   // All row addresses are read first and the element loads issued after them, so
   // the global-table case waits once for its addresses instead of once per row.
-  auto load_regs = [&](Cx<T>* buf, int nr, int b0, int nb, const int32_t* rt) {
+  // (sp: src by value.  Read through the closure, the address is added up again for
+  // every element: 170 64-bit adds instead of 110 and 18 more reloads of spilled
+  // scalars in the complex128 kernel, 2-3% of a launch.)
+  auto load_regs = [&](Cx<T>* buf, int nr, int b0, int nb, const int32_t* rt, const Cx<T>* sp) {
     int ra[CH];
     if (MODE == MODE_ROWS) {
       const int j = tid % W, i0 = tid / W;
@@ -451,7 +454,7 @@ __global__ void __launch_bounds__(NTHR)
 #pragma unroll
       for (int k = 0; k < CH; ++k) {
         buf[k] = Cx<T>{T(0), T(0)};
-        if (ra[k] >= 0) buf[k] = src[(long)ra[k] * ld_src + b0 + j];
+        if (ra[k] >= 0) buf[k] = sp[(long)ra[k] * ld_src + b0 + j];
       }
     } else {
 #pragma unroll
@@ -463,7 +466,7 @@ __global__ void __launch_bounds__(NTHR)
       for (int k = 0; k < CH; ++k) {
         const int j = k % W;
         buf[k] = Cx<T>{T(0), T(0)};
-        if (ra[k] >= 0) buf[k] = src[(long)(b0 + j) * ld_src + ra[k]];
+        if (ra[k] >= 0) buf[k] = sp[(long)(b0 + j) * ld_src + ra[k]];
       }
     }
   };
@@ -670,9 +673,9 @@ __global__ void __launch_bounds__(NTHR)
     // around the loop: a loop-carried buf makes the compiler copy it at the back
     // edge behind a vmcnt(0) that would also drain this tile's stores
     if (same_fiber)
-      load_regs(buf, nrn, b0n, nbn, rows);
+      load_regs(buf, nrn, b0n, nbn, rows, src);
     else
-      load_regs(buf, nrn, b0n, nbn, row_table + fdn.row_off);
+      load_regs(buf, nrn, b0n, nbn, row_table + fdn.row_off, src);
     if (FUSE) bfn = load_bfac(b0n);
 
     // ---- register sub-passes on the current tile
