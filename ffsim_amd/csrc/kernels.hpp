@@ -439,9 +439,10 @@ __global__ void __launch_bounds__(NTHR)
   // and waiting for those (vmcnt) would also drain the stores in flight.
   // All row addresses are read first and the element loads issued after them, so
   // the global-table case waits once for its addresses instead of once per row.
-  // (sp: src by value.  Read through the closure, the address is added up again for
-  // every element: 170 64-bit adds instead of 110 and 18 more reloads of spilled
-  // scalars in the complex128 kernel, 2-3% of a launch.)
+  // (complex128 takes the state's address by value, sp: read through the closure, it
+  // is added up again for every element, 170 64-bit adds instead of 110 and 18 more
+  // reloads of spilled scalars, 2.4-2.9% of a launch (norb 20 with (8, 1) electrons
+  // 2219 against 2281 us).  complex64 is the other way round, 2746 against 2795.)
   auto load_regs = [&](Cx<T>* buf, int nr, int b0, int nb, const int32_t* rt, const Cx<T>* sp) {
     int ra[CH];
     if (MODE == MODE_ROWS) {
@@ -454,7 +455,7 @@ __global__ void __launch_bounds__(NTHR)
 #pragma unroll
       for (int k = 0; k < CH; ++k) {
         buf[k] = Cx<T>{T(0), T(0)};
-        if (ra[k] >= 0) buf[k] = sp[(long)ra[k] * ld_src + b0 + j];
+        if (ra[k] >= 0) buf[k] = (sizeof(T) == 8 ? sp : src)[(long)ra[k] * ld_src + b0 + j];
       }
     } else {
 #pragma unroll
