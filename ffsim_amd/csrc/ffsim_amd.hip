@@ -2704,22 +2704,18 @@ int ffsim_transition_rdm(const void* lam, const void* psi, int dtype, int norb, 
       for (int t = 0; t <= norb; ++t) tab[(size_t)c * (norb + 1) + t] = binom(c, t);
     const size_t toff = prog.append(tab.data(), tab.size() * sizeof(uint64_t));
     // per-(pair, minor) dot products of a chunk of minors, then the transposes of
-    // a slab of lam's and psi's rows for the beta sector, whose strings then
-    // index rows as the alpha sector's do: all rows if they take no more than
-    // kTrdmSlabBytes (norb 13), else as many as fit, their sums added up
-    // (norb 14: 4 slabs, 19.6 -> 1.4 ms against strings read along columns)
+    // the beta sector's slabs (see trdm_beta_layout)
     const long n2 = 2l * norb * norb;
     const long n_str_max = std::max(da, db);
     const long chunk = std::min<long>(n_str_max, std::max<long>(4, (64l << 20) / (n2 * 8)));
     size_t poff = 0;
     require(prog.reserve((size_t)(n2 * chunk * 8), &poff), FFSIM_ERR_VALUE,
             "transition RDM: scratch too large");
-    constexpr long kTrdmSlabBytes = 96l << 20;
-    long slab = std::min<long>(da, kTrdmSlabBytes / (2 * db * (long)elem_bytes(dtype)));
-    if (slab < da && slab > 64) slab -= slab % 64;
-    // (a single row is its own transpose)
+    TrdmBeta lay = trdm_beta_layout(dtype, da, db, n_beta);
     size_t tpoff = 0;
-    if (slab < 2 || !prog.reserve((size_t)(2 * slab * db) * elem_bytes(dtype), &tpoff)) slab = 1;
+    if (lay.form == TrdmBeta::kSlabs &&
+        !prog.reserve((size_t)(2 * lay.slab * db) * elem_bytes(dtype), &tpoff))
+      lay.form = TrdmBeta::kColumns;
     prog.commit();
     double* part = prog.scratch<double>(poff);
     const uint64_t* dtab = prog.dev<uint64_t>(toff);
@@ -2727,8 +2723,9 @@ int ffsim_transition_rdm(const void* lam, const void* psi, int dtype, int norb, 
       using T = decltype(tag);
       const Cx<T>* L = (const Cx<T>*)lam;
       const Cx<T>* P = (const Cx<T>*)psi;
-      // one sector, its strings on rows
-      auto sector = [&](const Cx<T>* l, const Cx<T>* x, int nocc, long n_other, double* rdm) {
+      // one sector, its strings on rows (or on columns, rows ld apart)
+      auto sector = [&](const Cx<T>* l, const Cx<T>* x, int nocc, long n_other, bool cols, long ld,
+                        double* rdm) {
         if (nocc == 0) return;
         const long tiles = (norb - nocc + kMinorTile) / kMinorTile;
         const long n_minor = (long)binom(norb, nocc - 1);
@@ -2739,27 +2736,34 @@ int ffsim_transition_rdm(const void* lam, const void* psi, int dtype, int norb, 
           hipLaunchKernelGGL(fill_zero_kernel,
                              dim3((unsigned)std::min<long>((nz + 255) / 256, 65536)), dim3(256), 0,
                              st, part, nz);
-          hipLaunchKernelGGL(trdm_minors_kernel<T>,
-                             dim3((unsigned)cnt, (unsigned)((tiles * tiles + 3) / 4)), dim3(256),
-                             0, st, l, x, (int)n_other, norb, minors.d, dtab, r0, (int)cnt, part);
+          const dim3 grid((unsigned)cnt, (unsigned)((tiles * tiles + 3) / 4));
+          if (cols)
+            hipLaunchKernelGGL((trdm_minors_kernel<T, true>), grid, dim3(256), 0, st, l, x,
+                               (int)n_other, ld, norb, minors.d, dtab, r0, (int)cnt, part);
+          else
+            hipLaunchKernelGGL((trdm_minors_kernel<T, false>), grid, dim3(256), 0, st, l, x,
+                               (int)n_other, ld, norb, minors.d, dtab, r0, (int)cnt, part);
           hipLaunchKernelGGL(trdm_reduce_kernel, dim3((unsigned)n2), dim3(256), 0, st, part,
                              (int)cnt, rdm);
         }
       };
-      sector(L, P, n_alpha, db, out);
-      for (long o0 = 0; o0 < da; o0 += slab) {
-        const long cnt = std::min(slab, da - o0);
-        const Cx<T>*lt = L + o0 * db, *pt = P + o0 * db;
-        if (slab > 1) {
-          Cx<T>* t = prog.scratch<Cx<T>>(tpoff);
+      sector(L, P, n_alpha, db, false, 0, out);
+      if (lay.form == TrdmBeta::kAsRows) {
+        sector(L, P, n_beta, da, false, 0, out + n2);
+      } else if (lay.form == TrdmBeta::kColumns) {
+        sector(L, P, n_beta, da, true, db, out + n2);
+      } else if (lay.form == TrdmBeta::kSlabs) {
+        for (long o0 = 0; o0 < da; o0 += lay.slab) {
+          const long cnt = std::min(lay.slab, da - o0);
+          Cx<T>* lt = prog.scratch<Cx<T>>(tpoff);
+          Cx<T>* pt = lt + cnt * db;
           const dim3 tg((unsigned)((db + 31) / 32), (unsigned)((cnt + 31) / 32));
-          hipLaunchKernelGGL(transpose_kernel<T>, tg, dim3(256), 0, st, lt, t, (int)cnt, (int)db);
-          hipLaunchKernelGGL(transpose_kernel<T>, tg, dim3(256), 0, st, pt, t + cnt * db, (int)cnt,
+          hipLaunchKernelGGL(transpose_kernel<T>, tg, dim3(256), 0, st, L + o0 * db, lt, (int)cnt,
                              (int)db);
-          lt = t;
-          pt = t + cnt * db;
+          hipLaunchKernelGGL(transpose_kernel<T>, tg, dim3(256), 0, st, P + o0 * db, pt, (int)cnt,
+                             (int)db);
+          sector(lt, pt, n_beta, cnt, false, 0, out + n2);
         }
-        sector(lt, pt, n_beta, cnt, out + n2);
       }
     };
     if (dtype == FFSIM_C128)

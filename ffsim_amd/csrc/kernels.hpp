@@ -1061,12 +1061,13 @@ __device__ __forceinline__ uint64_t colex_rank_dev(uint64_t s, const uint64_t* b
 }
 
 // Transition one-body RDM of one spin sector, its strings on the rows of
-// n_str x n_other matrices lam and psi, from the strings R of one electron less:
+// n_str x n_other matrices lam and psi (COLS: on the columns of n_other x n_str
+// ones, their rows ld apart), from the strings R of one electron less:
 // every pair of orbitals (p, q) that R leaves empty adds
 //   sign_p sign_q sum_o conj(lam(R + p, o)) psi(R + q, o),
 // so R's u = norb - (k - 1) rows of each state give u^2 products, a small
 // matrix product.  A wave forms a 4 x 4 block of them in registers (grid.y:
-// groups of 4 blocks) and reduces its 32 sums across the lanes together, 31
+// groups of 4 blocks) and reduces its 32 sums across the lanes together, 32
 // exchanges instead of 192.  (p, q) of R - r_begin goes to
 //   part[(p norb + q) 2 + c][R - r_begin]   (c: re, im),
 // which must be zero elsewhere: trdm_reduce_kernel sums it in a fixed order.
@@ -1076,10 +1077,10 @@ __device__ __forceinline__ uint64_t colex_rank_dev(uint64_t s, const uint64_t* b
 // between the gates of a gradient), norb 13 321 -> 86, norb 14 1566 -> 418, norb
 // 16 with 2 electrons 487 -> 109; complex64 norb 12 75 -> 30.
 constexpr int kMinorTile = 4;
-template <typename T>
+template <typename T, bool COLS>
 __global__ void __launch_bounds__(256)
     trdm_minors_kernel(const Cx<T>* __restrict__ lam, const Cx<T>* __restrict__ psi, int n_other,
-                       int norb, const uint64_t* __restrict__ minors,
+                       long ld, int norb, const uint64_t* __restrict__ minors,
                        const uint64_t* __restrict__ binom_tab, long r_begin, int n_chunk,
                        double* __restrict__ part) {
   constexpr int M = kMinorTile;
@@ -1106,7 +1107,7 @@ __global__ void __launch_bounds__(256)
       if (e & (e - 1)) e &= e - 1;
       orb[h][i] = q;
       row[h][i] = (h == 0 ? lam : psi) +
-                  (long)colex_rank_dev(R | (1ull << q), binom_tab, stride) * n_other;
+                  (long)colex_rank_dev(R | (1ull << q), binom_tab, stride) * (COLS ? 1 : n_other);
     }
   }
   double acc[2 * M * M];
@@ -1116,8 +1117,8 @@ __global__ void __launch_bounds__(256)
     Cx<T> l[M], x[M];
 #pragma unroll
     for (int i = 0; i < M; ++i) {
-      l[i] = row[0][i][o];
-      x[i] = row[1][i][o];
+      l[i] = row[0][i][COLS ? o * ld : o];
+      x[i] = row[1][i][COLS ? o * ld : o];
     }
 #pragma unroll
     for (int i = 0; i < M; ++i)

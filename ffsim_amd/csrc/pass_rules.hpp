@@ -248,4 +248,41 @@ inline bool pipe_applies(const PassLimits& lim, int dtype, const SectorGeom& g, 
          (c128 ? 21.0 * rounds(8, 1) : 21.5 * rounds(4, 3));
 }
 
+// -------------------------------------------------------- transition RDM
+// How the beta sector of a transition RDM reads lam and psi (da x db, its
+// strings on columns): as they lie where one dimension is 1 (a row or a column
+// is its own transpose); in transposed slabs of rows, whose strings then index
+// rows as the alpha sector's do, all rows if their transposes take no more than
+// kTrdmSlabBytes (norb 13), else as many as fit, their sums added up (norb 14:
+// 4.3 ms along columns, 1.1 in 4 slabs); or along the columns in place, where a
+// slab would have fewer rows than a wave has lanes: few rows of many columns,
+// for each of which all slabs would be gone through.  Columns against slabs,
+// complex128: norb 24 with (1, 8) electrons 32 and 153 ms (slabs of 4 rows), (1, 12)
+// 178 and 3591 (1 row), norb 20 (2, 9) 18 and 43 (18 of 190 rows), (2, 7) 7.6 and
+// 9.0 (40); the other way round norb 18 (3, 9) 24.7 and 18.3 (64 of 816).
+struct TrdmBeta {
+  enum Form { kNone, kAsRows, kSlabs, kColumns } form = kNone;
+  long slab = 0;
+};
+constexpr long kTrdmSlabBytes = 96l << 20;
+constexpr long kTrdmMinSlab = 64;
+inline TrdmBeta trdm_beta_layout(int dtype, long da, long db, int n_beta) {
+  TrdmBeta r;
+  if (n_beta == 0 || da == 0 || db == 0) return r;
+  if (da == 1 || db == 1) {
+    r.form = TrdmBeta::kAsRows;
+    return r;
+  }
+  r.slab = std::min<long>(da, kTrdmSlabBytes / (2 * db * (long)elem_bytes(dtype)));
+  if (r.slab < da && r.slab < kTrdmMinSlab) {
+    r.form = TrdmBeta::kColumns;
+    return r;
+  }
+  // (grid.y of the transposition: 32 rows each)
+  r.slab = std::min(r.slab, 32l * 65535);
+  if (r.slab < da && r.slab > 64) r.slab -= r.slab % 64;
+  r.form = TrdmBeta::kSlabs;
+  return r;
+}
+
 }  // namespace ffsim_amd

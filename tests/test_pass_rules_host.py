@@ -1,0 +1,50 @@
+"""Rules on pass geometry (ffsim_amd/csrc/pass_rules.hpp), evaluated on the CPU."""
+
+import ctypes
+import subprocess
+from math import comb
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+C128, C64 = 0, 1
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    out = tmp_path_factory.mktemp("rules") / "pass_rules.so"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC",
+                    str(ROOT / "tests/native/pass_rules_check.cpp"),
+                    str(ROOT / "ffsim_amd/csrc/host_core.cpp"), "-o", str(out)], check=True)
+    return ctypes.CDLL(str(out))
+
+
+NONE, AS_ROWS, SLABS, COLUMNS = range(4)
+
+
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize("norb,nelec,form", [
+    (12, (6, 6), SLABS), (14, (7, 6), SLABS), (16, (8, 8), SLABS), (18, (9, 9), SLABS),
+    (20, (5, 1), SLABS),
+    # no electrons to reduce over: nothing is transposed
+    (16, (8, 0), NONE), (24, (12, 0), NONE),
+    # one row or one column is its own transpose
+    (24, (12, 24), AS_ROWS), (24, (0, 12), AS_ROWS), (1, (1, 1), AS_ROWS),
+    # few rows of very many columns
+    (24, (1, 8), COLUMNS), (24, (1, 12), COLUMNS), (22, (2, 9), COLUMNS), (20, (2, 7), None),
+])
+def test_transition_rdm_layout(rules, dtype, norb, nelec, form):
+    da, db = (comb(norb, n) for n in nelec)
+    slab = ctypes.c_long()
+    got = rules.trdm_layout(dtype, ctypes.c_long(da), ctypes.c_long(db), nelec[1],
+                            ctypes.byref(slab))
+    if form is not None:
+        assert got == form
+    if got == SLABS:
+        elem = 16 if dtype == C128 else 8
+        assert 1 <= slab.value <= da
+        assert 2 * slab.value * db * elem <= 96 << 20
+        # 64 lanes of a dot product have work, and the transposition's grid fits
+        assert slab.value == da or slab.value >= 64
+        assert (slab.value + 31) // 32 <= 65535
