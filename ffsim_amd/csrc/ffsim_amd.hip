@@ -806,7 +806,8 @@ void pipe_pass(int dtype, const SectorGeom& g, PipeLaunch L, const DevWindow& wi
   const bool dg = !fuse && L.diag != nullptr;
   const bool whole = L.small || units < 8;
   int rows = L.all_fibers ? win.max_rows : win.max_rows_active;
-  require(L.n_batch >= (L.small ? (int)(16 / elem) : W) && rows <= pipe_max_rows(units, g.sweeps),
+  require(L.n_batch >= (L.cols ? 1 : L.small ? (int)(16 / elem) : W) &&
+              rows <= pipe_max_rows(units, g.sweeps),
           FFSIM_ERR_VALUE, "pipelined pass: shape");
   require((!L.tstore && !whole) || (win.lo == 0 && (!whole || win.n_fibers == 1)),
           FFSIM_ERR_VALUE, "pipelined pass: rows not contiguous");
@@ -1096,6 +1097,7 @@ void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, l
   if (!tstore) geom = small_geom(ctx.limits(), dtype, norb, nocc, n_batch, 1);
   if (!geom.small && mode == MODE_ROWS) geom = sector_geom(ctx.limits(), dtype, norb, nocc, n_batch);
   const int w = std::max(1, mode == MODE_COLS ? norb : geom.w);
+  const bool cols = geom.small && small_in_columns(dtype, mode == MODE_COLS, n_batch);
   std::vector<PlannedPass> passes = plan_passes(rot.steps, norb, w, tstore, -1);
   const DevStrings& ds = dev_strings(ctx, norb, nocc);
   const bool need_diag = !rot.trivial_diag;
@@ -1142,7 +1144,7 @@ void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, l
         PipeLaunch L{state, dst, ld, ld_dst, n_batch, ts, all, prog.dev<SubPass>(poff), n_sub,
                      prog.dev<LayerPair>(soff), n_layers, ph ? prog.dev<double>(doff) : nullptr,
                      ds.d, cf ? prog.scratch<Cx<double>>(coff) : nullptr, PipeFuse{nullptr, 0},
-                     geom.small, mode == MODE_COLS, PipeStates{nullptr, 1, 0, 0}};
+                     geom.small, cols, PipeStates{nullptr, 1, 0, 0}};
         if (fz_pipe) L.fz = PipeFuse{prog.scratch<Cx<double>>(fp.bfac_off), fp.n_fac};
         PipeTables tb = tb0;
         if (!tb.image) tb.image = prog.dev<uint32_t>(img_off);
@@ -1886,7 +1888,8 @@ void queue_multi_sector(Context& ctx, Program& prog, const MultiSector& ms,
     launches.push_back([=, &ctx, &prog, &win, &ds]() {
       PipeLaunch L{nullptr, nullptr, ld, ld, n_batch, false, dg, prog.dev<SubPass>(poff), n_sub,
                    prog.dev<LayerPair>(soff), n_layers, dg ? prog.dev<double>(diag_off) : nullptr,
-                   ds.d, nullptr, PipeFuse{nullptr, 0}, true, mode == MODE_COLS,
+                   ds.d, nullptr, PipeFuse{nullptr, 0}, true,
+                   small_in_columns(dtype, mode == MODE_COLS, n_batch),
                    PipeStates{prog.dev<void*>(states_off), m, (long)n_layers, 2l * norb}};
       PipeTables tb = tb0;
       if (!tb.image) tb.image = prog.dev<uint32_t>(img_off);

@@ -381,7 +381,11 @@ __global__ void __launch_bounds__(kPipeThreads)
   // first column of this thread's unit in the tile at column b0 (units that
   // reach past the last column are moved back: they then hold columns that
   // another unit stores, and the store skips those)
-  auto unit_col = [&](int b0) { return min(b0 + u * EU, n_batch - EU); };
+  // (a single complex64 column: strings on columns, both halves of a unit hold it)
+  auto unit_col = [&](int b0) {
+    const int c = min(b0 + u * EU, n_batch - EU);
+    return COLS && EU > 1 ? max(c, 0) : c;
+  };
   // register k holds sweep k of its tile, or sweep 28 - k (see exchange): string
   // first + k step.  Transposing passes work on contiguous rows (window [0, w)).
   auto load = [&](auto k0c, auto k1c, const Cx<T>* base, int first, int step, int slot, int nr,
@@ -395,11 +399,12 @@ __global__ void __launch_bounds__(kPipeThreads)
                            : (uint32_t)rslot[slot * R + first + k * step];
     if constexpr (COLS) {
       const Cx<T>* p = base + (uint64_t)(uint32_t)unit_col(b0) * (uint32_t)ld_src;
+      const uint32_t ldz = n_batch < EU ? 0 : (uint32_t)ld_src;
 #pragma unroll
       for (int k = K0; k < K1; ++k) {
         Cx<T> e[EU];
 #pragma unroll
-        for (int z = 0; z < EU; ++z) e[z] = p[(uint64_t)z * (uint32_t)ld_src + row[k - K0]];
+        for (int z = 0; z < EU; ++z) e[z] = p[(uint64_t)z * ldz + row[k - K0]];
         __builtin_memcpy(&buf[k], e, 16);
       }
     } else {
@@ -455,7 +460,8 @@ __global__ void __launch_bounds__(kPipeThreads)
         if constexpr (TST || COLS) {
 #pragma unroll
           for (int z = 0; z < EU; ++z)
-            if (full || z >= skip) base[(uint64_t)(uint32_t)(c0 + z) * (uint32_t)ld_dst + row] = e[z];
+            if (full || (z >= skip && (!COLS || z < n_batch)))
+              base[(uint64_t)(uint32_t)(c0 + z) * (uint32_t)ld_dst + row] = e[z];
         } else {
           Cx<T>* p = base + c0 + (uint64_t)row * (uint32_t)ld_dst;
           if (full || skip == 0) {

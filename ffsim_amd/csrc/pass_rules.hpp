@@ -169,13 +169,15 @@ inline size_t pipe_lds_bytes(const SectorGeom& g, size_t elem, int image_dwords,
 //   10: 3 of 5 chunks of 8 groups have no more than half their lanes).  32 states of
 //   norb 10: complex128 81 -> 51 us, complex64 48 -> 33; 8 states of norb 11:
 //   complex128 62 -> 54, complex64 54 -> 36.
+// A single column (the other sector empty or full) runs with strings on columns
+// (small_in_columns).
 inline SectorGeom small_geom(const PassLimits& lim, int dtype, int norb, int nocc, long n_batch,
                              int n_states) {
   SectorGeom g;
   g.w = norb;
   const size_t elem = elem_bytes(dtype);
   if (norb < kMaxSubWindow || norb > std::min(window_cap(), 12) || n_batch > (1l << 30) ||
-      tile_width(dtype) != (dtype == FFSIM_C64 ? 4 : 8) || n_batch < (long)(16 / elem))
+      tile_width(dtype) != (dtype == FFSIM_C64 ? 4 : 8))
     return g;
   const long rows = (long)binom(norb, nocc);
   if (rows == 0 || rows > pipe_max_rows(8, 29)) return g;
@@ -195,6 +197,13 @@ inline SectorGeom small_geom(const PassLimits& lim, int dtype, int norb, int noc
   }
   if (tiles() > lim.n_cu && g.sweeps == 29) g.cols = pipe_cols(g.units, elem);
   return g;
+}
+
+// Whether an in-place whole-sector pass takes its strings to be on columns.  One
+// column is contiguous either way; with strings on rows a unit of two complex64
+// columns would reach past it.
+inline bool small_in_columns(int dtype, bool strings_on_columns, long n_batch) {
+  return strings_on_columns || n_batch < (long)(16 / elem_bytes(dtype));
 }
 
 inline SectorGeom sector_geom(const PassLimits& lim, int dtype, int norb, int nocc, long n_batch) {

@@ -11,3 +11,14 @@ extern "C" int trdm_layout(int dtype, long da, long db, int n_beta, long* slab) 
   *slab = r.slab;
   return (int)r.form;
 }
+
+// In-place whole-sector passes: 16-byte units per string (0: no such pass), strings
+// taken to be on columns or not, sweeps, columns a lane.
+extern "C" void small_pass(int dtype, int norb, int nocc, long n_batch, int n_states,
+                           int on_columns, int* out) {
+  const SectorGeom g = small_geom(kLim, dtype, norb, nocc, n_batch, n_states);
+  out[0] = g.small ? g.units : 0;
+  out[1] = small_in_columns(dtype, on_columns != 0, n_batch);
+  out[2] = g.sweeps;
+  out[3] = g.cols;
+}

@@ -48,3 +48,23 @@ def test_transition_rdm_layout(rules, dtype, norb, nelec, form):
         # 64 lanes of a dot product have work, and the transposition's grid fits
         assert slab.value == da or slab.value >= 64
         assert (slab.value + 31) // 32 <= 65535
+
+
+def _small(rules, dtype, norb, nocc, n_batch, n_states=1, on_columns=0):
+    out = (ctypes.c_int * 4)()
+    rules.small_pass(dtype, norb, nocc, ctypes.c_long(n_batch), n_states, on_columns, out)
+    return out
+
+
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize("norb", range(6, 13))
+def test_every_sector_up_to_norb_12_runs_in_place(rules, dtype, norb):
+    """Whatever the other sector: empty and full ones leave a single column."""
+    for nocc in range(norb + 1):
+        for other in range(norb + 1):
+            n_batch = comb(norb, other)
+            for on_columns in (0, 1):
+                units, cols, sweeps, _ = _small(rules, dtype, norb, nocc, n_batch, 2, on_columns)
+                assert units and 256 // units * sweeps >= comb(norb, nocc)
+                # with strings on rows a 16-byte unit must not reach past the columns
+                assert cols or n_batch >= (1 if dtype == C128 else 2)
