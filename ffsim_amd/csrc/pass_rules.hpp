@@ -158,19 +158,26 @@ inline size_t pipe_lds_bytes(const SectorGeom& g, size_t elem, int image_dwords,
   return b;
 }
 
-// Geometry of the in-place whole-sector passes of norb 6 to 12 (units 0: none):
-// the least tile that holds the sector's strings.  A tile's time is the chain
-// of its sub-passes (one chunk each of 6-orbital groups: 25 to 40 us at norb
-// 10 to 12), not its width, so the width is chosen for the number of tiles:
-// - 64-byte rows where a sector of norb 12 alone would leave CUs without a
-//   tile (924 x 924 complex128: 231 tiles instead of 116, 50 -> 41 us);
-// - 256-byte rows for sectors of at most 464 strings once 128-byte rows would
-//   give a CU a second tile: half as many tiles, whose chunks are fuller (norb
-//   10: 3 of 5 chunks of 8 groups have no more than half their lanes).  32 states of
-//   norb 10: complex128 81 -> 51 us, complex64 48 -> 33; 8 states of norb 11:
-//   complex128 62 -> 54, complex64 54 -> 36.
+// Geometry of the in-place whole-sector passes of norb 6 to 12 (units 0: none),
+// from the tiles that hold the sector's strings.  A tile's time is the chain of
+// its sub-passes, one chunk each of 6-orbital groups, which a wider tile makes
+// longer; a launch takes rounds of one tile per CU.  So the form is the one whose
+// rounds take the least time.  SmallForm::first and ::more are the microseconds of
+// a launch's first round and of each further one, measured at the largest sectors
+// of each class (924 and 792, 495, 462, 252 strings; 1 to 64 states), where the
+// least sum is the fastest form for every count, or within 5% of it.  Examples,
+// us a launch, narrow against wide rows: norb 12 (6, 6) complex128 one state 42
+// and 50, two states 65 and 54; complex64 two states 42 and 61, three 68 and 64,
+// five 91 and 99, eight 118 and 102; norb 11 (5, 5) complex64 four states 32 and 37
+// (and 53 for 256-byte rows), ten 74, 60 and 57, 24 135, 88 and 91.
+// A lane takes both complex64 columns of a unit where that is the faster form of a
+// wide tile: 32 states of norb 12 (6, 6) 313 against 366 us, (4, 4) 159 against 141.
 // A single column (the other sector empty or full) runs with strings on columns
 // (small_in_columns).
+struct SmallForm {
+  int units, sweeps, cols;
+  double first, more;
+};
 inline SectorGeom small_geom(const PassLimits& lim, int dtype, int norb, int nocc, long n_batch,
                              int n_states) {
   SectorGeom g;
@@ -181,21 +188,31 @@ inline SectorGeom small_geom(const PassLimits& lim, int dtype, int norb, int noc
     return g;
   const long rows = (long)binom(norb, nocc);
   if (rows == 0 || rows > pipe_max_rows(8, 29)) return g;
+  static constexpr SmallForm kForms[2][4][3] = {
+      {{{8, 8, 1, 25, 19}, {16, 16, 1, 31, 21}},
+       {{4, 15, 1, 31, 21}, {8, 15, 1, 36, 25}, {16, 29, 1, 49, 33}},
+       {{4, 15, 1, 41, 23}, {8, 29, 1, 42, 26}},
+       {{4, 15, 1, 41, 23}, {8, 29, 1, 52, 31}}},
+      {{{8, 8, 1, 25, 19}, {16, 16, 1, 31, 21}},
+       {{4, 15, 1, 31, 21}, {8, 15, 1, 36, 25}, {16, 29, 2, 52, 35}},
+       {{4, 15, 1, 41, 25}, {8, 29, 1, 47, 32}},
+       {{4, 15, 1, 41, 25}, {8, 29, 2, 61, 37}}}};
+  const int cls = rows <= pipe_max_rows(16, 16)   ? 0
+                  : rows <= pipe_max_rows(16, 29) ? 1
+                  : rows <= 512                   ? 2
+                                                  : 3;
   g.whole = g.small = true;
-  g.units = 8;
-  g.sweeps = rows <= pipe_max_rows(8, 8) ? 8 : rows <= pipe_max_rows(8, 15) ? 15 : 29;
-  auto tiles = [&]() {
-    const long w = pipe_width(g.units, elem);
-    return (n_batch + w - 1) / w * n_states;
-  };
-  if (g.sweeps == 29 && tiles() < lim.n_cu) {
-    g.units = 4;
-    g.sweeps = 15;
-  } else if (rows <= pipe_max_rows(16, 29) && tiles() > lim.n_cu) {
-    g.units = 16;
-    g.sweeps = rows <= pipe_max_rows(16, 16) ? 16 : 29;
+  double best = 0.0;
+  for (const SmallForm& f : kForms[dtype == FFSIM_C64][cls]) {
+    if (f.units == 0) break;
+    const long w = pipe_width(f.units, elem), tiles = (n_batch + w - 1) / w * n_states;
+    const double t = f.first + f.more * (double)((tiles + lim.n_cu - 1) / lim.n_cu - 1);
+    if (g.units && t >= best) continue;
+    best = t;
+    g.units = f.units;
+    g.sweeps = f.sweeps;
+    g.cols = f.cols;
   }
-  if (tiles() > lim.n_cu && g.sweeps == 29) g.cols = pipe_cols(g.units, elem);
   return g;
 }
 

@@ -68,3 +68,27 @@ def test_every_sector_up_to_norb_12_runs_in_place(rules, dtype, norb):
                 assert units and 256 // units * sweeps >= comb(norb, nocc)
                 # with strings on rows a 16-byte unit must not reach past the columns
                 assert cols or n_batch >= (1 if dtype == C128 else 2)
+
+
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize("norb", range(6, 13))
+@pytest.mark.parametrize("n_states", [1, 2, 3, 8, 32, 256])
+def test_small_tiles_hold_their_sector(rules, dtype, norb, n_states):
+    """A compiled geometry whose tile has a row for every string."""
+    compiled = {(4, 15, 1), (8, 8, 1), (8, 15, 1), (8, 29, 1), (16, 16, 1), (16, 29, 1)}
+    if dtype == C64:
+        compiled |= {(8, 29, 2), (16, 29, 2)}
+    for nocc in range(norb + 1):
+        for other in range(norb + 1):
+            units, _, sweeps, cols = _small(rules, dtype, norb, nocc, comb(norb, other), n_states)
+            assert (units, sweeps, cols) in compiled
+            assert 256 // units * sweeps >= comb(norb, nocc)
+
+
+@pytest.mark.parametrize("dtype,nocc,n_states,units", [
+    # one round of 64-byte rows; two states of complex128 are one round of 128-byte rows
+    (C128, 6, 1, 4), (C128, 6, 2, 8), (C128, 5, 2, 8), (C128, 6, 32, 8),
+    (C64, 6, 2, 4), (C64, 6, 3, 8), (C64, 6, 5, 4), (C64, 6, 8, 8), (C64, 4, 6, 8),
+])
+def test_small_tile_width_norb_12(rules, dtype, nocc, n_states, units):
+    assert _small(rules, dtype, 12, nocc, comb(12, nocc), n_states)[0] == units
