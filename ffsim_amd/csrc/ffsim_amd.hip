@@ -1286,13 +1286,15 @@ Fused orbital_rotation_impl(Context& ctx, void* vec, void* work, int dtype, int 
   if (ld_w == 0) ld_w = transposed_ld(dtype, dim_a);
   require(ld_w >= dim_a, FFSIM_ERR_VALUE, "work row pitch below dim_a");
   SectorRotation ra, rb;
-  if (mat_a) ra = prepare_rotation(mat_a, norb, w_a);
+  // (a sector of one string runs no rotations: any order serves, so the other's)
+  const int o_a = dim_a == 1 ? w_b : w_a, o_b = dim_b == 1 ? w_a : w_b;
+  if (mat_a) ra = prepare_rotation(mat_a, norb, o_a);
   if (mat_b) {
     if (mat_a && std::memcmp(mat_a, mat_b, sizeof(cdouble) * norb * norb) == 0 &&
-        triangle_order(norb, w_a) == triangle_order(norb, w_b))
+        triangle_order(norb, o_a) == triangle_order(norb, o_b))
       rb = ra;
     else
-      rb = prepare_rotation(mat_b, norb, w_b);
+      rb = prepare_rotation(mat_b, norb, o_b);
   }
   Program prog(ctx, stream);
   std::vector<std::function<void()>> launches;

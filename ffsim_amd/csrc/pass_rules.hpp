@@ -228,9 +228,12 @@ inline SectorGeom sector_geom(const PassLimits& lim, int dtype, int norb, int no
   g.w = choose_window(lim, norb, nocc, dtype);
   const size_t elem = elem_bytes(dtype);
   if (n_batch > (1l << 30) || tile_width(dtype) != (dtype == FFSIM_C64 ? 4 : 8)) return g;
-  if (norb > window_cap() && norb >= kMaxSubWindow && norb <= 16)
+  const long rows = (long)binom(norb, nocc);
+  // (a single string has nothing to rotate: windows skip all but the last pass,
+  // whose plain tiles are one row; norb 16 with (8, 0) electrons 116 against 138 us)
+  if (norb > window_cap() && norb >= kMaxSubWindow && norb <= 16 && rows > 1)
     for (int units : {8, 4, 2, 1})
-      if ((long)binom(norb, nocc) <= pipe_max_rows(units) &&
+      if (rows <= pipe_max_rows(units) &&
           n_batch >= pipe_width(units, elem)) {
         g.w = norb;
         g.units = units;

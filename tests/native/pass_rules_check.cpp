@@ -22,3 +22,17 @@ extern "C" void small_pass(int dtype, int norb, int nocc, long n_batch, int n_st
   out[2] = g.sweeps;
   out[3] = g.cols;
 }
+
+// Passes of a sector with strings on rows: window, units of a pipelined tile,
+// whether a tile holds the whole sector; returns whether a pass over all fibers
+// of the window [0, w) runs pipelined.
+extern "C" int sector_pass(int dtype, int norb, int nocc, long n_batch, int* out) {
+  const SectorGeom g = sector_geom(kLim, dtype, norb, nocc, n_batch);
+  out[0] = g.w;
+  out[1] = g.units;
+  out[2] = g.whole;
+  long n_f = 0;
+  for (int kp = std::max(0, nocc - (norb - g.w)); kp <= std::min(nocc, g.w); ++kp)
+    n_f += (long)binom(norb - g.w, nocc - kp);
+  return pipe_applies(kLim, dtype, g, max_fiber(norb, nocc, g.w), n_f, n_batch);
+}

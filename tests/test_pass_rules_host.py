@@ -92,3 +92,28 @@ def test_small_tiles_hold_their_sector(rules, dtype, norb, n_states):
 ])
 def test_small_tile_width_norb_12(rules, dtype, nocc, n_states, units):
     assert _small(rules, dtype, 12, nocc, comb(12, nocc), n_states)[0] == units
+
+
+def _sector(rules, dtype, norb, nocc, other):
+    """(window, units, whole sector in a tile, last pass pipelined)"""
+    out = (ctypes.c_int * 3)()
+    piped = rules.sector_pass(dtype, norb, nocc, ctypes.c_long(comb(norb, other)), out)
+    return out[0], out[1], bool(out[2]), bool(piped)
+
+
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize("norb", range(13, 19))
+def test_single_string_sectors_run_plain(rules, dtype, norb):
+    """Nothing to rotate: one plain pass, no tile of hundreds of rows for one."""
+    for nocc in (0, norb):
+        for other in range(norb + 1):
+            w, _, whole, piped = _sector(rules, dtype, norb, nocc, other)
+            assert w == 12 and not whole and not piped
+
+
+@pytest.mark.parametrize("dtype", [C128, C64])
+def test_sectors_of_norb_13_to_16_run_whole(rules, dtype):
+    for norb, nocc in [(13, 6), (14, 7), (15, 7), (16, 5), (16, 1), (13, 12)]:
+        assert _sector(rules, dtype, norb, nocc, nocc) == (norb, _sector(
+            rules, dtype, norb, nocc, nocc)[1], True, True)
+    assert _sector(rules, dtype, 16, 8, 8)[:3] == (12, 8, False)
