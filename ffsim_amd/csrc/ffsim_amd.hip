@@ -1047,13 +1047,48 @@ std::pair<size_t, size_t> append_diag_params(Program& prog, const DiagSpec& spec
   return {hoff, coff};
 }
 
-// Factor tables of a diagonal Coulomb evolution to fuse into the final
-// transposing pass (offsets in the call's program; see DiagFuse).
-struct FuseTables {
-  size_t bfac_off = 0, rfac_off = 0;
-  int n_fac = 0;
-  bool columns_later = false;  // pipelined: the tile strings' own factor is left to the next gate
+// What became of the diagonal evolution that follows a rotation.
+enum class Fused { kNo, kYes, kAllButColumns };
+
+// A diagonal Coulomb evolution that the last pass of the beta sector may take: a
+// transposing row pass, whose batch columns are the alpha strings.
+struct FuseRequest {
+  const DiagSpec* spec;
+  int norb, na, nb;
+  // (pipelined) the beta strings' own factor may be left to the next gate
+  bool columns_later;
+  size_t bfac_off = 0, rfac_off = 0;  // factor tables in the call's program (see DiagFuse)
+  Fused done = Fused::kNo;
+  int n_fac() const { return norb + 1; }
 };
+
+// Queues the factor tables of a fused diagonal, for a pass that then takes it;
+// false, with nothing queued, if the program's scratch has no room for them.
+bool queue_fuse_tables(Context& ctx, Program& prog, FuseRequest& f, bool columns_later,
+                       hipStream_t stream, std::vector<std::function<void()>>& launches) {
+  const long dim_a = (long)binom(f.norb, f.na), dim_b = (long)binom(f.norb, f.nb);
+  const int n_fac = f.n_fac();
+  if (!prog.reserve((size_t)dim_a * n_fac * sizeof(Cx<double>), &f.bfac_off)) return false;
+  if (!columns_later && !prog.reserve((size_t)dim_b * sizeof(Cx<double>), &f.rfac_off))
+    return false;
+  const auto [hoff, coff] = append_diag_params(prog, *f.spec);
+  const DevStrings& sa = dev_strings(ctx, f.norb, f.na);
+  const DevStrings& sb = dev_strings(ctx, f.norb, f.nb);
+  launches.push_back([=, &prog, &sa, &sb, h = hoff, c = coff, bfac = f.bfac_off,
+                      rfac = f.rfac_off]() {
+    const long n_a = dim_a * n_fac;
+    hipLaunchKernelGGL(diag_row_factor_kernel, dim3((unsigned)((n_a + 255) / 256)), dim3(256), 0,
+                       stream, (int)dim_a, sa.d, prog.dev<DiagHeader>(h), prog.dev<double>(c),
+                       prog.scratch<Cx<double>>(bfac));
+    HIP_CHECK(hipGetLastError());
+    if (columns_later) return;
+    launch_diag_col_term(dim_b, sb.d, prog.dev<DiagHeader>(h), prog.dev<double>(c),
+                         prog.scratch<double>(rfac), 1, stream);
+    HIP_CHECK(hipGetLastError());
+  });
+  f.done = columns_later ? Fused::kAllButColumns : Fused::kYes;
+  return true;
+}
 
 // The sub-window slots of a pass and the largest group tables that any fiber
 // of the pass stages (over the window's electron counts kp).
@@ -1089,9 +1124,7 @@ size_t append_unit_phases(Program& prog, int norb) {
 void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, long ld,
                 int n_batch, int norb, int nocc, const SectorRotation& rot, void* tstore_dst,
                 long ld_t, hipStream_t stream, std::vector<std::function<void()>>& launches,
-                const FuseTables* fuse = nullptr, bool* fused = nullptr,
-                const size_t* cfac_off = nullptr) {
-  if (fused) *fused = false;
+                FuseRequest* fuse = nullptr, const size_t* cfac_off = nullptr) {
   const bool tstore = tstore_dst != nullptr;
   SectorGeom geom;
   if (!tstore) geom = small_geom(ctx.limits(), dtype, norb, nocc, n_batch, 1);
@@ -1127,13 +1160,38 @@ void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, l
     void* dst = ts ? tstore_dst : state;
     const long ld_dst = ts ? ld_t : ld;
     const bool all = ts || dg;
-    if (geom.small || (mode == MODE_ROWS && pipe_applies(ctx, dtype, geom, win, all, n_batch))) {
+    const bool piped = geom.small ||
+                       (mode == MODE_ROWS && pipe_applies(ctx, dtype, geom, win, all, n_batch));
+    const bool fz_pipe = piped && ts && fuse && fuse->columns_later &&
+                         queue_fuse_tables(ctx, prog, *fuse, true, stream, launches);
+    // The plain kernel's fused store (window [0, w), w <= 16, production tile widths).
+    // A complex128 pass over part of the orbitals takes it even where it would run
+    // pipelined and the diagonal follow by itself: LUCJ n_reps=2 of norb 17 with (4, 8)
+    // electrons 26.2 against 26.8 ms, 18 (4, 7) 54.0 against 55.0; in complex64 the two
+    // are equal (24.4 and 24.5, 52.4 and 52.5, but norb 20 (3, 5) 34.9 and 34.4).
+    // Whole sectors stay pipelined: norb 16 (8, 3) complex64 1.6 against 6.3 ms.
+    LoSlots los{};
+    int gd_cap = 0, gm_cap = 0;
+    bool fz_on = false;
+    const int wf = dtype == FFSIM_C128 ? 8 : 4;
+    if (ts && fuse && !fz_pipe && (!piped || (!geom.whole && dtype == FFSIM_C128)) &&
+        mode == MODE_ROWS && tile_width(dtype) == wf && w >= kMaxSubWindow && w <= 16 &&
+        n_sub > 0 && P.lo == 0) {
+      pass_slots(dev_groups(ctx, w, dtype == FFSIM_C64), subs, los, gd_cap, gm_cap);
+      const int rows = win.max_rows;
+      const size_t lds = fiber_lds_bytes(elem_bytes(dtype), wf, false, 16, rows, gd_cap, gm_cap,
+                                         dg, true, norb, fuse->n_fac(), w);
+      const int nthr = 2 * lds > ctx.lds_max ? 512 : 256;
+      fz_on = lds <= ctx.lds_max && rows <= 1024 && wf * fuse->n_fac() <= nthr &&
+              queue_fuse_tables(ctx, prog, *fuse, false, stream, launches);
+    }
+    const size_t bfac_off = fz_pipe || fz_on ? fuse->bfac_off : 0;
+    const size_t rfac_off = fz_on ? fuse->rfac_off : 0;
+    const int n_fac = fz_pipe || fz_on ? fuse->n_fac() : 0;
+    if (piped && !fz_on) {
       size_t img_off = 0;
       const PipeTables tb0 =
           pass_tables(ctx, sector_pipe(ctx, dtype, norb, nocc, geom), subs, prog, &img_off);
-      const bool fz_pipe = ts && fuse && fuse->columns_later;
-      if (fz_pipe && fused) *fused = true;
-      const FuseTables fp = fz_pipe ? *fuse : FuseTables{};
       const bool cf = ts && cfac_off;
       const size_t coff = cf ? *cfac_off : 0;
       // (column factors ride on the phases of the pass: phases of one if it has none)
@@ -1145,7 +1203,7 @@ void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, l
                      prog.dev<LayerPair>(soff), n_layers, ph ? prog.dev<double>(doff) : nullptr,
                      ds.d, cf ? prog.scratch<Cx<double>>(coff) : nullptr, PipeFuse{nullptr, 0},
                      geom.small, cols, PipeStates{nullptr, 1, 0, 0}};
-        if (fz_pipe) L.fz = PipeFuse{prog.scratch<Cx<double>>(fp.bfac_off), fp.n_fac};
+        if (fz_pipe) L.fz = PipeFuse{prog.scratch<Cx<double>>(bfac_off), n_fac};
         PipeTables tb = tb0;
         if (!tb.image) tb.image = prog.dev<uint32_t>(img_off);
         pipe_pass(dtype, geom, L, win, tb, ctx.lds_max, stream);
@@ -1153,29 +1211,13 @@ void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, l
       continue;
     }
     const DevGroups& gr = dev_groups(ctx, w, dtype == FFSIM_C64);
-    LoSlots los{};
-    int gd_cap = 0, gm_cap = 0;
-    pass_slots(gr, subs, los, gd_cap, gm_cap);
+    if (!fz_on) pass_slots(gr, subs, los, gd_cap, gm_cap);
     require(!(ts && cfac_off), FFSIM_ERR_VALUE, "column factors need a pipelined pass");
-    // fuse the diagonal into this pass when the kernel's fused layout applies
-    bool fz_on = false;
-    // (the fused store takes the pass's window to be [0, w), w <= 16)
-    const int wf = dtype == FFSIM_C128 ? 8 : 4;
-    if (ts && fuse && !fuse->columns_later && mode == MODE_ROWS && tile_width(dtype) == wf && gr.w2 == kMaxSubWindow &&
-        n_sub > 0 && P.lo == 0 && w <= 16) {
-      const int rows = win.max_rows;
-      const size_t lds = fiber_lds_bytes(elem_bytes(dtype), wf, false, 16, rows, gd_cap, gm_cap,
-                                         dg, true, norb, fuse->n_fac, w);
-      const int nthr = 2 * lds > ctx.lds_max ? 512 : 256;
-      fz_on = lds <= ctx.lds_max && rows <= 1024 && wf * fuse->n_fac <= nthr;
-    }
-    if (fz_on && fused) *fused = true;
-    const FuseTables ft = fz_on ? *fuse : FuseTables{};
     launches.push_back([=, &ctx, &prog, &win, &gr, &ds]() {
       DiagFuse dfz{};
       if (fz_on)
-        dfz = DiagFuse{prog.scratch<Cx<double>>(ft.bfac_off), prog.scratch<Cx<double>>(ft.rfac_off),
-                       ft.n_fac, w};
+        dfz = DiagFuse{prog.scratch<Cx<double>>(bfac_off), prog.scratch<Cx<double>>(rfac_off),
+                       n_fac, w};
       fiber_pass(dtype, mode, state, dst, ld, ld_dst, n_batch, ts, win, all, gr, los, gd_cap,
                  gm_cap, prog.dev<SubPass>(poff), n_sub, prog.dev<LayerPair>(soff), n_layers,
                  dg ? prog.dev<double>(diag_off) : nullptr, ds.d, norb, ctx, stream,
@@ -1193,9 +1235,6 @@ long transposed_ld(int dtype, long dim_a) {
   const long q = 32 / (long)elem_bytes(dtype);
   return (dim_a + q - 1) / q * q;
 }
-
-// What became of the diagonal evolution that follows a rotation.
-enum class Fused { kNo, kYes, kAllButColumns };
 
 // Whether the fused diagonal of this shape runs in the pipelined kernel: both
 // transposing passes (the beta sector's, which applies it, and the alpha
@@ -1300,20 +1339,12 @@ Fused orbital_rotation_impl(Context& ctx, void* vec, void* work, int dtype, int 
   std::vector<std::function<void()>> launches;
   const bool beta_transposed = mat_b && !beta_cols;
   if (beta_transposed) require(work != nullptr, FFSIM_ERR_VALUE, "work buffer required");
-  // factor tables of the fused diagonal: alpha strings are the final pass's
-  // batch columns, beta strings its tile rows
-  FuseTables ft;
-  bool want_fuse = then_diag && then_diag->flags && !then_diag->z_rep &&
-                   then_diag->norb == norb && beta_transposed &&
-                   norb + 1 <= 64;
-  if (want_fuse) {
-    ft.n_fac = norb + 1;
-    ft.columns_later = may_leave_columns &&
-                       pipe_fuse_applies(ctx, dtype, norb, na, nb, ft.n_fac);
-    want_fuse = prog.reserve((size_t)dim_a * ft.n_fac * sizeof(Cx<double>), &ft.bfac_off) &&
-                (ft.columns_later ||
-                 prog.reserve((size_t)dim_b * sizeof(Cx<double>), &ft.rfac_off));
-  }
+  FuseRequest fuse{then_diag, norb, na, nb, false};
+  const bool want_fuse = then_diag && then_diag->flags && !then_diag->z_rep &&
+                         then_diag->norb == norb && beta_transposed && norb + 1 <= 64;
+  if (want_fuse)
+    fuse.columns_later =
+        may_leave_columns && pipe_fuse_applies(ctx, dtype, norb, na, nb, fuse.n_fac());
   // the previous gate's diagonal left its factor of the beta strings alone to
   // this rotation: the last alpha pass multiplies its columns by it
   size_t cfac_off = 0;
@@ -1328,32 +1359,11 @@ Fused orbital_rotation_impl(Context& ctx, void* vec, void* work, int dtype, int 
       HIP_CHECK(hipGetLastError());
     });
   }
-  if (want_fuse) {
-    const std::pair<size_t, size_t> par = append_diag_params(prog, *then_diag);
-    const size_t hoff = par.first, coff = par.second;
-    const DevStrings& sa = dev_strings(ctx, norb, na);
-    const DevStrings& sb = dev_strings(ctx, norb, nb);
-    const int nf = ft.n_fac;
-    const bool later = ft.columns_later;
-    launches.push_back([=, &prog, &sa, &sb]() {
-      const long n_a = dim_a * nf;
-      hipLaunchKernelGGL(diag_row_factor_kernel, dim3((unsigned)((n_a + 255) / 256)), dim3(256),
-                         0, stream, (int)dim_a, sa.d, prog.dev<DiagHeader>(hoff),
-                         prog.dev<double>(coff), prog.scratch<Cx<double>>(ft.bfac_off));
-      HIP_CHECK(hipGetLastError());
-      if (later) return;
-      hipLaunchKernelGGL(diag_col_term_kernel, dim3((unsigned)((dim_b + 255) / 256)), dim3(256),
-                         0, stream, (int)dim_b, sb.d, prog.dev<DiagHeader>(hoff),
-                         prog.dev<double>(coff), prog.scratch<double>(ft.rfac_off), 1, 0l, 0l);
-      HIP_CHECK(hipGetLastError());
-    });
-  }
-  bool fused = false;
   if (mat_a || beta_transposed) {
     SectorRotation empty;
     const SectorRotation& r = mat_a ? ra : empty;
     run_sector(ctx, prog, dtype, MODE_ROWS, vec, dim_b, (int)dim_b, norb, na, r,
-               beta_transposed ? work : nullptr, ld_w, stream, launches, nullptr, nullptr,
+               beta_transposed ? work : nullptr, ld_w, stream, launches, nullptr,
                left_columns ? &cfac_off : nullptr);
   }
   if (mat_b) {
@@ -1362,18 +1372,19 @@ Fused orbital_rotation_impl(Context& ctx, void* vec, void* work, int dtype, int 
                  stream, launches);
     } else {
       run_sector(ctx, prog, dtype, MODE_ROWS, work, ld_w, (int)dim_a, norb, nb, rb, vec, dim_b,
-                 stream, launches, want_fuse ? &ft : nullptr, &fused);
+                 stream, launches, want_fuse ? &fuse : nullptr);
     }
   }
   // a diagonal that no pass took follows in the same program: one upload less
-  const bool columns_left = fused && ft.columns_later;
-  if (then_diag && then_diag->flags && !fused)
-    fused = queue_diag(ctx, prog, DIAG_EVOLVE, vec, vec, dtype, norb, na, nb, *then_diag, stream,
-                       launches);
+  Fused fused = fuse.done;
+  if (then_diag && then_diag->flags && fused == Fused::kNo &&
+      queue_diag(ctx, prog, DIAG_EVOLVE, vec, vec, dtype, norb, na, nb, *then_diag, stream,
+                 launches))
+    fused = Fused::kYes;
   prog.commit();
   for (auto& f : launches) f();
   prog.finish();
-  return !fused ? Fused::kNo : columns_left ? Fused::kAllButColumns : Fused::kYes;
+  return fused;
 }
 
 

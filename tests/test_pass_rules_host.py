@@ -117,3 +117,17 @@ def test_sectors_of_norb_13_to_16_run_whole(rules, dtype):
         assert _sector(rules, dtype, norb, nocc, nocc) == (norb, _sector(
             rules, dtype, norb, nocc, nocc)[1], True, True)
     assert _sector(rules, dtype, 16, 8, 8)[:3] == (12, 8, False)
+
+
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize("norb,nocc,other", [(17, 2, 3), (17, 3, 2), (18, 3, 3), (16, 8, 1),
+                                             (18, 0, 3), (18, 3, 0), (18, 3, 18), (18, 18, 3)])
+def test_passes_that_run_plain(rules, dtype, norb, nocc, other):
+    """The shapes that tests/test_gpu_plain_passes.py takes for plain ones."""
+    assert not _sector(rules, dtype, norb, nocc, other)[3]
+
+
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize("norb,nocc,other", [(16, 8, 8), (18, 9, 9), (17, 8, 4), (14, 2, 7)])
+def test_passes_that_run_pipelined(rules, dtype, norb, nocc, other):
+    assert _sector(rules, dtype, norb, nocc, other)[3]
