@@ -1611,13 +1611,14 @@ void ucj_impl(Context& ctx, void* vec, void* work, int dtype, int n, int na, int
 // 8 dim^3 flops per state and sector against one HBM pass of the state on the
 // Givens path, and the path's fixed cost (a compound-matrix launch and two
 // batched GEMMs per rotation) is shared by the batch, as the Givens path's
-// launches are when all states share them.  Measured per state (LUCJ
-// n_reps=2, complex128, MI355X; GEMM vs Givens with all states per launch):
-// norb=8 (70 strings) 0.26 vs 0.54 ms alone, 0.051 vs 0.067 ms in a batch of
-// 8 and 0.017 vs 0.024 in a batch of 32; norb=9 (126 strings) 0.052 vs 0.061
-// and 0.021 vs 0.029; norb=10 (4,4) (210 strings) 0.067 vs 0.047 and 0.053 vs
-// 0.033; norb=10 (5,5) (252 strings) 0.077 vs 0.051 and 0.069 vs 0.033;
-// norb=12 (924 strings) 2.6 vs 0.16 ms in a batch of 32.
+// launches are when all states share them.  Measured per call (LUCJ n_reps=2,
+// complex128, MI355X, the call waited for; GEMM against Givens passes with all
+// states per launch), once every slot of the program ring has grown to the call's
+// scratch (the compound matrices'; until then a GEMM call allocates, norb=8 (4,4)
+// 550 to 720 us in batches of 32): norb=8 (4,3) 133 and 196 us alone, 157 and 254
+// in a batch of 8, 245 and 412 in 32; norb=9 (4,5) 238 and 264 in 8, 457 and 487 in
+// 32; norb=10 (3,3) 222 and 298 in 8; norb=10 (5,5) 569 and 319 in 8, 1896 and 731
+// in 32.
 constexpr long kGemmAlwaysDim = 100;   // any batch
 constexpr long kGemmBatchDim = 150;    // batches of at least kGemmMinBatch states
 constexpr int kGemmMinBatch = 8;
