@@ -282,7 +282,7 @@ __global__ void __launch_bounds__(kPipeThreads)
     }
   };
   if constexpr (DG && !SMALL) build_ptab(diag);
-  // what this thread needs of a fiber's strings (i = i0 + 32 k): their rows, and
+  // what this thread needs of a fiber's strings (i = i0 + STEP k): their rows, and
   // their bits inside the window for the phases
   auto stage_rows = [&](const Fiber& fd, int slot) {
     if constexpr (!CONTIG || DG || FUSE) {
@@ -386,7 +386,7 @@ __global__ void __launch_bounds__(kPipeThreads)
     const int c = min(b0 + u * EU, n_batch - EU);
     return COLS && EU > 1 ? max(c, 0) : c;
   };
-  // register k holds sweep k of its tile, or sweep 28 - k (see exchange): string
+  // register k holds sweep k of its tile, or sweep SWEEPS - 1 - k (see exchange): string
   // first + k step.  Transposing passes work on contiguous rows (window [0, w)).
   auto load = [&](auto k0c, auto k1c, const Cx<T>* base, int first, int step, int slot, int nr,
                   int row0, int b0) {
