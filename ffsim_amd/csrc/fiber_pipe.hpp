@@ -421,6 +421,7 @@ __global__ void __launch_bounds__(kPipeThreads)
     constexpr int K0 = decltype(k0c)::value, K1 = decltype(k1c)::value;
     const bool full = b0 + W <= n_batch;
     const int c0 = unit_col(b0), skip = b0 + u * EU - c0;
+    const bool single = COLS && n_batch < EU;
 #pragma unroll
     for (int k = K0; k < K1; ++k) {
       const int i = first + k * step;
@@ -460,7 +461,7 @@ __global__ void __launch_bounds__(kPipeThreads)
         if constexpr (TST || COLS) {
 #pragma unroll
           for (int z = 0; z < EU; ++z)
-            if (full || (z >= skip && (!COLS || z < n_batch)))
+            if (full || (z >= skip && (z == 0 || !single)))
               base[(uint64_t)(uint32_t)(c0 + z) * (uint32_t)ld_dst + row] = e[z];
         } else {
           Cx<T>* p = base + c0 + (uint64_t)row * (uint32_t)ld_dst;
