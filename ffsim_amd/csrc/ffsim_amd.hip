@@ -1174,9 +1174,10 @@ void run_sector(Context& ctx, Program& prog, int dtype, int mode, void* state, l
     int gd_cap = 0, gm_cap = 0;
     bool fz_on = false;
     const int wf = dtype == FFSIM_C128 ? 8 : 4;
-    if (ts && fuse && !fz_pipe && (!piped || (!geom.whole && dtype == FFSIM_C128)) &&
-        mode == MODE_ROWS && tile_width(dtype) == wf && w >= kMaxSubWindow && w <= 16 &&
-        n_sub > 0 && P.lo == 0) {
+    const bool plain = !piped || (!geom.whole && dtype == FFSIM_C128 &&
+                                  w - kMaxSubWindow < kMaxLoSlots);
+    if (ts && fuse && !fz_pipe && plain && mode == MODE_ROWS && tile_width(dtype) == wf &&
+        w >= kMaxSubWindow && w <= 16 && n_sub > 0 && P.lo == 0) {
       pass_slots(dev_groups(ctx, w, dtype == FFSIM_C64), subs, los, gd_cap, gm_cap);
       const int rows = win.max_rows;
       const size_t lds = fiber_lds_bytes(elem_bytes(dtype), wf, false, 16, rows, gd_cap, gm_cap,
